@@ -31,8 +31,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("NSFPS_OFFLOAD_ARCH", "gfx950")
 
 LIB = os.path.join(HERE, "libnsfps.so")
-SOURCES = ("nsfps_build.hip", "nsfps_sample.hip", "nsfps_runs.hip", "nsfps_group.hip",
-           "nsfps_host.cpp")
+SOURCES = ("nsfps_build.hip", "nsfps_sample.hip", "nsfps_runs.hip", "nsfps_small.hip",
+           "nsfps_group.hip", "nsfps_host.cpp")
 
 # Exact fp32: no contraction, IEEE division/sqrt, denormals kept.
 # "-packed-fp32-ops" turns off the gfx950 packed fp32 instructions

@@ -521,6 +521,7 @@ nsfps_status prepare_device(int dev) {
   if (g_kernels_loaded[dev]) return NSFPS_OK;
   HIP_TRY(preload_build_kernels());
   HIP_TRY(preload_runs_kernels());
+  HIP_TRY(preload_small_kernels());
   HIP_TRY(preload_group_kernels());
   g_kernels_loaded[dev] = true;
   return NSFPS_OK;
@@ -1685,6 +1686,174 @@ bool choose_runs(std::vector<CloudPlan> &plans) {
   return runs;
 }
 
+// Calls whose clouds all have the same, small point count are sorted and
+// sampled by one workgroup per cloud (nsfps_small.hip): two launches and one
+// read-back for the call.  The switches that choose or trace the general
+// engines' parts, and the failure injection that counts their operations,
+// take those engines; NSFPS_SMALL=0 or 1 decides it alone.
+bool small_wanted(const std::vector<CloudPlan> &plans) {
+  for (auto &p : plans)
+    if (p.n != plans[0].n || p.n > kSmallMaxPoints || p.rng.dev.T > (1u << kSmallMaxBits))
+      return false;
+  if (const char *e = getenv("NSFPS_SMALL")) return atoi(e) != 0;
+  for (const char *v : {"NSFPS_ENGINE", "NSFPS_NO_PADDED", "NSFPS_MIXED", "NSFPS_LEAF_BOUND",
+                        "NSFPS_STREAMS", "NSFPS_GLOBAL_SORT", "NSFPS_HOT", "NSFPS_DENSE_WALK",
+                        "NSFPS_WHOLE", "NSFPS_PROFILE", "NSFPS_INJECT"})
+    if (getenv(v)) return false;
+  return true;
+}
+
+// Where a call of small clouds keeps its data.
+struct SmallLayout {
+  SmallDev *devs = nullptr;
+  SmallStatus *st = nullptr;
+  float4 *pts = nullptr;
+  uint16_t *rows = nullptr;
+  float *stage = nullptr;   // host input
+  int32_t *out = nullptr;   // samples of clouds without a device buffer of the caller's
+};
+void layout_small(Bump &bp, const std::vector<CloudPlan> &plans, SmallLayout &L) {
+  const size_t nc = plans.size(), n = plans[0].n;
+  L.devs = bp.take<SmallDev>(nc);
+  L.st = bp.take<SmallStatus>(nc);
+  L.pts = bp.take<float4>(nc * n);
+  L.rows = bp.take<uint16_t>(nc * n);
+  L.stage = plans[0].h_xyz ? bp.take<float>(nc * n * 3) : nullptr;
+  L.out = plans[0].d_out_user ? nullptr : bp.take<int32_t>(nc * plans[0].m);
+}
+
+// The sort of every cloud, enqueued on st; devs: the clouds' parameters, a
+// source of an asynchronous copy that the caller keeps until st is waited for.
+nsfps_status small_sort(const std::vector<CloudPlan> &plans, const SmallLayout &L,
+                        std::vector<SmallDev> &devs, hipStream_t st) {
+  const size_t nc = plans.size(), n = plans[0].n;
+  std::vector<HostUp> ups;
+  bool one_copy = plans[0].h_xyz != nullptr;
+  for (size_t i = 1; i < nc && one_copy; ++i)
+    one_copy = plans[i].h_xyz == plans[i - 1].h_xyz + n * 3;
+  for (size_t i = 0; i < nc && plans[0].h_xyz; ++i)
+    if (!one_copy || i == 0)
+      ups.push_back({L.stage + i * n * 3, plans[i].h_xyz, (one_copy ? nc : 1) * n * 12});
+  const nsfps_status rc = upload_host(ups, st);
+  if (rc) return rc;
+  devs.assign(nc, SmallDev{});
+  for (size_t i = 0; i < nc; ++i) {
+    SmallDev &d = devs[i];
+    const CloudPlan &p = plans[i];
+    d.xyz = p.h_xyz ? L.stage + i * n * 3 : p.d_xyz_in;
+    d.n = p.n;
+    d.m = p.m;
+    d.out = p.d_out_user ? p.d_out_user : L.out + i * (size_t)p.m;
+    d.pts = L.pts + i * n;
+    d.rows = L.rows + i * n;
+    d.st = L.st + i;
+    d.bbox = p.bbox_dev ? 1u : 0u;
+    d.r = p.rng.dev;
+  }
+  if (nc > 1)
+    HIP_TRY(hipMemcpyAsync(L.devs, devs.data(), nc * sizeof(SmallDev), hipMemcpyHostToDevice, st));
+  HIP_TRY(launch_small_sort(nc == 1 ? devs.data() : nullptr, L.devs, (uint32_t)nc, (uint32_t)n, st));
+  return NSFPS_OK;
+}
+
+// The sort's findings, as the general build reports them.
+nsfps_status small_check(const std::vector<CloudPlan> &plans, const std::vector<SmallStatus> &fin) {
+  for (auto &f : fin)
+    if (f.bad & 1u) return fail(NSFPS_EINVAL, "points must be finite");
+  for (size_t i = 0; i < fin.size(); ++i) {
+    if (!fin[i].bad) continue;
+    const float *b = fin[i].bounds;
+    const uint32_t *bl = plans[i].rng.dev.blocks;
+    const nsfps_status rc =
+        check_range(nsfps_range{b[0], b[1], b[2], b[3], b[4], b[5], bl[0], bl[1], bl[2]});
+    return rc ? rc : fail(NSFPS_EDEVICE, "internal: range of the points' bounds");
+  }
+  return NSFPS_OK;
+}
+
+void small_stats(const std::vector<CloudPlan> &plans, const std::vector<SmallStatus> &fin,
+                 const hipEvent_t *ev, std::chrono::steady_clock::time_point t0) {
+  nsfps_stats &S = g_stats;
+  if (ev) {
+    S.build_ms = ms_between(ev[0], ev[1]);
+    S.sample_ms = S.late_ms = ms_between(ev[1], ev[2]);
+    S.device_ms = S.build_ms + S.sample_ms;
+  }
+  S.n_clouds = plans.size();
+  S.n_points = (uint64_t)plans[0].n * plans.size();
+  S.n_leaves = (uint64_t)((plans[0].n + kLeaf - 1) / kLeaf) * plans.size();
+  for (auto &f : fin) {
+    S.samples += f.len;
+    S.rounds = std::max<uint64_t>(S.rounds, f.rounds);
+  }
+  S.mixed = 1;
+  S.engine = 1;
+  S.update_split = 1;
+  S.hot_set = 64;
+  memset(g_prof, 0, sizeof(g_prof));
+  S.e2e_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+}
+
+// One call of small clouds over workspace ws, as run_clouds_once.
+nsfps_status run_small(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_host, int32_t *h_out,
+                       uint64_t out_stride, uint64_t *out_lens) {
+  auto t0 = std::chrono::steady_clock::now();
+  const size_t nc = plans.size();
+  SmallLayout L;
+  Bump meas(nullptr);
+  layout_small(meas, plans, L);
+  if (!ws.base) {
+    Arena *ap = nullptr;
+    nsfps_status rc = arena_for_device(&ap);
+    if (rc) return rc;
+    rc = arena_reserve(*ap, meas.off);
+    if (rc) return rc;
+    ws.base = ap->base;
+    ws.cap = ap->cap;
+    if (!ws.st) ws.st = ap->stream;
+    ws.ev = ap->ev;
+  } else if (meas.off > ws.cap) {
+    return fail(NSFPS_EUNSUPPORTED,
+                "the call needs %zu bytes of device workspace, more than the %zu available",
+                meas.off, ws.cap);
+  }
+  Bump bp(ws.base);
+  layout_small(bp, plans, L);
+  hipStream_t st = ws.st;
+  ws.st_used = true;
+  std::vector<SmallDev> devs;
+  if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[0], st));
+  nsfps_status rc = small_sort(plans, L, devs, st);
+  if (rc) return rc;
+  if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[1], st));
+  HIP_TRY(launch_small_sample(L.devs, (uint32_t)nc, plans[0].n, 0, nullptr, st));
+  if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[2], st));
+  std::vector<SmallStatus> fin(nc);
+  rc = readback(fin.data(), L.st, nc * sizeof(SmallStatus), st);
+  if (rc) return rc;
+  rc = small_check(plans, fin);
+  if (rc) return rc;
+  for (size_t i = 0; i < nc; ++i) {
+    if (fin[i].err) return fail(NSFPS_EDEVICE, "internal: sampling rounds did not end");
+    out_lens[i] = fin[i].len;
+  }
+  if (out_on_host) {
+    if (nc > 1 && out_stride == plans[0].m) {  // rows of m entries on both sides
+      rc = download_host(h_out, L.out, nc * (size_t)out_stride * 4, st);
+      if (rc) return rc;
+    } else {
+      for (size_t i = 0; i < nc; ++i) {
+        rc = download_host(h_out + i * out_stride, L.out + i * (size_t)plans[0].m,
+                           (size_t)fin[i].len * 4, st);
+        if (rc) return rc;
+      }
+    }
+    HIP_TRY(hipStreamSynchronize(st));
+  }
+  small_stats(plans, fin, ws.ev, t0);
+  return NSFPS_OK;
+}
+
 // Samples the built clouds (descriptors in plans[i].dev): grid-wide steps for
 // the first iterations of a single cloud on the tree engine, then its loop;
 // or the speculative-run rounds.
@@ -1812,7 +1981,9 @@ nsfps_status run_clouds_once(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_
 nsfps_status run_clouds(std::vector<CloudPlan> &plans, Ws ws, bool out_on_host, int32_t *h_out,
                         uint64_t out_stride, uint64_t *out_lens) {
   CallLayout L;
-  const nsfps_status rc = run_clouds_once(plans, ws, out_on_host, h_out, out_stride, out_lens, L);
+  const nsfps_status rc =
+      small_wanted(plans) ? run_small(plans, ws, out_on_host, h_out, out_stride, out_lens)
+                          : run_clouds_once(plans, ws, out_on_host, h_out, out_stride, out_lens, L);
   if (rc && ws.st_used) {
     (void)hipStreamSynchronize(ws.st);
     // a failed call may leave rounds of its second half queued
@@ -1915,6 +2086,8 @@ struct PlanImpl {
   float4 *lp_0 = nullptr;
   hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   bool runs = true;
+  bool small = false;  // sorted by nsfps_small.hip's kernels (SL), no general structure
+  SmallLayout SL;
   PlanImpl() = default;
   PlanImpl(const PlanImpl &) = delete;
   PlanImpl &operator=(const PlanImpl &) = delete;
@@ -2384,6 +2557,36 @@ nsfps_status nsfps_plan_create(const float *xyz, uint64_t n, const nsfps_range *
       *out = plan.release();
       return NSFPS_OK;
     }
+    P.small = small_wanted(P.plans);
+    if (P.small) {
+      Bump meas(nullptr);
+      layout_small(meas, P.plans, P.SL);
+      const hipError_t inj = injected(kInjAlloc);
+      const hipError_t e = inj != hipSuccess ? inj : hipMalloc(&P.mem, meas.off + 256);
+      if (e != hipSuccess) {
+        P.mem = nullptr;
+        return fail(NSFPS_ENOMEM, "hipMalloc(%zu) failed: %s", meas.off + 256,
+                    inj != hipSuccess ? "injected failure (NSFPS_INJECT)" : hipGetErrorString(e));
+      }
+      P.cap = meas.off + 256;
+      for (auto &ev : P.ev) HIP_TRY(hipEventCreate(&ev));
+      Bump bp(P.mem);
+      layout_small(bp, P.plans, P.SL);
+      std::vector<SmallDev> devs;
+      std::vector<SmallStatus> fin(1);
+      rc = small_sort(P.plans, P.SL, devs, nullptr);
+      if (!rc) rc = readback(fin.data(), P.SL.st, sizeof(SmallStatus), nullptr);
+      if (rc) {
+        (void)hipStreamSynchronize(nullptr);  // nothing enqueued outlives the plan's memory
+        return rc;
+      }
+      rc = small_check(P.plans, fin);
+      if (rc) return rc;
+      P.plans[0].h_xyz = nullptr;  // the input is not read again
+      P.plans[0].d_xyz_in = nullptr;
+      *out = plan.release();
+      return NSFPS_OK;
+    }
     const size_t need = measure_call(P.plans, P.L);
     Bump snap(nullptr);
     snap.off = need;
@@ -2463,6 +2666,24 @@ nsfps_status nsfps_plan_sample(nsfps_plan *plan, uint64_t m, int32_t *d_out, uin
     }
     if (m > 0x7fffffffull) return fail(NSFPS_EUNSUPPORTED, "at most 2^31-1 samples");
     auto t0 = std::chrono::steady_clock::now();
+    if (P.small) {
+      const auto small = [&]() -> nsfps_status {
+        HIP_TRY(hipEventRecord(P.ev[0], st));
+        HIP_TRY(hipEventRecord(P.ev[1], st));
+        HIP_TRY(launch_small_sample(P.SL.devs, 1, p.n, (uint32_t)m, d_out, st));
+        HIP_TRY(hipEventRecord(P.ev[2], st));
+        std::vector<SmallStatus> fin(1);
+        const nsfps_status rc = readback(fin.data(), P.SL.st, sizeof(SmallStatus), st);
+        if (rc) return rc;
+        if (fin[0].err) return fail(NSFPS_EDEVICE, "internal: sampling rounds did not end");
+        *out_len = fin[0].len;
+        small_stats(P.plans, fin, P.ev, t0);
+        return NSFPS_OK;
+      };
+      const nsfps_status rc = small();
+      if (rc) (void)hipStreamSynchronize(st);
+      return rc;
+    }
     p.m = (uint32_t)m;
     p.dev.m = (uint32_t)m;
     p.dev.out = d_out;

@@ -173,4 +173,32 @@ __host__ __device__ inline float key_dist(uint64_t k) {
   return c.f;
 }
 
+// Clouds of at most kSmallMaxPoints points, sampled by one workgroup each
+// (nsfps_small.hip).
+constexpr uint32_t kSmallMaxPoints = 16384;
+constexpr uint32_t kSmallMaxBits = 18;  // bucket bits: 14 row bits beside them in 32
+
+// What the kernels leave for the host, one per cloud.
+struct SmallStatus {
+  uint32_t bad;     // bit 0: a non-finite point; bit 1: a bounds range that cannot be one
+  uint32_t len;     // samples written
+  uint32_t rounds;  // rounds the sampling took
+  uint32_t err;     // set if the rounds did not end (internal error)
+  uint32_t pos0;    // where input row 0 is stored
+  uint32_t rank0;   //   and its logical rank
+  float bounds[6];  // compute_bbox's range, when it was asked for
+};
+
+struct SmallDev {
+  const float *xyz;  // n x 3, device; read by the sort alone
+  uint32_t n, m;
+  int32_t *out;      // m samples
+  float4 *pts;       // x, y, z, logical rank (bits) as stored
+  uint16_t *rows;    // input row of each rank
+  SmallStatus *st;
+  uint32_t bbox;     // 1: the range is compute_bbox of the points with r's block counts
+  uint32_t pad;
+  RangeDev r;
+};
+
 }  // namespace nsfps

@@ -16,6 +16,7 @@ namespace nsfps {
 // call's device time.
 hipError_t preload_build_kernels();
 hipError_t preload_runs_kernels();
+hipError_t preload_small_kernels();
 hipError_t preload_group_kernels();
 
 // hipFuncGetAttributes on every kernel given (it loads the kernel's code
@@ -149,6 +150,14 @@ hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t ma
                          uint32_t rounds, uint32_t passes, bool profile, bool alias,
                          bool leaf_bound, bool split, bool mixed, uint32_t hot, bool dense,
                          bool whole, hipStream_t st);
+
+// small clouds: nclouds clouds of n <= kSmallMaxPoints points each (devs[b];
+// or, nclouds = 1, *one, which the sort leaves in devs[0])
+hipError_t launch_small_sort(const SmallDev *one, SmallDev *devs, uint32_t nclouds, uint32_t n,
+                             hipStream_t st);
+// m, out: in place of the clouds' own when not zero / null (one cloud)
+hipError_t launch_small_sample(const SmallDev *devs, uint32_t nclouds, uint32_t n, uint32_t m,
+                               int32_t *out, hipStream_t st);
 
 // grouping after sampling (nsfps_group.hip): out[i] = xyz[idx[i]] (bad gets 1
 // for an index outside [0, n), whose row is zeroed); ball query rows of
