@@ -432,17 +432,14 @@ def run_ball_query(lib, hip, steps, radius=0.05, nsample=32):
 
 # ------------------------------------------------------------ phase clocks
 
-RUN_PHASES = ["load", "select", "gather", "phases", "apply", "tail", "big", "rank", "picks",
-              "rounds", "hot_sets", "phase_count", "walk", "publish", "rt_load", "rt_total"]
 PASS_COUNTERS = ["update_leaves", "update_points", "gather_leaves", "gather_points"]
 
 
 def run_phases(lib, hip, w):
-    """One call with NSFPS_PROFILE=1: the run kernel's phase clocks summed over
-    rounds (s_memtime cycles of wave 0 between its barriers, and s_memrealtime
-    ticks of 10 ns for the load and the whole kernel), per round and per hot
-    set.  Batched clouds: one call of all of them, the counters of cloud 0
-    (every kernel adds to its own cloud's words)."""
+    """One call with NSFPS_PROFILE=1: the update and gather passes' phase clocks
+    and counters summed over rounds, per round.  Batched clouds: one call of
+    all of them, the counters of cloud 0 (every kernel adds to its own cloud's
+    words)."""
     os.environ["NSFPS_PROFILE"] = "1"
     try:
         P = np.ascontiguousarray(np.stack(w["clouds"]))
@@ -461,7 +458,6 @@ def run_phases(lib, hip, w):
             hip.free(d_out)
     finally:
         del os.environ["NSFPS_PROFILE"]
-    v = dict(zip(RUN_PHASES, words[:16]))
     ctr = dict(zip(PASS_COUNTERS, words[24:28]))
     ctr.update(zip(["up_t_picks", "up_t_leaves", "up_t_flush", "up_groups"], words[32:36]))
     ctr.update(zip(["up_t_load", "up_t_zero", "up_t_hits", "up_t_points"], words[40:44]))
@@ -472,27 +468,9 @@ def run_phases(lib, hip, w):
     ctr.update(zip(["update_touched_leaves", "update_touched_points"], words[53:55]))
     ctr.update(zip(["up_w_hits_max", "up_w_hits_sum"], words[55:57]))
     ctr.update(zip(["window_keys", "listed", "window_keys_max"], words[57:60]))
-    v["walk_wait"], v["alias"], v["alias_entries"] = words[28], words[29], words[30]
-    rounds = max(1, v["rounds"])
-    hot = max(1, v["hot_sets"])
-    cycles = {k: v[k] for k in ["load", "select", "gather", "rank", "phases", "walk", "walk_wait",
-                                "alias", "apply", "big", "publish", "tail"]}
-    cyc_total = sum(cycles.values())
-    rt_us = v["rt_total"] * 0.01
-    clock_ghz = cyc_total / (rt_us * 1e3) if rt_us else None
-    return {"workload": w["name"], "profile": "run kernel phase clocks (NSFPS_PROFILE=1)",
-            "rounds": v["rounds"], "hot_sets": v["hot_sets"], "picks": v["picks"],
-            "phases": v["phase_count"], "samples_per_hot_set": round(v["picks"] / hot, 2),
-            "phases_per_hot_set": round(v["phase_count"] / hot, 2),
-            "multi_cell_entries_per_hot_set": round(v["alias_entries"] / hot, 1),
-            "run_kernel_us_per_round": round(rt_us / rounds, 2),
-            "load_us_per_round": round(v["rt_load"] * 0.01 / rounds, 2),
-            "run_kernel_us_total": round(rt_us, 1),
-            "s_memtime_ghz": round(clock_ghz, 3) if clock_ghz else None,
-            "cycles_per_hot_set": {k: round(cycles[k] / hot, 1) for k in cycles
-                                   if k not in ("load", "tail")},
-            "cycles_per_round": {"load": round(cycles["load"] / rounds, 1),
-                                 "tail": round(cycles["tail"] / rounds, 1)},
+    rounds = max(1, st["rounds"])
+    return {"workload": w["name"], "profile": "pass phase clocks (NSFPS_PROFILE=1)",
+            "rounds": st["rounds"], "samples_per_round": round(m / rounds, 1),
             "sample_ms": round(st["sample_ms"], 3), "device_ms": round(st["device_ms"], 3),
             "passes": pass_counts(w["name"], ctr, rounds)}
 
@@ -645,7 +623,7 @@ def main():
     ap.add_argument("--ball-query", action="store_true",
                     help="time only the grouping step after FPS (ball query) and print its line")
     ap.add_argument("--phases", action="store_true",
-                    help="print the run kernel's phase clocks of one profiled call and exit")
+                    help="print the sampling passes' phase clocks of one profiled call and exit")
     ap.add_argument("--calibrate", type=int, default=0, metavar="MIB",
                     help="first copy MIB MiB device-to-device (a copy kernel of known size for "
                          "calibrating rocprofv3 FETCH_SIZE / WRITE_SIZE)")

@@ -97,13 +97,14 @@ typedef struct {
   uint64_t samples;     /* samples produced (sum over clouds) */
   uint32_t padded;      /* 1 when the single cloud used the padded cell layout */
   uint32_t lds_bytes;   /* dynamic LDS of the single-workgroup loop */
-  uint64_t rounds;      /* speculative-run rounds (max over clouds; 0 for the tree loop) */
-  uint32_t engine;      /* 1: speculative runs, 0: grid-wide steps + tree loop */
+  uint64_t rounds;      /* sampling rounds of the runs engine (max over clouds; 0 for the tree loop) */
+  uint32_t engine;      /* 1: runs (rounds), 0: grid-wide steps + tree loop */
   uint32_t update_split; /* workgroups per level-1 node of the runs engine's update pass
                            (1, or 4 when the call has few level-1 nodes) */
   uint32_t mixed;       /* 1 when leaves were runs of 64 slots that may hold several buckets */
-  uint32_t hot_set;     /* copies per hot set of the runs engine's run kernel (64 or 128;
-                           0 for the tree loop) */
+  uint32_t hot_set;     /* density class of the clouds: 128 when every one fills at least 6,912
+                           buckets, else 64 (0 for the tree loop); earlier versions' hot sets
+                           had that many copies, no kernel depends on it now */
 } nsfps_stats;
 
 /* Library constants mirrored from src/yuezu_fps.h:19-50. */

@@ -582,7 +582,7 @@ __device__ __forceinline__ void leaf_desc_mixed_at(uint32_t l, uint32_t n, uint3
   leaf_lo[l] = make_float4(0.f, 0.f, 0.f, __uint_as_float(first));
   leaf_hi[l] = make_float4(0.f, 0.f, 0.f, __uint_as_float(cnt));
   leaf_sc[l] = make_uint2(first, cnt);
-  leaf_cell[l] = 0;      // a leaf of several cells: its cell box is leaf_cbox
+  leaf_cell[l] = 0;      // a leaf of several cells: each point's own cell counts
   leaf_al[l] = kNoCell;  // one cell per bucket (r.na == 1)
 }
 
@@ -606,16 +606,13 @@ __global__ void k_cells(const uint32_t *__restrict__ cell_start,
                  leaf_al, leaf_sc);
 }
 
-// Leaf bounding boxes, the corners of their points' cells, and initial keys
-// (FLT_MAX with the smallest rank of the leaf); empty leaves get an empty box
-// (its cell corners lo > hi) and key 0.  One wave per leaf.  cell_axis is
-// monotone, so the cells of the box's corners bound every point's cell.
-__device__ __forceinline__ void leaf_bbox_at(uint32_t leaf, uint32_t nleaves, const RangeDev &r,
+// Leaf bounding boxes and initial keys (FLT_MAX with the smallest rank of the
+// leaf); empty leaves get an empty box and key 0.  One wave per leaf.
+__device__ __forceinline__ void leaf_bbox_at(uint32_t leaf, uint32_t nleaves,
                                              const float4 *__restrict__ P4,
                                              const uint2 *__restrict__ RO,
                                              float4 *__restrict__ leaf_lo,
                                              float4 *__restrict__ leaf_hi,
-                                             uint2 *__restrict__ leaf_cbox,
                                              uint64_t *__restrict__ leaf_key,
                                              float4 *__restrict__ leaf_pos) {
   uint32_t lane = lane_id();
@@ -646,9 +643,6 @@ __device__ __forceinline__ void leaf_bbox_at(uint32_t leaf, uint32_t nleaves, co
   if (lane == 0) {
     leaf_lo[leaf] = make_float4(mnx, mny, mnz, lo.w);
     leaf_hi[leaf] = make_float4(mxx, mxy, mxz, hi.w);
-    leaf_cbox[leaf] =
-        make_uint2(cell_axis(r, 0, mnx) | (cell_axis(r, 1, mny) << 10) | (cell_axis(r, 2, mnz) << 20),
-                   cell_axis(r, 0, mxx) | (cell_axis(r, 1, mxy) << 10) | (cell_axis(r, 2, mxz) << 20));
     leaf_key[leaf] = km;
   }
   if (cnt == 0) {
@@ -658,16 +652,15 @@ __device__ __forceinline__ void leaf_bbox_at(uint32_t leaf, uint32_t nleaves, co
   }
 }
 
-__global__ __launch_bounds__(256) void k_leaf_bbox(uint32_t nleaves, RangeDev r,
+__global__ __launch_bounds__(256) void k_leaf_bbox(uint32_t nleaves,
                                                    const float4 *__restrict__ P4,
                                                    const uint2 *__restrict__ RO,
                                                    float4 *__restrict__ leaf_lo,
                                                    float4 *__restrict__ leaf_hi,
-                                                   uint2 *__restrict__ leaf_cbox,
                                                    uint64_t *__restrict__ leaf_key,
                                                    float4 *__restrict__ leaf_pos) {
-  leaf_bbox_at(blockIdx.x * 4 + (threadIdx.x >> 6), nleaves, r, P4, RO, leaf_lo, leaf_hi, leaf_cbox,
-               leaf_key, leaf_pos);
+  leaf_bbox_at(blockIdx.x * 4 + (threadIdx.x >> 6), nleaves, P4, RO, leaf_lo, leaf_hi, leaf_key,
+               leaf_pos);
 }
 
 // Level-1 nodes from the initial leaves: max key, its position, the union
@@ -907,7 +900,7 @@ hipError_t launch_leaf_build(const uint32_t *cell_start, const uint32_t *cell_le
                              uint32_t n, uint32_t nleaves, const RangeDev &r, const float4 *P4,
                              const uint2 *RO, float4 *leaf_lo, float4 *leaf_hi,
                              uint32_t *leaf_cell, uint32_t *leaf_al, uint2 *leaf_sc,
-                             uint2 *leaf_cbox, uint64_t *leaf_key, float4 *leaf_pos,
+                             uint64_t *leaf_key, float4 *leaf_pos,
                              uint2 *cell_info, hipStream_t st) {
   // the cell table has T + 1 entries; mixed leaves are described one a thread
   const uint64_t cells = (uint64_t)T + 1, threads = mixed && nleaves > cells ? nleaves : cells;
@@ -915,8 +908,8 @@ hipError_t launch_leaf_build(const uint32_t *cell_start, const uint32_t *cell_le
                                               nleaves, r, P4, cell_info, leaf_lo, leaf_hi,
                                               leaf_cell, leaf_al, leaf_sc);
   if (nleaves)
-    k_leaf_bbox<<<cdiv(nleaves, 4), 256, 0, st>>>(nleaves, r, P4, RO, leaf_lo, leaf_hi, leaf_cbox,
-                                                  leaf_key, leaf_pos);
+    k_leaf_bbox<<<cdiv(nleaves, 4), 256, 0, st>>>(nleaves, P4, RO, leaf_lo, leaf_hi, leaf_key,
+                                                  leaf_pos);
   return hipGetLastError();
 }
 
@@ -1006,9 +999,9 @@ __global__ void kb_cells(const BuildDev *__restrict__ bd) {
 
 __global__ __launch_bounds__(256) void kb_leaf_bbox(const BuildDev *__restrict__ bd) {
   const BuildDev &b = bd[blockIdx.y];
-  leaf_bbox_at(blockIdx.x * 4 + (threadIdx.x >> 6), b.c.nleaves, b.c.r, b.c.P4, b.c.RO,
+  leaf_bbox_at(blockIdx.x * 4 + (threadIdx.x >> 6), b.c.nleaves, b.c.P4, b.c.RO,
                const_cast<float4 *>(b.c.leaf_lo), const_cast<float4 *>(b.c.leaf_hi),
-               const_cast<uint2 *>(b.c.leaf_cbox), b.c.leaf_key, b.c.leaf_pos);
+               b.c.leaf_key, b.c.leaf_pos);
 }
 
 __global__ __launch_bounds__(256) void kb_l1_init(const BuildDev *__restrict__ bd) {

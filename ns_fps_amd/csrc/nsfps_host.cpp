@@ -795,6 +795,14 @@ int key_bits_for(uint32_t T) {
 // slots: cell -> leaf becomes arithmetic, no table lookup per iteration.
 uint64_t padded_slot_limit(uint32_t n) { return std::max<uint64_t>(4ull * n, 65536ull); }
 
+// Clouds of at most this many points keep their lists at kListShort entries:
+// longer ones hardly save rounds there (a CPU model: 30 rounds of the
+// 10,000-point quickstart at 1,024 as at 4,096 entries, but 57 against 41 of
+// a 120,000-point scan) and the pairs of many clouds' lists add up: 64 clouds
+// of 20,000 points 2.6 ms per call at 1,024 entries (39 rounds), 2.06 at 512
+// (42), 2.3 at 256 (56).
+constexpr uint32_t kShortListPoints = 32768;
+
 // Lays out the persistent buffers of one cloud (upper bounds: the padded /
 // dense decision is made on the device data during the build).
 void layout_cloud(Bump &bp, CloudPlan &p) {
@@ -817,7 +825,6 @@ void layout_cloud(Bump &bp, CloudPlan &p) {
   c.leaf_sc = bp.take<uint2>(leaves);
   c.leaf_cell = bp.take<uint32_t>(leaves);
   c.leaf_al = bp.take<uint32_t>(leaves * p.rng.dev.na);
-  c.leaf_cbox = bp.take<uint2>(leaves);
   c.leaf_key = bp.take<uint64_t>(leaves);
   c.leaf_pos = bp.take<float4>(leaves);
   c.l1_key = bp.take<uint64_t>(p.l1_ub);
@@ -831,12 +838,18 @@ void layout_cloud(Bump &bp, CloudPlan &p) {
   c.counter = bp.take<uint32_t>(1);
   c.prof = bp.take<uint64_t>(kProfWords);
   c.hist = bp.take<uint32_t>((size_t)kHists * kHistBins);
-  c.pick_p = bp.take<float4>(kListCap);
-  c.pick_c = bp.take<uint2>(kListCap);
   c.list_p = bp.take<float4>(kListCap);
   c.list_r = bp.take<uint2>(kListCap);
-  c.list_c = bp.take<uint32_t>(kListCap);
-  c.list_al = bp.take<uint32_t>((size_t)kListCap * p.rng.dev.na);
+  c.list_f = bp.take<uint32_t>(kListCap);
+  c.list_c = bp.take<uint2>(kListCap);
+  c.list_cap = n <= kShortListPoints ? kListShort : kListCap;
+  // every round settles a sample, and usually many; with a full log the later
+  // rounds share its last entry.  A plan learns m later: at most n.
+  const uint32_t mmax = p.m ? p.m : n;
+  c.log_cap = std::min<uint32_t>(std::max(kLogCap, mmax / 128), mmax + 1);
+  c.log_bmin = bp.take<uint64_t>(c.log_cap);
+  c.log_ktop = bp.take<uint64_t>(c.log_cap);
+  c.log_start = bp.take<uint32_t>(c.log_cap);
   c.lut = p.d_lut;
   c.n = n;
   c.m = p.m;
@@ -1165,7 +1178,7 @@ nsfps_status finish_cloud(CloudPlan &p, const uint32_t *lorig, const uint32_t *p
                             c.nleaves, p.rng.dev, c.P4, c.RO, const_cast<float4 *>(c.leaf_lo),
                             const_cast<float4 *>(c.leaf_hi), const_cast<uint32_t *>(c.leaf_cell),
                             const_cast<uint32_t *>(c.leaf_al), const_cast<uint2 *>(c.leaf_sc),
-                            const_cast<uint2 *>(c.leaf_cbox), c.leaf_key, c.leaf_pos,
+                            c.leaf_key, c.leaf_pos,
                             p.d_cell_info, st));
   HIP_TRY(launch_init_state(c, p.d_small + 2, st));
   c.lds = plan_lds(c);
@@ -1416,19 +1429,6 @@ struct RoundSchedule {
 };
 RoundSchedule g_schedule;
 
-// Rounds whose clouds all have at most this many points use the update pass
-// that also bounds each pick by each leaf's box of points (the bound's extra
-// work pays where cubes are large against the leaves: sparse clouds).
-// Measured on the MI355X: 10,000-point quickstart 1.04 -> 0.99 ms per call,
-// 120,000-point scan 4.55 -> 4.40; with it, the 1M-point uniform cube was
-// 1.8 % slower (0.6 % on the later kernels).
-constexpr uint32_t kLeafBoundMaxPoints = 262144;
-// Larger clouds whose filled buckets hold more than this many points on
-// average take it too: dense buckets fill several leaves each, and the bound
-// spares the leaves of a cube's cells that no pick can lower.  8M-point
-// clustered cloud (586 points a filled bucket) 61.25 against 61.79 ms per
-// call; the 1M-point uniform cube (32) was 7.28 against 7.24 with it.
-constexpr uint32_t kLeafBoundDensity = 64;
 // Rounds with at most this many level-1 nodes over all clouds split each
 // node's leaves over kUpdateSplit workgroups of the update pass (its work
 // then spreads over that many more CUs; a node's key is the largest of the
@@ -1438,36 +1438,20 @@ constexpr uint32_t kLeafBoundDensity = 64;
 // points (256 nodes) unchanged; the 1M-point uniform cube (512 nodes) 7.7 ->
 // 12.3 with it.
 constexpr uint32_t kSplitMaxNodes = 256;
-// Clouds whose points fill at least this many buckets are sampled with hot
-// sets of 128 copies.  The run's 1,024 list entries then average at most 4
-// in a cube of 3 x 3 x 3 cells, so the copies of a hot set seldom lower one
-// another and a set of 128 yields about twice the samples of a set of 64
-// (a CPU model of the acceptance rule on the 1M-point uniform cube's lists:
-// 84-118 samples against 53-63).  Where cubes hold many entries (clouds in
-// few cells, coarse grids, or many samples per point), the 128-copy sets
-// cost more than they yield.  Measured on the MI355X, 128 against 64
-// copies per call: 1M-point uniform cube (32,768 buckets filled) 7.35
-// against 7.69 ms, 8M-point clustered cloud (14,321) 62.4 against 70.6;
-// quickstart (8) 0.91 against 0.70, 120,000-point scan (1,266) 4.09 against
-// 3.90, 64 clouds of 16,384 points (about 2,530 each) 2.31 against 2.06.
+// Clouds whose points fill at least this many buckets report the density
+// class 128, others 64 (stats' hot_set; earlier versions' run kernel took
+// sets of that many copies).  No kernel depends on it.
 constexpr uint32_t kHot128MinCells = 6912;
-// Clouds whose points fill at most this many buckets take the run kernel that
-// applies a large-cube sample whose cube holds the list's cell box without a
-// cell test per entry.  The 10,000-point quickstart (8 buckets, every cube of
-// a positive distance holding every point), per call on the MI355X: 0.65-0.66
-// -> 0.62-0.63 ms (large-cube samples 4.5 k -> 3.2 k cycles a hot set).
-constexpr uint32_t kWholeMaxCells = 8;
 // Calls of at least this many clouds sample them in two halves on two
-// streams: each round's run kernel takes one CU per cloud, and one half's
-// update and gather passes then run on the other CUs beside the other half's
-// run kernel (clouds are independent).  NSFPS_STREAMS=n asks for n groups
+// streams: one half's passes run beside the other's, whose short launches
+// leave CUs idle (clouds are independent).  NSFPS_STREAMS=n asks for n groups
 // (at most kMaxStreams).  64 clouds of 16,384 points, per call on the
 // MI355X: one stream 1.94 ms, two 1.79-1.81, three 1.71-1.80.
 constexpr uint32_t kTwoStreamMinClouds = 8;
 constexpr uint32_t kStreamGroups = 2;
 
 // The shape of a call's sampling passes: the update pass's workgroups per
-// level-1 node and the run kernel's hot-set size (0 when the tree engine ran).
+// level-1 node and the density class (0 when the tree engine ran).
 struct PassShape {
   uint32_t split = 0, hot = 0;
 };
@@ -1478,37 +1462,25 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
                         const CloudStatus *d_status, hipStream_t st, bool profile,
                         uint64_t *rounds_out, PassShape *shape_out, hipEvent_t ev_end,
                         std::vector<CloudStatus> &fin) {
-  uint32_t max_nl1 = 1;
+  uint32_t max_nl1 = 1, list_cap = kListShort;
   bool alias = false;  // some cloud's cells share buckets
-  bool leaf_bound = true;  // every cloud small enough (or dense enough) for the leaf-box bound
-  bool dense = true;       // every cloud's filled buckets hold more than kLeafBoundDensity points
   for (auto &p : plans) {
     max_nl1 = std::max(max_nl1, p.dev.nl1);
     alias = alias || !p.rng.dev.bijective;
-    const bool d = (uint64_t)p.n > kLeafBoundDensity * std::max(1u, p.occupied);
-    leaf_bound = leaf_bound && (p.n <= kLeafBoundMaxPoints || d);
-    dense = dense && d;
+    list_cap = std::max(list_cap, p.dev.list_cap);
   }
-  if (const char *e = getenv("NSFPS_LEAF_BOUND")) leaf_bound = atoi(e) != 0;  // forced either way
-  if (const char *e = getenv("NSFPS_DENSE_WALK")) dense = atoi(e) != 0;
   const uint32_t nc = (uint32_t)plans.size();
   const bool mixed = plans[0].dev.mixed != 0;  // the same for every cloud of a call
   const bool split = (uint64_t)nc * max_nl1 <= kSplitMaxNodes;
-  // the run kernel's hot sets: 128 copies when every cloud's points fill at
-  // least kHot128MinCells buckets (and no cells share buckets); NSFPS_HOT=64
-  // or 128 forces either size
+  // the density class: 128 when every cloud's points fill at least
+  // kHot128MinCells buckets (and no cells share buckets); NSFPS_HOT=64 or 128
+  // forces either
   bool wide = !alias;
   for (auto &p : plans) wide = wide && p.occupied >= kHot128MinCells;
   const char *hot_env = getenv("NSFPS_HOT");
   if (hot_env && atoi(hot_env) == 64) wide = false;
   if (hot_env && atoi(hot_env) == 128) wide = !alias;
   const uint32_t hot = wide ? 128u : 64u;
-  // clouds in few buckets: their large cubes hold the whole list (a sample's
-  // cube is checked against the list's cell box in the kernel, so this only
-  // chooses the kernel); NSFPS_WHOLE=0 or 1 forces either
-  bool whole = !alias && hot == 64;
-  for (auto &p : plans) whole = whole && p.occupied <= kWholeMaxCells;
-  if (const char *e = getenv("NSFPS_WHOLE")) whole = atoi(e) != 0 && !alias && hot == 64;
   shape_out->split = split ? kUpdateSplit : 1u;
   shape_out->hot = hot;
   const uint64_t shape[5] = {nc, plans[0].n, plans[0].m, plans[0].rng.dev.T, max_nl1};
@@ -1522,7 +1494,7 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
   groups = std::min({groups, nc, kMaxStreams});
   const bool two = groups > 1;
   hipStream_t sts[kMaxStreams] = {st};
-  uint32_t g0[kMaxStreams + 1] = {}, gmax[kMaxStreams] = {};
+  uint32_t g0[kMaxStreams + 1] = {};
   Arena *ap2 = nullptr;
   if (two) {
     const nsfps_status rc = arena_for_device(&ap2);
@@ -1540,24 +1512,23 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
     for (uint32_t k = 1; k < groups; ++k) HIP_TRY(hipStreamWaitEvent(sts[k], ap2->fork, 0));
   }
   for (uint32_t k = 0; k <= groups; ++k) g0[k] = (uint32_t)((uint64_t)nc * k / groups);
-  for (uint32_t k = 0; k < groups; ++k) {
-    gmax[k] = 1;
-    for (uint32_t i = g0[k]; i < g0[k + 1]; ++i) gmax[k] = std::max(gmax[k], plans[i].dev.nl1);
-  }
+  uint64_t enqueued = 0;
   const auto enqueue = [&](uint32_t take, uint32_t np) -> hipError_t {
     if (!two)
-      return launch_rounds(d_clouds, nc, max_nl1, take, np, profile, alias, leaf_bound, split,
-                           mixed, hot, dense, whole, st);
+      return launch_rounds(d_clouds, nc, max_nl1, take, np, profile, alias, split, mixed,
+                           list_cap, (uint32_t)enqueued, st);
     for (uint32_t k = 0; k < groups; ++k) {
-      const hipError_t e = launch_rounds(d_clouds + g0[k], g0[k + 1] - g0[k], gmax[k], take, np,
-                                         profile, alias, leaf_bound, split, mixed, hot, dense,
-                                         whole, sts[k]);
+      const hipError_t e = launch_rounds(d_clouds + g0[k], g0[k + 1] - g0[k], max_nl1, take, np,
+                                         profile, alias, split, mixed, list_cap,
+                                         (uint32_t)enqueued, sts[k]);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
   };
+  uint32_t max_m = 0;
+  for (auto &p : plans) max_m = std::max(max_m, p.m);
   std::vector<CloudStatus> pr(nc);
-  uint64_t last_samples = 0, enqueued = 0;
+  uint64_t last_samples = 0;
   uint32_t batch = 4, stalled = 0, passes = 0;
   bool launched = false;  // rounds are in the queue and no status read has followed
   if (replay) {
@@ -1578,6 +1549,9 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
       used.emplace_back(batch, passes);
     }
     launched = false;
+    // the samples in order, once a cloud is done
+    for (uint32_t k = 0; k < groups; ++k)
+      HIP_TRY(launch_order(d_clouds + g0[k], g0[k + 1] - g0[k], max_m, sts[k]));
     for (uint32_t k = 1; k < groups; ++k) {  // the statuses are read on st once every group's rounds are done
       HIP_TRY(hipEventRecord(ap2->join[k - 1], sts[k]));
       HIP_TRY(hipStreamWaitEvent(st, ap2->join[k - 1], 0));
@@ -1591,16 +1565,11 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
     uint64_t samples = 0, rounds = 0;
     for (auto &q : pr) {
       if (q.rs.err) {
-        // 1: list overflow, 2: hot-copy overflow, 3: a live key above the hot
-        // histogram, 4: no crossing bin in a hot-threshold histogram
-        static const char *const what[] = {"", "list overflow", "hot-copy overflow",
-                                           "key above the hot histogram",
-                                           "no crossing bin in the hot histogram"};
-        return fail(NSFPS_EDEVICE, "internal: speculative run state: %s",
-                    q.rs.err < 5 ? what[q.rs.err] : "unknown");
+        return fail(NSFPS_EDEVICE, "internal: rounds engine state: %s",
+                    q.rs.err == 1 ? "list overflow" : "more samples than points");
       }
       all = all && q.done;
-      samples += q.iter;
+      samples += q.rs.ntaken;
       if (q.rs.forced) passes = kRefinePasses;
       rounds = std::max<uint64_t>(rounds, q.rs.rounds);
     }
@@ -1608,7 +1577,7 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
     if (all) {
       std::copy(shape, shape + 5, g_schedule.shape);
       g_schedule.batches = used;
-      g_schedule.rounds = rounds;
+      g_schedule.rounds = rounds + 1;  // and the one that finds the end
       fin = pr;
       break;
     }
@@ -1651,11 +1620,22 @@ void layout_all(Bump &bp, std::vector<CloudPlan> &plans, CallLayout &L) {
   layout_scratch(bp, L.nsort, L.tmax, L.sc);
   L.d_clouds = bp.take<CloudDev>(plans.size());
   L.d_status = bp.take<CloudStatus>(plans.size());
+  // the settled samples (at most a cloud's points): in the sorts' buffers,
+  // which the build is done with, where those hold every cloud's
+  size_t points = 0, at = 0;
+  for (auto &p : plans) points += p.n;
+  uint32_t *smp[3] = {L.sc.kA, L.sc.kB, L.sc.vA};
+  if (points > L.nsort)
+    for (auto &q : smp) q = bp.take<uint32_t>(points);
   if (bp.base)
     for (size_t i = 0; i < plans.size(); ++i) {
       plans[i].dev.done = &L.d_status[i].done;
       plans[i].dev.iter = &L.d_status[i].iter;
       plans[i].dev.rs = &L.d_status[i].rs;
+      plans[i].dev.smp_d = smp[0] + at;
+      plans[i].dev.smp_lo = smp[1] + at;
+      plans[i].dev.smp_row = smp[2] + at;
+      at += plans[i].n;
     }
 }
 
@@ -1675,7 +1655,7 @@ size_t measure_call(std::vector<CloudPlan> &plans, CallLayout &L) {
   return meas.off + 4096;
 }
 
-// The engine: speculative runs (for every grid; where cells share buckets its
+// The engine: rounds (for every grid; where cells share buckets its
 // kernels test every cell of a bucket), or the tree loop when
 // NSFPS_ENGINE=tree asks.
 bool choose_runs(std::vector<CloudPlan> &plans) {
@@ -1696,9 +1676,8 @@ bool small_wanted(const std::vector<CloudPlan> &plans) {
     if (p.n != plans[0].n || p.n > kSmallMaxPoints || p.rng.dev.T > (1u << kSmallMaxBits))
       return false;
   if (const char *e = getenv("NSFPS_SMALL")) return atoi(e) != 0;
-  for (const char *v : {"NSFPS_ENGINE", "NSFPS_NO_PADDED", "NSFPS_MIXED", "NSFPS_LEAF_BOUND",
-                        "NSFPS_STREAMS", "NSFPS_GLOBAL_SORT", "NSFPS_HOT", "NSFPS_DENSE_WALK",
-                        "NSFPS_WHOLE", "NSFPS_PROFILE", "NSFPS_INJECT"})
+  for (const char *v : {"NSFPS_ENGINE", "NSFPS_NO_PADDED", "NSFPS_MIXED", "NSFPS_STREAMS",
+                        "NSFPS_GLOBAL_SORT", "NSFPS_HOT", "NSFPS_PROFILE", "NSFPS_INJECT"})
     if (getenv(v)) return false;
   return true;
 }
@@ -1856,7 +1835,7 @@ nsfps_status run_small(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_host, 
 
 // Samples the built clouds (descriptors in plans[i].dev): grid-wide steps for
 // the first iterations of a single cloud on the tree engine, then its loop;
-// or the speculative-run rounds.
+// or the rounds.
 // fin: the runs engine's final statuses (left empty by the tree engine)
 nsfps_status sample_clouds(std::vector<CloudPlan> &plans, const CallLayout &L, const Ws &ws,
                            bool runs, uint64_t *rounds, uint64_t *wide_total,

@@ -25,10 +25,22 @@ constexpr uint32_t kCandCap = 1024;
 // Dynamic LDS budget of the single-workgroup loop (gfx950: 160 KiB per CU).
 constexpr uint32_t kLdsBudget = 160 * 1024 - 1024;
 constexpr uint32_t kNone = 0xffffffffu;
-// Speculative-run engine: list entries (one per thread of the run kernel; also
-// the most picks one run can accept), bins per key histogram, histograms per
-// round (one from the update pass, then two refinement passes).
-constexpr uint32_t kListCap = 1024;
+// Rounds engine: list entries (also the most samples a round can
+// settle), bins per key histogram, histograms per round (one from the update
+// pass, then two refinement passes).
+constexpr uint32_t kListCap = 4096;
+// A round's list takes at most kListGrow times the samples settled the round
+// before, at least kListMin and at most the cloud's list_cap entries: the
+// first rounds of a cloud settle few, however long their lists.
+constexpr uint32_t kListMin = 1024;
+constexpr uint32_t kListGrow = 4;
+// list_cap of small clouds (host's kShortListPoints)
+constexpr uint32_t kListShort = 512;
+// rounds in the log that orders the samples, for up to 131,072 samples (more
+// above; later rounds share its last entry)
+constexpr uint32_t kLogCap = 1024;
+// picks of one node the update pass holds in LDS at a time
+constexpr uint32_t kPickLds = 1024;
 // workgroups per level-1 node in the split update pass
 constexpr uint32_t kUpdateSplit = 4;
 constexpr uint32_t kHistBins = 4096;
@@ -85,19 +97,24 @@ struct LdsPlan {
   uint32_t total;         // bytes
 };
 
-// State of the speculative-run engine of one cloud, carried between the
+// State of the rounds engine of one cloud, carried between the
 // kernels of a round and from one round to the next.
 struct RunState {
   uint64_t kref0;     // every key is <= kref0 when the update pass runs
   uint64_t bkey;      // list threshold chosen by the selection
+  uint64_t ktop;      // no key was above this at the selection
+  uint64_t bmin;      // the smallest threshold so far
   uint32_t s0;        // bin shift of the update pass's key histogram
   uint32_t s0_next;   // bin shift proposed for the next round
-  uint32_t npicks;    // picks of the last run (applied by the next update pass)
-  uint32_t nlist;     // list entries gathered this round
+  uint32_t nb;        // bins of that histogram in use
+  uint32_t nb_next;
+  uint32_t nl[2];     // list entries, by the round's parity
+  uint32_t cap;       // the next list's capacity
+  uint32_t ntaken;    // samples settled and recorded
+  uint32_t nlog;      // rounds in the log
   uint32_t rounds;    // rounds that ran (statistics)
   uint32_t err;       // set if a list overflowed (internal error)
   uint32_t forced;    // rounds whose threshold was forced for want of refinement passes
-  uint32_t pad;
 };
 
 // Everything one cloud's kernels touch.  Device pointers; passed by value to
@@ -128,8 +145,6 @@ struct CloudDev {
   const uint2 *leaf_sc;       // first slot, point count (leaf_lo.w / leaf_hi.w packed)
   const uint32_t *leaf_cell;  // ix | iy << 10 | iz << 20
   const uint32_t *leaf_al;    // r.na per leaf: the cells of its bucket, kNoCell-padded
-  const uint2 *leaf_cbox;     // lo / hi corners of the cells of the leaf's points (10 bits
-                              // per axis; lo > hi on some axis: no points)
   uint64_t *leaf_key;         // max key of the leaf
   float4 *leaf_pos;           // x, y, z, input row (bits) of that key
   uint64_t *l1_key;
@@ -147,16 +162,21 @@ struct CloudDev {
   uint32_t *counter;          // arrival counter of the grid-wide step
   int32_t *out;               // m entries
   uint64_t *prof;             // loop phase clocks / counters, or null
-  // speculative-run engine
+  // rounds engine
   RunState *rs;
   uint32_t *hist;             // kHists x kHistBins
-  float4 *pick_p;             // kListCap: x, y, z, D of each pick of a run
-  uint2 *pick_c;              // kListCap: cube lo / hi cells, 11 bits per axis with guard bits
-                              // (lo, hi | guards: the run kernel's box-test form)
   float4 *list_p;             // kListCap: x, y, z, min distance
   uint2 *list_r;              // kListCap: logical rank, input row
-  uint32_t *list_c;           // kListCap: cell (10 bits per axis)
-  uint32_t *list_al;          // kListCap x r.na: the cells of each entry's bucket
+  uint32_t *list_f;           // kListCap: 0 when the entry is settled (a sample)
+  uint2 *list_c;              // kListCap: its cube's lo / hi cells as a sample, 11 bits per axis
+                              // with guard bits (lo, hi | guards: the box-test form)
+  uint32_t *smp_d;            // n: settled samples' distance bits,
+  uint32_t *smp_lo;           //    ~logical ranks
+  uint32_t *smp_row;          //    and input rows
+  uint64_t *log_bmin;         // log_cap: per round, the smallest threshold so far,
+  uint64_t *log_ktop;         //    a bound on its keys
+  uint32_t *log_start;        //    and the samples before it
+  uint32_t list_cap, log_cap;
 };
 
 // Argmax key: larger min-distance wins, equal distances go to the smaller

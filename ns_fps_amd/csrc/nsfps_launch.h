@@ -86,7 +86,7 @@ hipError_t launch_leaf_build(const uint32_t *cell_start, const uint32_t *cell_le
                              uint32_t n, uint32_t nleaves, const RangeDev &r, const float4 *P4,
                              const uint2 *RO, float4 *leaf_lo, float4 *leaf_hi,
                              uint32_t *leaf_cell, uint32_t *leaf_al, uint2 *leaf_sc,
-                             uint2 *leaf_cbox, uint64_t *leaf_key, float4 *leaf_pos,
+                             uint64_t *leaf_key, float4 *leaf_pos,
                              uint2 *cell_info, hipStream_t st);
 hipError_t launch_init_state(const CloudDev &c, const uint32_t *d_phys0, hipStream_t st);
 
@@ -133,23 +133,21 @@ hipError_t launch_late_loop(const CloudDev *d_clouds, uint32_t nclouds, uint32_t
                             bool profile, uint32_t threads, hipStream_t st);
 constexpr uint32_t kProfWords = 64;
 
-// speculative-run engine
+// rounds engine
 // split: the rounds' update pass is split (node keys move into their parts)
-hipError_t launch_runs_init(const CloudDev *d_clouds, uint32_t nclouds, bool split,
+hipError_t launch_runs_init(const CloudDev *d_clouds, uint32_t nclouds, uint32_t split,
                             hipStream_t st);
-// `rounds` rounds of update pass, refinement passes, gather pass and run.
-// alias: some cloud's cells share buckets.  leaf_bound: the update pass also
-// bounds each pick by each leaf's box; split: it takes kUpdateSplit
-// workgroups per level-1 node; mixed: the clouds' leaves are runs of 64 slots
-// that may hold several buckets (never with alias).  hot: the run kernel's
-// hot-set size, 64 or 128 (with alias always 64); dense: with 128, the walk
-// for clouds whose filled buckets hold many points; whole: with 64 and no
-// alias, the run kernel that applies a large-cube sample holding the list's
-// cell box with no cell test (for clouds in few buckets).
+// `rounds` rounds of update, refinement, gather and accept passes.
+// alias: some cloud's cells share buckets; split: the update pass takes
+// kUpdateSplit workgroups per level-1 node; mixed: the clouds' leaves are runs of 64 slots
+// that may hold several buckets (never with alias).  list_cap: the clouds'
+// longest list; first: the rounds enqueued before for these clouds.
 hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t max_nl1,
                          uint32_t rounds, uint32_t passes, bool profile, bool alias,
-                         bool leaf_bound, bool split, bool mixed, uint32_t hot, bool dense,
-                         bool whole, hipStream_t st);
+                         bool split, bool mixed, uint32_t list_cap, uint32_t first,
+                         hipStream_t st);
+// The samples of every finished cloud (at most m each) into its out, in order.
+hipError_t launch_order(const CloudDev *d_clouds, uint32_t nclouds, uint32_t m, hipStream_t st);
 
 // small clouds: nclouds clouds of n <= kSmallMaxPoints points each (devs[b];
 // or, nclouds = 1, *one, which the sort leaves in devs[0])

@@ -1,28 +1,43 @@
-// Speculative-run sampling engine (gfx950).
+// Round-based sampling engine (gfx950).
 //
-// Keys (min-distance bits << 32 | ~logical rank) only ever decrease.  Take a
-// threshold key B and the list of every point whose key is >= B: a point
-// outside the list stays below B for the rest of the sampling, so while the
-// list's maximum is >= B it is the global maximum, i.e. the reference's next
-// sample (src/yuezu_fps.cpp:703-722).  The run kernel holds the list in one
-// workgroup (one entry per thread) and takes samples from it one after
-// another, applying each sample's cube update (src/yuezu_fps.cpp:560-597) to
-// the list alone, until the list maximum drops below B or sampling ends.
+// Keys (min-distance bits << 32 | ~logical rank) only ever decrease, and the
+// reference takes the point of the largest key each time
+// (src/yuezu_fps.cpp:703-722).  Take a threshold key B and the list of every
+// point whose key is >= B, and call two points in conflict when their squared
+// distance is below the larger of their min-distances: only then can either
+// lower the other.  A listed point that conflicts with none of a larger key
+// is a sample with the key it has (k_accept gives the proof); all such points
+// of a list are settled at once, over the whole chip, and the samples' order
+// is the order of their keys, found once at the end.  The sampling ends when
+// m samples have keys above every key left, or only points at distance 0 are
+// left.
 //
-// A grid-wide pass then applies every sample of the run to every point.
-// min() of exact fp32 distances commutes, so each point ends with the same
-// bits as after the reference's one-by-one updates.  The same pass rebuilds
-// the leaf and level-1 keys and histograms the keys for the next threshold.
+// A grid-wide pass applies a round's samples to every point (each sample's
+// cube update, src/yuezu_fps.cpp:560-597).  min() of exact fp32 distances
+// commutes, so a point's distance has the same bits as after the reference's
+// one-by-one updates by the time its key counts.  The same pass rebuilds the
+// leaf and level-1 keys and histograms the keys for the next threshold.
 // Only the keys: the samples come from the list, so the winners' positions
 // (leaf_pos, l1_pos, which the tree engine keeps) are not maintained.
 //
 // One round, in stream order:
-//   k_update     picks -> points, leaf and level-1 keys, key histogram
+//   k_update     samples -> points, leaf and level-1 keys, key histogram
 //   k_refine x2  finer histograms inside the crossing bin, only when needed
-//   k_gather     threshold B (<= kListCap keys above it), list of those points
-//   k_run        samples from the list
-// The first round's only pick is input row 0 with a cube covering the whole
+//   k_gather     threshold B (<= list_cap keys above it), list of those points
+//   k_accept     the list's conflicts: its samples and their cubes
+// and after the last one k_sort_rounds and k_order, the samples' order.
+// The first round's only sample is input row 0 with a cube covering the whole
 // grid: the reference's first full pass (src/yuezu_fps.cpp:431-438).
+//
+// What bounds it: the rounds' launches (three of 5 to 17 us each; the points
+// that a round touches are read from cache) times the rounds.  They are few:
+// samples settle as soon as the few larger keys near them have, so a round of
+// 4,096 listed points settles some 800 to 1,300.  Per call on one MI355X, device-resident,
+// against lists sampled one after another by one workgroup: 120,000-point
+// scan -> 16,384 (55 rounds) 3.65 -> 1.38 ms, 1M-point cube -> 65,536 (82)
+// 7.02 -> 2.56, the same on 30^3 cells 10.6 -> 3.95, 8M clustered points ->
+// 524,288 (292) 59 -> 17.9, 1M -> 524,288 (236) 38 -> 7.2.  Clouds in few
+// samples gain least: 17,000 -> 64 0.34 -> 0.37 ms, 14 rounds for 7.
 //
 // The cube test compares cell coordinates.  Where cells share buckets (block
 // counts that are not powers of two: the Morton code is taken modulo the
@@ -91,30 +106,19 @@ __device__ __forceinline__ uint64_t node_key(const CloudDev &c, uint32_t g) {
   return k;
 }
 
-// Cube overlapping the cell range [lo, hi] (packed corners).
-__device__ __forceinline__ bool cube_overlaps(uint2 cube, uint32_t lo, uint32_t hi) {
-  bool ok = true;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const uint32_t s = 10u * a;
-    ok &= ((cube.x >> s) & 1023u) <= ((hi >> s) & 1023u);
-    ok &= ((cube.y >> s) & 1023u) >= ((lo >> s) & 1023u);
-  }
-  return ok;
-}
-
-// Histogram window of a selection pass: kHistBins bins of 2^S keys each, bin
-// 0 ending at kref.  Lowest key inside the window:
-__device__ __forceinline__ uint64_t window_lo(uint64_t kref, uint32_t S) {
+// Histogram window of a selection pass: nb bins of 2^S keys each, bin 0 ending
+// at kref (S = kMaxShift: all keys).  Lowest key inside the window:
+__device__ __forceinline__ uint64_t window_lo(uint64_t kref, uint32_t S, uint32_t nb = kHistBins) {
   if (S >= kMaxShift) return 0;
-  const uint64_t w = ((uint64_t)kHistBins << S) - 1;
+  const uint64_t w = ((uint64_t)nb << S) - 1;
   return kref >= w ? kref - w : 0;
 }
 
-__device__ __forceinline__ uint32_t key_bin(uint64_t key, uint64_t kref, uint32_t S) {
+__device__ __forceinline__ uint32_t key_bin(uint64_t key, uint64_t kref, uint32_t S,
+                                            uint32_t nb = kHistBins) {
   if (key > kref) return kNone;
   const uint64_t b = (kref - key) >> S;
-  return b < kHistBins ? (uint32_t)b : kNone;
+  return b < nb ? (uint32_t)b : kNone;
 }
 
 // The key histograms (kHists of kHistBins each): the update pass counts
@@ -142,15 +146,17 @@ struct Sel {
   uint32_t state;    // 0: refinement pass `pass` needed, 1: resolved, 2: use the maximum key
   uint32_t pass;
   uint32_t win;      // keys inside the update pass's histogram window
+  uint64_t ktop;     // no key is above this (0 when the window is empty)
 };
 
 struct Step {
   uint32_t tot;     // keys in the window
   uint32_t bs;      // crossing bin, kNone when tot <= cap
   uint32_t before;  // keys in the bins before it
+  uint32_t first;   // first bin that holds a key, kNone when none does
 };
 
-// Block-wide, all kPassThreads threads; sc holds kPassWaves + 2 words of LDS.
+// Block-wide, all kPassThreads threads; sc holds kPassWaves + 3 words of LDS.
 // h: this thread's four bins of the histogram.
 __device__ Step hist_step(uint4 h, uint32_t cap, uint32_t *sc) {
   const uint32_t tid = threadIdx.x;
@@ -164,6 +170,7 @@ __device__ Step hist_step(uint4 h, uint32_t cap, uint32_t *sc) {
       sc[kPassWaves] = 4 * tid + j;
       sc[kPassWaves + 1] = c;
     }
+    if (c == 0 && bins[j]) sc[kPassWaves + 2] = 4 * tid + j;  // one thread, once
     c += bins[j];
   }
   __syncthreads();
@@ -171,6 +178,7 @@ __device__ Step hist_step(uint4 h, uint32_t cap, uint32_t *sc) {
   st.tot = tot;
   st.bs = tot <= cap ? kNone : sc[kPassWaves];
   st.before = tot <= cap ? 0u : sc[kPassWaves + 1];
+  st.first = tot ? sc[kPassWaves + 2] : kNone;
   __syncthreads();
   return st;
 }
@@ -191,24 +199,26 @@ __device__ Sel sel_replay(const CloudDev &c, uint32_t avail, uint32_t passes, ui
   s.kref = rs.kref0;
   s.bkey = 0;
   s.S = rs.s0;
-  s.cap = kListCap;
+  s.cap = min(max(rs.cap, 1u), kListCap);
+  const uint32_t cap0 = s.cap;
   s.total = 0;
   s.state = 0;
   s.pass = 0;
   const uint32_t *H0 = c.hist;
   Step st = h0 ? hist_step(*h0, s.cap, sc) : hist_step(H0, s.cap, sc);
   s.win = st.tot;
+  s.ktop = st.first == kNone ? 0ull : s.kref - ((uint64_t)st.first << s.S);
   for (uint32_t p = 0;; ++p) {
     if (st.bs == kNone) {  // the whole window fits
       s.total += st.tot;
-      s.bkey = window_lo(s.kref, s.S);
+      s.bkey = window_lo(s.kref, s.S, p ? kHistBins : rs.nb);
       s.state = s.total ? 1u : 2u;
       return s;
     }
     s.total += st.before;
     if (st.before >= s.cap / 2 || s.S == 0 || p == passes) {
       // forced, and the list under a quarter full: refinement would have paid
-      if (forced) *forced = st.before < s.cap / 2 && s.S != 0 && s.total < kListCap / 4;
+      if (forced) *forced = st.before < s.cap / 2 && s.S != 0 && s.total < cap0 / 4;
       s.bkey = s.kref - ((uint64_t)st.bs << s.S) + 1;  // keys above bin bs
       s.state = s.total ? 1u : 2u;
       return s;
@@ -226,6 +236,63 @@ __device__ Sel sel_replay(const CloudDev &c, uint32_t avail, uint32_t passes, ui
 
 __device__ __forceinline__ const NSFPS_GLOBAL RunState &rstate(const CloudDev &c) {
   return *gptr(c.rs);
+}
+
+// ------------------------------------------------------------ the samples
+
+// By one workgroup of the update pass: the last list's settled entries join
+// the samples (keys and rows), with a log entry per round: the samples
+// before it, the smallest threshold up to it and the largest key in it.
+__device__ void record_samples(const CloudDev &c, uint32_t par, uint32_t *sc) {
+  const uint32_t tid = threadIdx.x;
+  NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
+  const uint32_t nl = min(rs.nl[par ^ 1u], kListCap), base = rs.ntaken, nlog = rs.nlog;
+  const uint64_t bkey = rs.bkey, bmin = rs.bmin, ktop = rs.ktop;
+  const uint32_t done = *gptr(c.done);
+  constexpr uint32_t kSlots = kListCap / kPassThreads;
+  bool take[kSlots];
+  float4 p[kSlots];
+  uint2 r[kSlots];
+  uint32_t n = 0;
+#pragma unroll
+  for (uint32_t s = 0; s < kSlots; ++s) {
+    const uint32_t i = kSlots * tid + s;
+    p[s] = gptr(c.list_p)[i];
+    r[s] = gptr(c.list_r)[i];
+    take[s] = i < nl && gptr(c.list_f)[i] == 0u;
+    n += take[s] ? 1u : 0u;
+  }
+  if (done) return;
+  uint32_t total;
+  uint32_t at = base + block_excl_scan<kPassWaves>(n, sc, &total);
+#pragma unroll
+  for (uint32_t s = 0; s < kSlots; ++s) {
+    if (take[s]) {
+      if (at < c.n) {
+        gptr(c.smp_d)[at] = __float_as_uint(p[s].w);
+        gptr(c.smp_lo)[at] = ~r[s].x;
+        gptr(c.smp_row)[at] = r[s].y;
+      } else {
+        rs.err = 2;  // cannot happen (a point is settled once)
+      }
+      ++at;
+    }
+  }
+  if (tid == 0) {
+    const uint64_t b = bkey < bmin ? bkey : bmin;
+    rs.bmin = b;
+    rs.ntaken = base + total;
+    *gptr(c.iter) = min(base + total, c.m);
+    rs.cap = min(max(kListGrow * total, kListMin), c.list_cap);
+    // a full log's last entry stands for all later rounds
+    const uint32_t i = nlog < c.log_cap ? nlog : c.log_cap - 1;
+    gptr(c.log_bmin)[i] = b;
+    if (nlog < c.log_cap) {
+      gptr(c.log_ktop)[i] = ktop;
+      gptr(c.log_start)[i] = base;
+      rs.nlog = nlog + 1;
+    }
+  }
 }
 
 // ------------------------------------------------------------ update pass
@@ -247,27 +314,30 @@ __device__ __forceinline__ const NSFPS_GLOBAL RunState &rstate(const CloudDev &c
 // ALIAS: cells share buckets, and a pick touches a leaf when its cube holds
 // any cell of the leaf's bucket (src/yuezu_fps.cpp:573-597 updates every point
 // of every bucket of the cube's cells); nodes are screened by the corners of
-// those cells.  LB: a pick also takes part in a leaf only if its distance
-// bound to the leaf's box is below the leaf key's distance (the node test
-// again, per leaf).  SPLIT: the node's leaves are split over SPLIT
-// workgroups, each storing the largest key of its leaves as one of the
+// those cells.  SPLIT: the node's leaves are split over SPLIT workgroups, each
+// storing the largest key of its leaves as one of the
 // node's parts (node_key reads the node's key back as the largest part).
 // MIXED: a leaf is a run of 64 slots of the logical order and may hold
-// several buckets (one cell each); a pick touches the leaf when its cube
-// overlaps the leaf's cell box, and lowers a point only when the point's own
-// cell lies in the cube (the reference's rule, point by point).
-template <bool PROF, bool ALIAS, bool LB, uint32_t SPLIT, bool MIXED>
-__global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60))) void k_update(
-    const CloudDev *__restrict__ clouds) {
+// several buckets (one cell each); a pick lowers a point only when the point's
+// own cell lies in the cube (the reference's rule, point by point).
+template <bool PROF, bool ALIAS, uint32_t SPLIT, bool MIXED>
+__global__ __launch_bounds__(kPassThreads) __attribute__((amdgpu_num_sgpr(60), amdgpu_waves_per_eu(8, 8))) void k_update(
+    const CloudDev *__restrict__ clouds, uint32_t round) {
   static_assert(!(ALIAS && MIXED), "leaves of several buckets need one cell per bucket");
   __shared__ uint32_t s_hist[kHistBins];
-  __shared__ float4 s_pp[kListCap];
-  __shared__ uint2 s_pc[kListCap];  // the picks' cube corners: pack11(lo), pack11(hi) | kGuards
+  __shared__ float4 s_pp[kPickLds];
+  __shared__ uint2 s_pc[kPickLds];  // the picks' cube corners: pack11(lo), pack11(hi) | kGuards
+  __shared__ uint16_t s_more[kListCap - kPickLds];  // the node's picks past kPickLds
   __shared__ uint64_t s_lk[kFan];
   __shared__ uint32_t s_np;
   __shared__ uint32_t s_ct[4];  // PROF: leaves and points read by the workgroup, and of them touched
   __shared__ uint32_t s_wt[PROF ? 3 * kPassWaves : 1];  // PROF: per-wave clocks
   const CloudDev &c = clouds[blockIdx.y];
+  const uint32_t par = round & 1u;
+  if (blockIdx.x + 1 == gridDim.x) {  // the last workgroup records the last list's samples
+    if (round) record_samples(c, par, s_hist);
+    return;
+  }
   // SPLIT workgroups per node: this one takes leaves sub * kFan / SPLIT ..
   constexpr uint32_t kLPW = kLeavesPerWave / SPLIT;  // leaves per wave
   static_assert(kLPW >= 1 && kLPW * SPLIT == kLeavesPerWave, "whole leaves per wave");
@@ -278,30 +348,19 @@ __global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60)
   const uint32_t leaf0 = g * kFan + sub * (kFan / SPLIT) + wave * kLPW;
   uint64_t mkey = 0;
   uint32_t mcell = 0, mst = 0, mcnt = 0;
-  uint32_t mchi = 0;  // MIXED: the leaf's cell box is mcell .. mchi
-  // LB (leaf bounds): the leaf's box of points (an absent leaf's stays empty)
-  constexpr bool lbound = LB;
   float4 mlo = make_float4(0.f, 0.f, 0.f, 0.f), mhi = mlo;
   if (lane < kLPW && leaf0 + lane < c.nleaves) {
     mkey = gptr(c.leaf_key)[leaf0 + lane];
-    if (MIXED) {
-      const uint2 cb = gptr(c.leaf_cbox)[leaf0 + lane];
-      mcell = cb.x;
-      mchi = cb.y;
-    } else {
-      mcell = gptr(c.leaf_cell)[leaf0 + lane];
-    }
+    if (!MIXED && !ALIAS) mcell = gptr(c.leaf_cell)[leaf0 + lane];
     const uint2 sc = gptr(c.leaf_sc)[leaf0 + lane];
     mst = sc.x;
     mcnt = sc.y;
-    if (lbound) {
-      mlo = gptr(c.leaf_lo)[leaf0 + lane];
-      mhi = gptr(c.leaf_hi)[leaf0 + lane];
-    }
+    mlo = gptr(c.leaf_lo)[leaf0 + lane];
+    mhi = gptr(c.leaf_hi)[leaf0 + lane];
   }
   const NSFPS_GLOBAL RunState &rs = rstate(c);
   const uint32_t done = *gptr(c.done);
-  const uint32_t npicks = min(rs.npicks, kListCap);
+  const uint32_t npicks = min(rs.nl[par ^ 1u], kListCap);
   const uint64_t kref = rs.kref0;
   const uint32_t S = rs.s0;
   const uint32_t gn = g < c.nl1 ? g : 0u;  // read unconditionally, used only if g < nl1
@@ -334,7 +393,8 @@ __global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60)
     clo = pack_cell(cell_axis(c.r, 0, nlo.x), cell_axis(c.r, 1, nlo.y), cell_axis(c.r, 2, nlo.z));
     chi = pack_cell(cell_axis(c.r, 0, nhi.x), cell_axis(c.r, 1, nhi.y), cell_axis(c.r, 2, nhi.z));
   }
-  const uint64_t wlo = window_lo(kref, S);
+  const uint32_t nb = rs.nb;
+  const uint64_t wlo = window_lo(kref, S, nb);
   // the node's cell range in the picks' box-test form
   const uint32_t clo11 = pack11(clo), chi11g = pack11(chi) | kGuards;
   for (uint32_t j = tid; j < kHistBins; j += kPassThreads) s_hist[j] = 0;
@@ -342,89 +402,103 @@ __global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60)
   if (PROF && tid < 4) s_ct[tid] = 0;
   __syncthreads();
   if (PROF) utb = __builtin_amdgcn_s_memrealtime();
-  for (uint32_t i = tid; i < npicks; i += kPassThreads) {
-    const uint2 cb = gptr(c.pick_c)[i];
-    const float4 pp = gptr(c.pick_p)[i];
-    const float px = pp.x, py = pp.y, pz = pp.z;
-    const uint32_t c0 = cb.x, c1 = cb.y;
-    pin_vgpr(c0, c1, px, py, pz);  // both reads in flight together
-    // the cube overlaps the node's cells (cube lo <= node hi and node lo <=
-    // cube hi on every axis: the guard test of in_box11 crosswise), and the
-    // pick may lower one of its points (the node key holds their largest
-    // distance)
-    if (in_box11(c1, c0, clo11, chi11g) &&
-        !(box_bound(px, py, pz, nlo.x, nlo.y, nlo.z, nhi.x, nhi.y, nhi.z) >=
+  // every thread's list entries are read together (entries past the list are
+  // stale and unused)
+  constexpr uint32_t kPickSlots = kListCap / kPassThreads;
+  uint2 pcb[kPickSlots];
+  float4 ppp[kPickSlots];
+  uint32_t ppf[kPickSlots];
+#pragma unroll
+  for (uint32_t s = 0; s < kPickSlots; ++s) {
+    if (s == 0 || s * kPassThreads < npicks) {
+      pcb[s] = gptr(c.list_c)[s * kPassThreads + tid];
+      ppp[s] = gptr(c.list_p)[s * kPassThreads + tid];
+      ppf[s] = gptr(c.list_f)[s * kPassThreads + tid];
+    }
+  }
+#pragma unroll
+  for (uint32_t s = 0; s < kPickSlots; ++s) {
+    const uint32_t i = s * kPassThreads + tid;
+    if (s * kPassThreads >= npicks) break;  // uniform
+    // a settled entry (a pick) whose cube overlaps the node's cells (cube lo
+    // <= node hi and node lo <= cube hi on every axis: the guard test of
+    // in_box11 crosswise), and that may lower one of its points (the node
+    // key holds their largest distance)
+    if (i < npicks && ppf[s] == 0u && in_box11(pcb[s].y, pcb[s].x, clo11, chi11g) &&
+        !(box_bound(ppp[s].x, ppp[s].y, ppp[s].z, nlo.x, nlo.y, nlo.z, nhi.x, nhi.y, nhi.z) >=
           __uint_as_float((uint32_t)(nkey >> 32)))) {
       const uint32_t k = atomicAdd(&s_np, 1u);
-      s_pp[k] = make_float4(px, py, pz, 0.f);
-      s_pc[k] = make_uint2(c0, c1);
+      if (k < kPickLds) {
+        s_pp[k] = make_float4(ppp[s].x, ppp[s].y, ppp[s].z, 0.f);
+        s_pc[k] = pcb[s];
+      } else {
+        s_more[k - kPickLds] = (uint16_t)i;
+      }
     }
   }
   __syncthreads();
-  const uint32_t nsel = s_np;
+  const uint32_t nall = s_np;
   const uint64_t ut1 = PROF ? __builtin_amdgcn_s_memrealtime() : 0;
-  if (nsel == 0 && nkey < wlo) return;  // nothing changes, nothing to count
-  // which leaves a pick touches (hm: the first 64 picks whose cube holds the
-  // leaf's cell), and which must be read
-  uint32_t c11[kLPW], st[kLPW], cnt[kLPW];
-  uint32_t ch11g[MIXED ? kLPW : 1];  // MIXED: pack11 of the leaf's cell box hi, with guards
+  if (nall == 0 && nkey < wlo) return;  // nothing changes, nothing to count
+  // which leaves a pick may lower a point of (hm: the first 64 picks), and
+  // which must be read
+  uint32_t st[kLPW], cnt[kLPW];
   uint64_t okey[kLPW], hm[kLPW];
   bool hit[kLPW], need[kLPW];
-  // pick i's cube (its s_pc record) holds (a cell of the bucket of) leaf k.
-  // Testing the leaf's box against the pick as the node's is tested costs
-  // more here than the reads it saves on points that fill their cells.
-  const auto touches_pick = [&](uint32_t k, uint2 cube) -> bool {
-    uint32_t in;
-    if (MIXED) {  // the cube overlaps the leaf's cell box (in_box11 crosswise)
-      in = in_box11(cube.y, cube.x, c11[k], ch11g[MIXED ? k : 0]);
-    } else if (!ALIAS) {
-      in = in_box11(c11[k] | kGuards, c11[k], cube.x, cube.y);
-    } else if (na == 2) {
-      const uint32_t a0 = pack11(rdlane(mal, 2 * k)), a1 = pack11(rdlane(mal, 2 * k + 1));
-      in = in_box11(a0 | kGuards, a0, cube.x, cube.y) | in_box11(a1 | kGuards, a1, cube.x, cube.y);
-    } else {
-      in = 0;
-      for (uint32_t a = 0; a < na; ++a) {
-        const uint32_t a0 = pack11(rdlane(mal, k * na + a));
-        in |= in_box11(a0 | kGuards, a0, cube.x, cube.y);
-      }
+  uint32_t nsel = min(nall, kPickLds);
+#pragma unroll
+  for (uint32_t k = 0; k < kLPW; ++k) {
+    okey[k] = ((uint64_t)rdlane((uint32_t)(mkey >> 32), k) << 32) | rdlane((uint32_t)mkey, k);
+    st[k] = rdlane(mst, k);
+    cnt[k] = rdlane(mcnt, k);
+  }
+  // A pick takes part in leaf k only if its squared distance to the leaf's
+  // box (in sqdist's operation order, so never above a point's distance) is
+  // below the leaf key's distance, the largest of its points: otherwise it
+  // lowers none of them.
+  const auto may_lower = [&](uint32_t k, float4 q) -> bool {
+    return !(box_bound(q.x, q.y, q.z, __uint_as_float(rdlane(__float_as_uint(mlo.x), k)),
+                       __uint_as_float(rdlane(__float_as_uint(mlo.y), k)),
+                       __uint_as_float(rdlane(__float_as_uint(mlo.z), k)),
+                       __uint_as_float(rdlane(__float_as_uint(mhi.x), k)),
+                       __uint_as_float(rdlane(__float_as_uint(mhi.y), k)),
+                       __uint_as_float(rdlane(__float_as_uint(mhi.z), k))) >=
+             __uint_as_float((uint32_t)(okey[k] >> 32)));
+  };
+  // A pick of this cube updates the lane's point (lanes of leaf k): the cube
+  // holds the cell of the point's bucket.  A pick nearer to a point than the
+  // point's distance nearly always passes, so this is looked at only for
+  // those; with shared buckets a leaf's box can span the grid, and the test
+  // (any cell of the bucket) goes ahead of the points.
+  const auto in_cube = [&](uint32_t k, uint32_t pc11, uint2 cube) -> bool {
+    if (ALIAS) return true;
+    const uint32_t a0 = MIXED ? pc11 : pack11(rdlane(mcell, k));
+    return in_box11(a0 | kGuards, a0, cube.x, cube.y) != 0;
+  };
+  const auto touches = [&](uint32_t k, uint32_t i) -> bool {
+    if (!ALIAS) return true;
+    const uint2 cube = s_pc[i];
+    uint32_t in = 0;
+    for (uint32_t a = 0; a < na; ++a) {
+      const uint32_t a0 = pack11(rdlane(mal, k * na + a));
+      in |= in_box11(a0 | kGuards, a0, cube.x, cube.y);
     }
     return in != 0;
   };
-  const auto touches = [&](uint32_t k, uint32_t i) -> bool { return touches_pick(k, s_pc[i]); };
-  // the first 64 picks' cubes, lane i holding pick i's, read once for the
-  // four leaves (past nsel: stale LDS, masked out)
-  const uint2 pc0 = s_pc[lane];
+  // kPickLds picks at a time: a node rarely has more (few nodes, many
+  // samples a round), and the last of these passes counts the keys
+  for (uint32_t ch = 0;;) {
+  const bool last = nall - ch <= kPickLds;
   const bool in0 = lane < nsel;
-  const float4 pp0 = lbound ? s_pp[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float4 pp0 = s_pp[lane];  // past nsel: stale LDS, masked out
 #pragma unroll
   for (uint32_t k = 0; k < kLPW; ++k) {
-    c11[k] = pack11(rdlane(mcell, k));
-    if (MIXED) ch11g[MIXED ? k : 0] = pack11(rdlane(mchi, k)) | kGuards;
-    st[k] = rdlane(mst, k);
-    cnt[k] = rdlane(mcnt, k);
-    okey[k] = ((uint64_t)rdlane((uint32_t)(mkey >> 32), k) << 32) | rdlane((uint32_t)mkey, k);
-    // with leaf bounds, a pick takes part in leaf k only if its squared
-    // distance to the leaf's box (in sqdist's operation order, so never above
-    // a point's distance) is below the leaf key's distance, the largest of
-    // its points: otherwise it lowers none of them
-    const float lmax = __uint_as_float((uint32_t)(okey[k] >> 32));
-    const float4 blo = make_float4(__uint_as_float(rdlane(__float_as_uint(mlo.x), k)),
-                                   __uint_as_float(rdlane(__float_as_uint(mlo.y), k)),
-                                   __uint_as_float(rdlane(__float_as_uint(mlo.z), k)), 0.f);
-    const float4 bhi = make_float4(__uint_as_float(rdlane(__float_as_uint(mhi.x), k)),
-                                   __uint_as_float(rdlane(__float_as_uint(mhi.y), k)),
-                                   __uint_as_float(rdlane(__float_as_uint(mhi.z), k)), 0.f);
-    const auto may_lower = [&](float4 q) -> bool {
-      return !lbound ||
-             !(box_bound(q.x, q.y, q.z, blo.x, blo.y, blo.z, bhi.x, bhi.y, bhi.z) >= lmax);
-    };
-    hm[k] = __ballot((uint32_t)in0 & (uint32_t)touches_pick(k, pc0) & (uint32_t)may_lower(pp0));
+    hm[k] = __ballot(in0 && touches(k, lane) && may_lower(k, pp0));
     bool h = hm[k] != 0;
     for (uint32_t cb = 64; cb < nsel && !h; cb += 64)
-      h = __ballot((cb + lane < nsel) && touches(k, cb + lane) && may_lower(s_pp[cb + lane])) != 0;
+      h = __ballot((cb + lane < nsel) && touches(k, cb + lane) && may_lower(k, s_pp[cb + lane])) != 0;
     hit[k] = h;
-    need[k] = leaf0 + k < c.nleaves && (h || okey[k] >= wlo);
+    need[k] = leaf0 + k < c.nleaves && (h || (last && okey[k] >= wlo));
   }
   if (PROF) {
     utc = __builtin_amdgcn_s_memrealtime();
@@ -485,17 +559,17 @@ __global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60)
             pc11 = pack11(pack_cell(cell_axis(c.r, 0, p[k].x), cell_axis(c.r, 1, p[k].y),
                                     cell_axis(c.r, 2, p[k].z)));
           for (uint32_t cb = 0; cb < nsel; cb += 64) {
-            uint64_t m = cb == 0 ? hm[k] : __ballot((cb + lane < nsel) & touches(k, cb + lane));
+            uint64_t m = cb == 0 ? hm[k]
+                                 : __ballot((cb + lane < nsel) && touches(k, cb + lane) &&
+                                            may_lower(k, s_pp[cb + lane]));
             while (m) {
               const uint32_t j = (uint32_t)__ffsll((long long)m) - 1;
               m &= m - 1;
               const float4 q = s_pp[cb + j];
               const float dd = sqdist(p[k].x, p[k].y, p[k].z, q.x, q.y, q.z);
-              if (MIXED) {
+              if (__ballot(dd < d)) {
                 const uint2 qc = s_pc[cb + j];
-                d = in_box11(pc11 | kGuards, pc11, qc.x, qc.y) && dd < d ? dd : d;
-              } else {
-                d = dd < d ? dd : d;
+                d = dd < d && in_cube(k, pc11, qc) ? dd : d;
               }
             }
           }
@@ -509,14 +583,27 @@ __global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60)
             if (lane == 0) gptr(c.leaf_key)[leaf0 + k] = key;
           }
         }
-        if (act) {
+        if (act && last) {
           const uint32_t hi = __float_as_uint(d);
-          const uint32_t b = key_bin(((uint64_t)hi << 32) | lo, kref, S);
+          const uint32_t b = key_bin(((uint64_t)hi << 32) | lo, kref, S, nb);
           if (b != kNone) atomicAdd(&s_hist[b], 1u);
         }
       }
     }
+    okey[k] = key;
     if (lane == 0) s_lk[li] = key;
+  }
+  if (last) break;
+  ch += kPickLds;
+  nsel = min(nall - ch, kPickLds);
+  __syncthreads();  // every wave is through with the picks before
+  if (tid < nsel) {
+    const uint32_t i = s_more[ch - kPickLds + tid];
+    const float4 pp = gptr(c.list_p)[i];
+    s_pp[tid] = make_float4(pp.x, pp.y, pp.z, 0.f);
+    s_pc[tid] = gptr(c.list_c)[i];
+  }
+  __syncthreads();
   }
   if (PROF && lane == 0) s_wt[kPassWaves + wave] = (uint32_t)(__builtin_amdgcn_s_memrealtime() - ut1);
   __syncthreads();
@@ -581,7 +668,7 @@ __global__ __launch_bounds__(kPassThreads, 2) __attribute__((amdgpu_num_sgpr(60)
 __global__ __launch_bounds__(kPassThreads) void k_refine(const CloudDev *__restrict__ clouds,
                                                          uint32_t pass, uint32_t passes) {
   __shared__ uint32_t s_hist[kHistBins];
-  __shared__ uint32_t s_sc[kPassWaves + 2];
+  __shared__ uint32_t s_sc[kPassWaves + 3];
   const CloudDev &c = clouds[blockIdx.y];
   if (blockIdx.x >= c.nl1 || *gptr(c.done)) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -622,14 +709,13 @@ __device__ __forceinline__ uint32_t bit_length(uint64_t v) { return v ? 64u - __
 // (more than kListCap keys inside the finest bin), the threshold is the
 // maximum key itself: a run of one sample.  Few workgroups, each striding over
 // the level-1 nodes; most nodes hold no key above the threshold.  PROF: counts
-// the hot leaves whose points it reads and those points.  An entry's cell is
-// its point's own (where its cube is centred when it becomes a sample).
-// ALIAS (cells share buckets): the entry also carries the cells of its
-// bucket.
-template <bool PROF, bool ALIAS>
+// the hot leaves whose points it reads and those points.  Its first workgroup
+// also ends the sampling: when m samples have keys above every key left, or
+// only points at distance 0 are left (src/yuezu_fps.cpp:705-706).
+template <bool PROF>
 __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restrict__ clouds,
-                                                         uint32_t passes) {
-  __shared__ uint32_t s_sc[kPassWaves + 2];
+                                                         uint32_t passes, uint32_t par) {
+  __shared__ uint32_t s_sc[kPassWaves + 3];
   __shared__ uint64_t s_wk[kPassWaves];
   const CloudDev &c = clouds[blockIdx.y];
   const uint64_t gt0 = PROF ? __builtin_amdgcn_s_memrealtime() : 0;
@@ -662,7 +748,7 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
   uint64_t gt1 = 0, gt2 = 0, gt3 = 0;
   bool forced = false;
   const Sel s = sel_replay(c, passes + 1, passes, s_sc, &forced, &h0);
-  uint64_t bkey = s.bkey;
+  uint64_t bkey = s.bkey, ktop = s.ktop;
   if (s.state == 2) {
     uint64_t best = 0;
     for (uint32_t j = tid; j < c.nl1; j += kPassThreads) {
@@ -674,18 +760,56 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
     __syncthreads();
     best = 0;
     for (uint32_t w = 0; w < kPassWaves; ++w) best = s_wk[w] > best ? s_wk[w] : best;
-    bkey = best;
+    bkey = ktop = best;
   }
   if (PROF) gt1 = __builtin_amdgcn_s_memrealtime();
-  if (blockIdx.x == 0 && tid == 0) {
-    rs.bkey = bkey;
-    // the first rounds start from windows over the whole key range and are
-    // forced as a rule; later forced rounds ask for refinement passes
-    rs.forced += forced && rs.rounds >= 2 ? 1u : 0u;
-    // next round: fine bins of about 1/2048 of this round's key span
-    uint32_t nx = bit_length(rs.kref0 - bkey + 1);
-    nx = nx > 11u ? nx - 11u : 0u;
-    rs.s0_next = nx < kMaxShift ? nx : kMaxShift;
+  if (blockIdx.x == 0) {  // uniform
+    const uint32_t T = rs.ntaken, m = c.m;
+    bool fin = (uint32_t)(ktop >> 32) == 0u;  // only points at distance 0 are left
+    if (!fin && T >= m) {
+      // the samples above every key left: all of the rounds whose thresholds
+      // were, and those of the later rounds that are
+      __shared__ uint32_t s_first, s_above;
+      if (tid == 0) {
+        s_first = T;
+        s_above = 0;
+      }
+      __syncthreads();
+      for (uint32_t j = tid; j < rs.nlog; j += kPassThreads)
+        if (gptr(c.log_bmin)[j] <= ktop) atomicMin(&s_first, gptr(c.log_start)[j]);
+      __syncthreads();
+      const uint32_t w0 = s_first;
+      uint32_t n = 0;
+      for (uint32_t j = w0 + tid; j < T; j += kPassThreads)
+        n += (((uint64_t)gptr(c.smp_d)[j] << 32) | gptr(c.smp_lo)[j]) > ktop ? 1u : 0u;
+      n = rdlane(wave_incl_scan(n), 63);
+      if (lane == 0) atomicAdd(&s_above, n);
+      __syncthreads();
+      fin = w0 + s_above >= m;
+    }
+    if (tid == 0) {
+      rs.bkey = bkey;
+      rs.ktop = ktop;
+      // the first rounds start from windows over the whole key range and are
+      // forced as a rule; later forced rounds ask for refinement passes
+      rs.forced += forced && rs.rounds >= 2 ? 1u : 0u;
+      // next round: bins of 1/1024 to 1/2048 of this round's key span, over
+      // 1.75 spans (the next threshold lies about half a span below this one;
+      // every leaf with a key in the window is read); where the list came out
+      // short, over two to four times the whole window down to the threshold
+      const bool grow = 2 * s.total < rs.cap;
+      const uint64_t span = (grow ? rs.kref0 : ktop) - bkey + 1;
+      uint32_t nx = bit_length(span);
+      nx = nx > 11u ? nx - 11u : 0u;
+      nx = nx < kMaxShift ? nx : kMaxShift;
+      rs.s0_next = nx;
+      rs.nb_next = grow ? kHistBins : min((uint32_t)(span >> nx) * 7 / 4 + 1, kHistBins);
+      if (fin) {
+        *gptr(c.iter) = min(T, m);
+        *gptr(c.done) = 1;
+      }
+    }
+    if (fin) return;
   }
   // Nodes in chunks of kGatherNodes; lane l of a wave holds leaf l % 4 of the
   // wave's four leaves of node l / 4 of the chunk, so one read brings in all
@@ -696,8 +820,6 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
   __shared__ uint32_t s_cnt, s_base;
   for (uint32_t c0 = blockIdx.x; c0 < c.nl1; c0 += kGatherNodes * gridDim.x) {
     if (c0 != blockIdx.x) read_leaf(c0);
-    uint32_t gq;
-    const uint32_t lf = leaf_of(c0, gq);
     const bool hot = lcnt != 0 && lkey >= bkey;  // an empty or absent leaf has key 0
     if (PROF) {
       pin_vgpr(lst, lcnt, (uint32_t)hot);
@@ -716,9 +838,8 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
     }
     float4 hp[kGatherHold];
     uint2 hr[kGatherHold];
-    uint32_t hn[kGatherHold], hal[kGatherHold];
+    uint32_t hn[kGatherHold];
     uint64_t htk[kGatherHold];
-    const uint32_t na = ALIAS ? c.r.na : 1u;
     // the held leaves' points: every lane loads, without a branch, so that
     // the loads are in flight together; a lane past the leaf's points, or of
     // a wave with fewer hot leaves, reads slot 0 and its values go unused
@@ -733,8 +854,6 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
       const uint32_t idx = lane < cnt ? st + lane : 0u;
       hp[u] = gptr(c.P4)[idx];
       hr[u] = gptr(c.RO)[idx];
-      hal[u] = kNoCell;  // lane a < na: cell a of the held leaf's bucket
-      if (ALIAS && have && lane < na) hal[u] = gptr(c.leaf_al)[(size_t)rdlane(lf, j) * na + lane];
     }
     uint32_t mine = 0;
 #pragma unroll
@@ -759,7 +878,7 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
     uint32_t base = 0;
     if (lane == 0 && mine) base = atomicAdd(&s_cnt, mine);
     __syncthreads();
-    if (tid == 0) s_base = s_cnt ? atomicAdd(&rs.nlist, s_cnt) : 0u;
+    if (tid == 0) s_base = s_cnt ? atomicAdd(&rs.nl[par], s_cnt) : 0u;
     __syncthreads();
     base = s_base + rdlane(base, 0);
     if (PROF && !gt3) gt3 = __builtin_amdgcn_s_memrealtime();
@@ -767,20 +886,16 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
     // the arguments after a store would first wait for the store
     NSFPS_GLOBAL float4 *const LP = vgpr_ptr(gptr(c.list_p));
     NSFPS_GLOBAL uint2 *const LR = vgpr_ptr(gptr(c.list_r));
-    NSFPS_GLOBAL uint32_t *const LC = vgpr_ptr(gptr(c.list_c));
+    NSFPS_GLOBAL uint32_t *const LF = vgpr_ptr(gptr(c.list_f));
     // arguments by value: a reference into hp / hr would make those arrays
     // memory (the compiler then keeps them in LDS)
-    const auto put = [&](float4 p, uint2 ro, uint32_t al, uint64_t m) {
+    const auto put = [&](float4 p, uint2 ro, uint64_t m) {
       if ((m >> lane) & 1u) {
         const uint32_t i = base + lanes_below(m);
         if (i < kListCap) {
           LP[i] = p;
           LR[i] = ro;
-          // the point's own cell (its bucket's, when buckets have one cell;
-          // a leaf may hold several buckets)
-          LC[i] = pack_cell(cell_axis(c.r, 0, p.x), cell_axis(c.r, 1, p.y), cell_axis(c.r, 2, p.z));
-          if (ALIAS)
-            for (uint32_t a = 0; a < na; ++a) gptr(c.list_al)[(size_t)i * na + a] = rdlane(al, a);
+          LF[i] = 0u;  // not in conflict, until the accept pass finds it is
         } else {
           rs.err = 1;
         }
@@ -788,7 +903,7 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
       base += (uint32_t)__popcll(m);
     };
 #pragma unroll
-    for (uint32_t u = 0; u < kGatherHold; ++u) put(hp[u], hr[u], hal[u], htk[u]);
+    for (uint32_t u = 0; u < kGatherHold; ++u) put(hp[u], hr[u], htk[u]);
     rest = later;
     while (rest) {
       const uint32_t j = (uint32_t)__builtin_ctzll(rest);
@@ -796,14 +911,12 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
       const uint32_t st = rdlane(lst, j), cnt = rdlane(lcnt, j);
       float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
       uint2 ro = make_uint2(0u, 0u);
-      uint32_t al = kNoCell;
       if (lane < cnt) {
         p = gptr(c.P4)[st + lane];
         ro = gptr(c.RO)[st + lane];
       }
-      if (ALIAS && lane < na) al = gptr(c.leaf_al)[(size_t)rdlane(lf, j) * na + lane];
       const bool take = lane < cnt && (((uint64_t)__float_as_uint(p.w) << 32) | ~ro.x) >= bkey;
-      put(p, ro, al, __ballot(take));
+      put(p, ro, __ballot(take));
     }
     __syncthreads();  // s_base is read before the next chunk's claim
   }
@@ -824,1156 +937,266 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
   }
 }
 
-// ---------------------------------------------------------------- the run
+// ------------------------------------------------------------- accept pass
 
-// One workgroup per cloud, eight waves (two per SIMD: the kernel is bound by
-// instruction latency, which the second wave hides); every thread holds
-// kOwnSlots list entries.  The list sits in LDS sorted by coarse cell (x >> sx, y >> sy,
-// z >> sz; at most kCells of them) with the first entry of every coarse cell,
-// so the entries inside a cube are found by walking, for each coarse (y, z)
-// row the cube spans, the entries of its x range.
+// Settles the list.  Two entries conflict when their sqdist is below the
+// larger of their distances: only then can either lower the other.  An entry
+// that conflicts with no entry of a larger key is a sample with the key it
+// has:
+//   - every point of a larger key is in the list, and those not settled yet
+//     are too far to lower it;
+//   - every sample that precedes it and was near enough has been applied by
+//     the update passes since.
+// It may be applied to all points at once: a point of a larger key that it
+// could lower would have been in conflict with it.  The largest key never has
+// a conflict above it, so every round settles at least one entry; entries
+// that stay come again in the next round's list.  The samples' order is the
+// order of their keys (k_order).
 //
-// The threshold argument is applied once more inside the list: a hot
-// threshold H leaves at most HOT entries at or above it (64, or 128 where the
-// points fill many buckets), and those are resolved in parallel phases.  Rank the remaining hot copies by key; copy j
-// is "lowered" when the cube of a higher-ranked copy contains it and brings
-// its distance down.  Every copy ranked above the first lowered one is a
-// sample, in rank order: all copies ranked above it are samples too, a copy
-// lowered by one of them started below it, and the rest of the list is below
-// H.  The copies that are not lowered go on being samples past a lowered copy
-// j as long as they exceed K_j, j's key once every copy above it that is not
-// lowered has been applied (j's key can only be lower when their turn
-// comes).  So a phase takes those samples at once, applies their cubes to
-// the remaining copies, and ranks again, until no copy is >= max(H, B).  Then the
-// hot run's samples are applied to every list entry (a
-// sample with a small cube is applied by its copy's lanes walking its rows of
-// the cell index, one with a large cube by every thread to its own entries)
-// and the next hot set is chosen.  The run ends when no entry is >= B.
-constexpr uint32_t kRunThreads = 512;
-constexpr uint32_t kRunWaves = kRunThreads / 64;
-constexpr uint32_t kOwnSlots = kListCap / kRunThreads;
-// A hot set holds at most HOT copies (64, or 128 when no cells share
-// buckets).  Each copy has kLanes threads, each comparing it with kCmp other
-// copies; masks over the copies (or their ranks) take kWords 64-bit words.
-template <uint32_t HOT>
-struct HotSet {
-  static constexpr uint32_t kLanes = kRunThreads / HOT;  // threads per hot copy (and per sample)
-  static constexpr uint32_t kCmp = HOT / kLanes;         // copies each of them compares against
-  static constexpr uint32_t kWords = HOT / 64;
-  static constexpr uint32_t kCmpMask = kCmp >= 32 ? 0xffffffffu : (1u << kCmp) - 1u;
-  static_assert((kLanes == 4 || kLanes == 8 || kLanes == 16) && (HOT == 64 || HOT == 128) &&
-                    kCmp <= 32 && kCmp % 8 == 0,
-                "the run kernel layout");
-};
-constexpr uint32_t kHotMax = 128;
-constexpr uint32_t kSelBins = 256;
-constexpr uint32_t kCells = 4096;    // coarse cells of the list's cell index
-// Copies >= the hot threshold left after a phase that justify another phase.
-// A phase accepts at least the first-ranked copy, so a value of at least the
-// hot set's size means one phase per hot set, the copies left over going back
-// to the next selection: ranking
-// them again in further phases measured slower (uniform cube 8.36 ms per call
-// at 12, 8.26 at 32, 8.20 at 48, 8.09 at kHot; LiDAR scan 5.38 / 5.26 / 5.19 /
-// 5.14 ms).  Measured again on the later kernels, further phases at 32 gain
-// only where phases accept few samples (quickstart, about 20 of 64: 0.711
-// against 0.732 ms) and lose elsewhere (uniform cube 8.02 against 7.70 ms,
-// clustered cloud 73.5 against 69.8); allowing them only after a phase of at
-// most 24 samples still cost the uniform cube 3 % and the clustered cloud 4 %.
-constexpr uint32_t kPhaseMin = kHotMax;
-// Cubes over more coarse rows, or with more list entries in one lane's rows,
-// are applied by every thread to its own entries instead of walked.  Rows
-// below 64 keep the walk's row arithmetic exact.  With a lane's rows walked
-// as one list, 16 rows (two a lane) measured best: per call, uniform cube
-// 7.73 ms at 16 rows and 7.88 at 24, LiDAR scan 4.49 and 4.50, clustered
-// 71.0 and 73.4 (row by row at 24 rows: 7.94, 4.75, 69.3).
-constexpr uint32_t kWalkRows = 16;
-constexpr uint32_t kWalkLaneEntries = 16;
-constexpr uint32_t kDenseWalkRows = 12;  // 128-copy sets on dense clouds
-static_assert(kWalkRows <= 64, "the walk's row arithmetic");
-// With hot sets of 128 copies a sample has 4 lanes: ROWS rows (16, or 12 for
-// dense clouds) and 24 entries a lane.  Measured per call (rows / entries):
-// uniform cube 7.21 ms at 16 / 16, 16 / 24 and 16 / 32, 7.26 at 12 / 24,
-// 7.38 at 24 / 16, 8.47 at 8 / 16; clustered cloud 62.1, 61.6, 61.6, 60.5,
-// 63.8 and 60.5 ms.  The rows' gain is the lane's row slots (3 against 4 in
-// the walk's entry-to-row mapping): a limit of 12 rows read at run time, the
-// slots still sized for 16, left the clustered cloud at 61.9 ms.
-template <uint32_t HOT, uint32_t ROWS>
-struct WalkLimits {
-  static constexpr uint32_t kRows = ROWS;
-  static constexpr uint32_t kLaneEntries = HOT == 128 ? 24 : kWalkLaneEntries;
-  static_assert(kRows <= 64, "the walk's row arithmetic");
-};
-constexpr uint32_t kCellsPerThread = kCells / kRunThreads;
-static_assert(kCellsPerThread % 4 == 0, "the cell scan reads whole uint4s");
+// All pairs of the list: a wave's lanes hold two entries each and meet a
+// chunk of others, read through the scalar cache (uniform addresses), at 10
+// vector instructions a pair.  At 4,096 entries (16.7 M pairs) that is 4.3 us
+// of the chip's issue; 1,024 entries are bound by the kernel's latency.  A
+// few workgroups beside these find the entries' cubes for the update pass.
+constexpr uint32_t kAcceptThreads = 256;
+constexpr uint32_t kAcceptWaves = kAcceptThreads / 64;
+constexpr uint32_t kAcceptX = 128;  // entries held by a wave
+constexpr uint32_t kAcceptChunk = 16;  // others they meet
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+#if defined(__HIP_DEVICE_COMPILE__)
+#define NSFPS_CONSTANT __attribute__((address_space(4)))
+#else
+#define NSFPS_CONSTANT
+#endif
 
-// Phase clocks of the run kernel (s_memtime cycles of wave 0, summed over
-// rounds into the cloud's profile words) when PROF is set.
-enum : uint32_t {
-  kRpLoad = 0, kRpSelect, kRpGather, kRpPhases, kRpApply, kRpTail, kRpBig, kRpRank,
-  kRpPicks = 8, kRpRounds, kRpHotRounds, kRpPhaseCount, kRpWalk, kRpPublish,
-  kRpRtLoad = 14,  // s_memrealtime ticks (100 MHz) from the kernel's start to the end of the load
-  kRpRtTotal = 15, //   and to the kernel's end
-  kRpWords = 16,
-  // words kept past the first kRpWords (local words 16.., profile words
-  // 28.., after the work counters of the passes): the wait at the barrier
-  // after the walk, the pass over entries whose bucket has several cells,
-  // and those entries summed over hot sets
-  kRpWalkWait = 16, kRpAlias = 17, kRpAliasN = 18, kRpLocal = 19, kRpExtraAt = 28
-};
-
-// LDS slot of hot copy i.  Lane q of a copy's group compares against copies
-// q * kCmp + u; the kLanes copies read together for one u sit side by side,
-// so one read by a wave touches distinct banks.
-template <uint32_t HOT>
-__device__ __forceinline__ uint32_t hot_slot(uint32_t i) {
-  return (i % HotSet<HOT>::kCmp) * HotSet<HOT>::kLanes + i / HotSet<HOT>::kCmp;
-}
-
-// Sum / minimum over the L lanes of a group (aligned lanes).
-template <uint32_t L>
-__device__ __forceinline__ uint32_t group_sum(uint32_t v) {
-  v += dpp_mov<kDppQuad1032>(v);
-  v += dpp_mov<kDppQuad2301>(v);
-  if (L >= 8) v += dpp_mov<kDppHalfMirror>(v);  // lane i and 7 - i: the other quad
-  if (L >= 16) v += dpp_mov<kDppMirror>(v);     // lane i and 15 - i: the other half
-  return v;
-}
-template <uint32_t L>
-__device__ __forceinline__ uint32_t group_min(uint32_t v) {
-  v = min(v, dpp_mov<kDppQuad1032>(v));
-  v = min(v, dpp_mov<kDppQuad2301>(v));
-  if (L >= 8) v = min(v, dpp_mov<kDppHalfMirror>(v));
-  if (L >= 16) v = min(v, dpp_mov<kDppMirror>(v));
-  return v;
-}
-
-// Bin shift of a hot-threshold histogram whose kSelBins bins end at kref and
-// cover every key down to bkey.
-__device__ __forceinline__ uint32_t sel_shift(uint64_t kref, uint64_t bkey) {
-  const uint32_t n = bit_length(kref - bkey);
-  return n > 8u ? n - 8u : 0u;
-}
-
-// Counts this thread's live keys (>= bkey) into histogram H (window kref, S);
-// every live key is <= kref.
-__device__ __forceinline__ void hist_live(const float *d, const uint32_t *lo, uint64_t bkey,
-                                          uint64_t kref, uint32_t S, uint32_t *H,
-                                          NSFPS_GLOBAL uint32_t *err) {
-#pragma unroll
-  for (uint32_t s = 0; s < kOwnSlots; ++s) {
-    const uint64_t key = ((uint64_t)__float_as_uint(d[s]) << 32) | lo[s];
-    if (lo[s] != 0u && key >= bkey) {
-      if (key <= kref) atomicAdd(&H[(uint32_t)((kref - key) >> S)], 1u);
-      else *err = 3;  // cannot happen (kref bounds every live key)
-    }
-  }
-}
-
-// The run of one cloud by one workgroup of kRunThreads.  ALIAS: cells share
-// buckets.  A sample then updates
-// every entry whose bucket has a cell inside its cube (src/yuezu_fps.cpp:
-// 573-597).  The walk finds entries by their own cell; the entries whose
-// bucket has further cells are few and listed apart, and after each walk
-// every one of them is tested against every sample of the hot set; the
-// phases test every cell of a hot copy's bucket.  HOT: copies per hot set;
-// ROWS: the walk's row limit.  WHOLE (clouds in few buckets): the list's
-// cell box is taken at its load, and a large-cube sample whose cube holds it
-// is applied to every entry with no cell test.
-template <bool PROF, bool ALIAS, uint32_t HOT, uint32_t ROWS, bool WHOLE>
-__device__ __forceinline__ void run_list(const CloudDev &c) {
-  static_assert(!(WHOLE && ALIAS), "the list box is of the entries' own cells");
-  // the alias pass holds one sample per lane
-  static_assert(!ALIAS || HOT == 64, "shared buckets take hot sets of 64");
-  constexpr uint32_t kHot = HOT, kCopyLanes = HotSet<HOT>::kLanes, kCmp = HotSet<HOT>::kCmp,
-                     kWords = HotSet<HOT>::kWords;
-  __shared__ uint4 s_pc[kListCap];      // sorted list: {x, y, z, pack11(cell)}
-  __shared__ uint32_t s_dd[kListCap];   // its distances (bits)
-  __shared__ uint2 s_rk[kListCap];      // its {~logical rank, input row}
-  __shared__ uint4 s_hq[2][kHot];       // hot copies at hot_slot<HOT>(i), one buffer per phase parity:
-                                        //   {pack11(cube lo), pack11(cube hi) | guards, ~rank,
-                                        //   distance bits}; key 0 once taken
-  __shared__ __align__(16) uint32_t s_rank[kHot];  // rank of each hot copy in the phase
-  __shared__ unsigned long long s_lowm[2][kWords];  // bit r: the copy ranked r is lowered
-  __shared__ unsigned long long s_lowc[2][kWords];  // bit j: hot copy j is lowered
-  __shared__ unsigned long long s_kmax[2];  // the largest bound K_j of a lowered copy
-  __shared__ uint4 s_hx[kHot];          // hot copies: {cell, pack11(cell) | guards, pack11(cell),
-                                        //   half-widths}
-  __shared__ uint4 s_hp[kHot];          // hot copies: {x, y, z, row}
-  __shared__ uint4 s_rp[kHot];          // accepted hot copies at their slot: {x, y, z, row}
-  __shared__ uint2 s_rc[kHot];          //   cube corners, pack11 (hi with guards)
-  __shared__ __align__(16) uint32_t s_cell[kCells + 4];  // first entry of each coarse cell
-  __shared__ uint32_t s_big[2 * kWords];                // samples with large cubes
-  __shared__ uint32_t s_bigw[WHOLE ? 2 * kWords : 1];  // WHOLE: those whose cube holds the list box
-  __shared__ __align__(16) uint32_t s_sel[3][kSelBins];  // hot-threshold histograms, rotating
-  __shared__ uint32_t s_nhot;
-  __shared__ unsigned long long s_kmr;   // largest key of a hot copy left unaccepted
-  __shared__ uint32_t s_wn[2 * kRunWaves];  // wave sums of the two cell-count scans
-  __shared__ uint32_t s_wr[2][kRunWaves][2];
-  __shared__ uint32_t s_geo[4];  // coarse cell shifts (x | y << 8 | z << 16), ncx, ncy
-  // ALIAS: the cells of each entry's bucket (pack11, kNoCell-padded, at the
-  // entry's sorted position), the sorted positions of the entries whose
-  // bucket has several cells, the hot copies' positions, and the hot set's
-  // samples by output order: cube corners (pack11; hi with guards) and x, y, z
-  __shared__ uint32_t s_al[ALIAS ? kListCap * kMaxAlias : 1];
-  // ALIAS: a second coarse cell index, of records {x, y, z, pack11(cell)} of
-  // the entries' other cells (the cells of their bucket besides their own)
-  // and the entry each belongs to, so that the walk reaches an entry through
-  // any cell of its bucket; entries whose records do not fit go to a pass
-  // over every sample of the hot set (s_alist)
-  __shared__ __align__(16) uint32_t s_xc[ALIAS ? kCells + 4 : 4];
-  __shared__ uint4 s_xp[ALIAS ? kListCap : 1];
-  __shared__ uint32_t s_xe[ALIAS ? kListCap : 1];
-  __shared__ uint32_t s_nx;
-  __shared__ uint32_t s_alist[ALIAS ? kListCap : 1];
-  __shared__ uint32_t s_nal;
-  __shared__ uint32_t s_hpos[kHot];
-  // WHOLE: the list's cell box, per axis the largest cell and 1023 - the smallest
-  __shared__ uint32_t s_lb[WHOLE ? 6 : 1];
-  __shared__ uint2 s_sbox[ALIAS ? kHot : 1];
-  __shared__ float4 s_spos[ALIAS ? kHot : 1];
-  const uint64_t rt0 = PROF ? __builtin_amdgcn_s_memrealtime() : 0;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+__global__ __launch_bounds__(kAcceptThreads) void k_accept(const CloudDev *__restrict__ clouds,
+                                                           uint32_t par, uint32_t ncube) {
+  const CloudDev &c = clouds[blockIdx.y];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
   NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
-  // every input of the run is read at once: the done flag, the run state and
-  // the whole list buffer (entries at or beyond the list length are stale
-  // and ignored)
-  const uint32_t done_in = *gptr(c.done);
-  const uint32_t nlist = min(rs.nlist, kListCap);
-  const uint64_t bkey = rs.bkey, kref0 = rs.kref0;
-  float4 P[kOwnSlots];
-  uint2 R[kOwnSlots];
-  uint32_t C[kOwnSlots];
-  const uint32_t na = ALIAS ? c.r.na : 1u;
-  uint32_t AL[ALIAS ? kOwnSlots : 1][kMaxAlias];
+  // list_cap / kAcceptX groups of entries, each against every chunk
+  const uint32_t xgs = c.list_cap / kAcceptX;
+  const bool cubes = blockIdx.x < ncube;
+  const uint32_t w = uniform(cubes ? 0u : (blockIdx.x - ncube) * kAcceptWaves + (tid >> 6));
+  const uint32_t x0 = (w % xgs) * kAcceptX + lane, q0 = (w / xgs) * kAcceptChunk;
+  const uint32_t nl = min(rs.nl[par], kListCap), done = *gptr(c.done);
+  // entries past the list are stale and unused
+  float4 X[2];
+  uint32_t XR[2];
 #pragma unroll
-  for (uint32_t s = 0; s < kOwnSlots; ++s) {
-    const uint32_t i = s * kRunThreads + tid;
-    P[s] = gptr(c.list_p)[i];
-    R[s] = gptr(c.list_r)[i];
-    C[s] = gptr(c.list_c)[i];
-    if (ALIAS) {
+  for (uint32_t t = 0; t < 2; ++t) {
+    X[t] = gptr(c.list_p)[x0 + 64 * t];
+    XR[t] = gptr(c.list_r)[x0 + 64 * t].x;
+  }
+  if (done) return;
+  // the histograms this round's selection read are cleared for the next
+  // round's update pass
+  NSFPS_GLOBAL uint4 *const hz = reinterpret_cast<NSFPS_GLOBAL uint4 *>(hist_set(c));
+  for (uint32_t j = blockIdx.x * kAcceptThreads + tid; j < kHists * kHistBins / 4;
+       j += gridDim.x * kAcceptThreads)
+    hz[j] = make_uint4(0u, 0u, 0u, 0u);
+  if (blockIdx.x == 0 && tid == 0) {
+    rs.nl[par ^ 1u] = 0;  // the next round's list
+    rs.kref0 = rs.ktop;   // keys only decrease
+    rs.s0 = rs.s0_next;
+    rs.nb = rs.nb_next;
+    rs.rounds += 1;
+  }
+  if (cubes) {
+    const uint32_t i = blockIdx.x * kAcceptThreads + tid;
+    if (i < nl) {
+      const float4 p = gptr(c.list_p)[i];
+      gptr(c.list_c)[i] = sample_cube(
+          c.r, pack11(pack_cell(cell_axis(c.r, 0, p.x), cell_axis(c.r, 1, p.y), cell_axis(c.r, 2, p.z))),
+          p.w);
+      // a point at distance 0 is never a sample
+      if (p.w == 0.0f) gptr(c.list_f)[i] = 1u;
+    }
+    return;
+  }
+  if (x0 - lane >= nl || q0 >= nl) return;
+  uint64_t kx[2];
 #pragma unroll
-      for (uint32_t a = 0; a < kMaxAlias; ++a)
-        AL[s][a] = a < na && i < nlist ? gptr(c.list_al)[(size_t)i * na + a] : kNoCell;
-    }
+  for (uint32_t t = 0; t < 2; ++t)
+    kx[t] = x0 + 64 * t < nl ? make_key(X[t].w, XR[t]) : ~0ull;  // absent: nothing lies above it
+  const NSFPS_CONSTANT v4f *const LP = (const NSFPS_CONSTANT v4f *)c.list_p + q0;
+  const NSFPS_CONSTANT v2u *const LR = (const NSFPS_CONSTANT v2u *)c.list_r + q0;
+  const uint32_t nq = min(nl - q0, kAcceptChunk);
+  bool blocked[2] = {false, false};
+#pragma unroll 8
+  for (uint32_t j = 0; j < nq; ++j) {
+    const v4f q = LP[j];
+    const uint64_t kq = make_key(q.w, LR[j].x);
+#pragma unroll
+    for (uint32_t t = 0; t < 2; ++t)
+      blocked[t] |= (kq > kx[t]) & (sqdist(X[t].x, X[t].y, X[t].z, q.x, q.y, q.z) < q.w);
   }
-  uint64_t pf[kRpLocal] = {}, tl = 0;
-  if (PROF) tl = __builtin_amdgcn_s_memtime();
-#define NSFPS_RMARK(ph)                                  \
-  do {                                                   \
-    if (PROF) {                                          \
-      const uint64_t t_ = __builtin_amdgcn_s_memtime();  \
-      pf[ph] += t_ - tl;                                 \
-      tl = t_;                                           \
-    }                                                    \
-  } while (0)
-  const uint32_t b0 = c.r.blocks[0], b1 = c.r.blocks[1], b2 = c.r.blocks[2];
-  // coarse cells (x >> sx, y >> sy, z >> sz), at most kCells of them: the
-  // longest coarse axis is halved until they fit
-  uint32_t sx = 0, sy = 0, sz = 0;
-  while (true) {
-    const uint32_t ex = ((b0 - 1) >> sx) + 1, ey = ((b1 - 1) >> sy) + 1, ez = ((b2 - 1) >> sz) + 1;
-    if (ex * ey * ez <= kCells) break;
-    if (ex >= ey && ex >= ez) ++sx;
-    else if (ey >= ez) ++sy;
-    else ++sz;
-  }
-  const uint32_t ncx = ((b0 - 1) >> sx) + 1, ncy = ((b1 - 1) >> sy) + 1;
-  for (uint32_t j = tid; j < kCells + 4; j += kRunThreads) {
-    s_cell[j] = 0;
-    if (ALIAS) s_xc[j] = 0;
-  }
-  if (tid < kSelBins) {
-    s_sel[0][tid] = 0;
-    s_sel[1][tid] = 0;
-  }
-  if (tid < kHot) s_hq[0][tid] = make_uint4(0u, 0u, 0u, 0u);  // key 0: an unused slot
-  if (WHOLE && tid < 6) s_lb[tid] = 0;
-  if (tid == 0) {
-    s_nhot = 0;
-    if (ALIAS) {
-      s_nal = 0;
-      s_nx = 0;
-    }
-    s_geo[0] = sx | (sy << 8) | (sz << 16);
-    s_geo[1] = ncx;
-    s_geo[2] = ncy;
-  }
-  __syncthreads();
-  if (done_in) return;  // uniform: the whole workgroup leaves
+#pragma unroll
+  for (uint32_t t = 0; t < 2; ++t)
+    if (blocked[t]) gptr(c.list_f)[x0 + 64 * t] = 1u;
+}
 
-  // ---- list -> LDS in coarse-cell order (counting sort)
-  {
-    const auto coarse = [&](uint32_t c10) {
-      return (((c10 >> 20) >> sz) * ncy + (((c10 >> 10) & 1023u) >> sy)) * ncx +
-             ((c10 & 1023u) >> sx);
-    };
-    uint32_t G[kOwnSlots], K[kOwnSlots];
-    // ALIAS: per entry, its other cells' number and whether their records
-    // fit the second index, and each record's place among its coarse cell's
-    uint32_t NO[ALIAS ? kOwnSlots : 1] = {};
-    bool XI[ALIAS ? kOwnSlots : 1] = {};
-    uint32_t XK[ALIAS ? kOwnSlots : 1][kMaxAlias];
+// Sorts each round's samples by key, descending (one workgroup a round; a
+// round settles at most kListCap; the log's last entry may stand for more,
+// and is left as it is): bins of equal width over the round's span, then each
+// sample's place among its bin's.
+constexpr uint32_t kSortThreads = 512;
+__global__ __launch_bounds__(kSortThreads) void k_sort_rounds(const CloudDev *__restrict__ clouds) {
+  const CloudDev &c = clouds[blockIdx.y];
+  constexpr uint32_t kSlots = kListCap / kSortThreads, kWaves = kSortThreads / 64;
+  __shared__ uint2 s_key[kListCap];
+  __shared__ __align__(16) uint32_t s_bin[kListCap + 4];
+  __shared__ uint16_t s_at[kListCap];
+  __shared__ uint32_t s_wn[kWaves];
+  __shared__ uint64_t s_mx[2];
+  if (!*gptr(c.done)) return;
+  const NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
+  const uint32_t nlog = rs.nlog, T = min(rs.ntaken, c.n), tid = threadIdx.x;
+  for (uint32_t r = blockIdx.x; r < nlog; r += gridDim.x) {
+    const uint32_t b = gptr(c.log_start)[r], e = r + 1 < nlog ? gptr(c.log_start)[r + 1] : T;
+    const uint32_t n = e - b;
+    if (n < 2 || n > kListCap) continue;
+    uint2 k[kSlots];
+    uint32_t row[kSlots], bin[kSlots], at[kSlots];
+    for (uint32_t j = tid; j < kListCap + 4; j += kSortThreads) s_bin[j] = 0;
+    if (tid < 2) s_mx[tid] = 0;
+    __syncthreads();
+    uint64_t mx = 0, mn = 0;
 #pragma unroll
-    for (uint32_t s = 0; s < kOwnSlots; ++s) {
-      const uint32_t i = s * kRunThreads + tid;
-      if (i < nlist) {
-        G[s] = coarse(C[s]);
-        K[s] = atomicAdd(&s_cell[G[s]], 1u);
-        if (ALIAS) {
-          uint32_t no = 0;
+    for (uint32_t s = 0; s < kSlots; ++s) {
+      const uint32_t i = s * kSortThreads + tid;
+      k[s] = make_uint2(0u, 0u);
+      if (i < n) {
+        k[s] = make_uint2(gptr(c.smp_lo)[b + i], gptr(c.smp_d)[b + i]);
+        row[s] = gptr(c.smp_row)[b + i];
+        const uint64_t kk = ((uint64_t)k[s].y << 32) | k[s].x;
+        mx = kk > mx ? kk : mx;
+        mn = ~kk > mn ? ~kk : mn;
+        s_key[i] = k[s];
+      }
+    }
+    mx = wave_max_u64(mx);
+    mn = wave_max_u64(mn);
+    if ((tid & 63u) == 0) {
+      atomicMax((unsigned long long *)&s_mx[0], (unsigned long long)mx);
+      atomicMax((unsigned long long *)&s_mx[1], (unsigned long long)mn);
+    }
+    __syncthreads();
+    const uint64_t top = s_mx[0], span = top - ~s_mx[1];
+    const uint32_t bl = bit_length(span), S = bl > 12u ? bl - 12u : 0u;
 #pragma unroll
-          for (uint32_t a = 0; a < kMaxAlias; ++a) no += AL[s][a] != kNoCell && AL[s][a] != C[s];
-          NO[s] = no;
-          if (no && atomicAdd(&s_nx, no) + no <= kListCap) {
-            XI[s] = true;
-#pragma unroll
-            for (uint32_t a = 0; a < kMaxAlias; ++a)
-              if (AL[s][a] != kNoCell && AL[s][a] != C[s]) XK[s][a] = atomicAdd(&s_xc[coarse(AL[s][a])], 1u);
-          }
-        }
+    for (uint32_t s = 0; s < kSlots; ++s) {
+      if (s * kSortThreads + tid < n) {
+        bin[s] = (uint32_t)((top - (((uint64_t)k[s].y << 32) | k[s].x)) >> S);
+        at[s] = atomicAdd(&s_bin[bin[s]], 1u);
       }
     }
     __syncthreads();
-    {  // exclusive scan of the cell counts, kCellsPerThread consecutive cells per thread
-      constexpr uint32_t kV = kCellsPerThread / 4;
-      uint4 v[kV];
-      uint32_t sum = 0;
+    {
+      static_assert(kSlots == 8, "two uint4 of bins a thread");
+      uint4 v[2];
+      uint32_t sum = 0, tot;
 #pragma unroll
-      for (uint32_t j = 0; j < kV; ++j) {
-        v[j] = reinterpret_cast<const uint4 *>(s_cell)[kV * tid + j];
+      for (uint32_t j = 0; j < 2; ++j) {
+        v[j] = reinterpret_cast<const uint4 *>(s_bin)[2 * tid + j];
         sum += v[j].x + v[j].y + v[j].z + v[j].w;
       }
-      uint32_t tot;
-      uint32_t pre = block_excl_scan<kRunWaves>(sum, s_wn, &tot);
+      uint32_t pre = block_excl_scan<kWaves>(sum, s_wn, &tot);
 #pragma unroll
-      for (uint32_t j = 0; j < kV; ++j) {
-        const uint4 o = make_uint4(pre, pre + v[j].x, pre + v[j].x + v[j].y,
-                                   pre + v[j].x + v[j].y + v[j].z);
+      for (uint32_t j = 0; j < 2; ++j) {
+        reinterpret_cast<uint4 *>(s_bin)[2 * tid + j] =
+            make_uint4(pre, pre + v[j].x, pre + v[j].x + v[j].y, pre + v[j].x + v[j].y + v[j].z);
         pre += v[j].x + v[j].y + v[j].z + v[j].w;
-        reinterpret_cast<uint4 *>(s_cell)[kV * tid + j] = o;
       }
-      if (tid == 0) s_cell[kCells] = tot;
-      if (ALIAS) {  // the second index's counts, the same way (its own wave sums)
-        uint32_t sum2 = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < kV; ++j) {
-          v[j] = reinterpret_cast<const uint4 *>(s_xc)[kV * tid + j];
-          sum2 += v[j].x + v[j].y + v[j].z + v[j].w;
-        }
-        uint32_t tot2;
-        uint32_t pre2 = block_excl_scan<kRunWaves>(sum2, s_wn + kRunWaves, &tot2);
-#pragma unroll
-        for (uint32_t j = 0; j < kV; ++j) {
-          const uint4 o = make_uint4(pre2, pre2 + v[j].x, pre2 + v[j].x + v[j].y,
-                                     pre2 + v[j].x + v[j].y + v[j].z);
-          pre2 += v[j].x + v[j].y + v[j].z + v[j].w;
-          reinterpret_cast<uint4 *>(s_xc)[kV * tid + j] = o;
-        }
-        if (tid == 0) s_xc[kCells] = tot2;
-      }
+      if (tid == 0) s_bin[kListCap] = tot;
     }
     __syncthreads();
 #pragma unroll
-    for (uint32_t s = 0; s < kOwnSlots; ++s) {
-      const uint32_t i = s * kRunThreads + tid;
-      if (i < nlist) {
-        const uint32_t pos = s_cell[G[s]] + K[s];
-        s_pc[pos] = make_uint4(__float_as_uint(P[s].x), __float_as_uint(P[s].y),
-                               __float_as_uint(P[s].z), pack11(C[s]));
-        s_dd[pos] = __float_as_uint(P[s].w);
-        s_rk[pos] = make_uint2(~R[s].x, R[s].y);
-        if (ALIAS) {
-          // the bucket's cells (pack11), and the records of the other cells
-          // in the second index, or the entry in the pass's list
+    for (uint32_t s = 0; s < kSlots; ++s)
+      if (s * kSortThreads + tid < n) s_at[s_bin[bin[s]] + at[s]] = (uint16_t)(s * kSortThreads + tid);
+    __syncthreads();
 #pragma unroll
-          for (uint32_t a = 0; a < kMaxAlias; ++a) {
-            s_al[pos * kMaxAlias + a] = pack11(AL[s][a]);
-            if (XI[s] && AL[s][a] != kNoCell && AL[s][a] != C[s]) {
-              const uint32_t dst = s_xc[coarse(AL[s][a])] + XK[s][a];
-              s_xp[dst] = make_uint4(__float_as_uint(P[s].x), __float_as_uint(P[s].y),
-                                     __float_as_uint(P[s].z), pack11(AL[s][a]));
-              s_xe[dst] = pos;
-            }
-          }
-          if (NO[s] && !XI[s]) s_alist[atomicAdd(&s_nal, 1u)] = pos;
+    for (uint32_t s = 0; s < kSlots; ++s) {
+      if (s * kSortThreads + tid < n) {
+        const uint32_t b0 = s_bin[bin[s]], b1 = s_bin[bin[s] + 1];
+        const uint64_t kk = ((uint64_t)k[s].y << 32) | k[s].x;
+        uint32_t p = b0;
+        for (uint32_t j = b0; j < b1; ++j) {
+          const uint2 o = s_key[s_at[j]];
+          p += (((uint64_t)o.y << 32) | o.x) > kk ? 1u : 0u;
         }
+        gptr(c.smp_d)[b + p] = k[s].y;
+        gptr(c.smp_lo)[b + p] = k[s].x;
+        gptr(c.smp_row)[b + p] = row[s];
       }
     }
     __syncthreads();
   }
-  // owned entries: sorted entry s * kRunThreads + tid; an empty slot has
-  // distance 0 and key 0 and is never live
-  float x[kOwnSlots], y[kOwnSlots], z[kOwnSlots], d[kOwnSlots];
-  // own cells in pack11 form (the box tests of samples with large cubes) and
-  // 10 bits per axis (a sample's cube centre)
-  uint32_t lo[kOwnSlots], row[kOwnSlots], cc[kOwnSlots], c11[kOwnSlots];
-#pragma unroll
-  for (uint32_t s = 0; s < kOwnSlots; ++s) {
-    const uint32_t i = s * kRunThreads + tid;
-    uint4 e0 = make_uint4(0u, 0u, 0u, 0u);
-    uint2 e1 = make_uint2(0u, 0u);
-    uint32_t e2 = 0;
-    if (i < nlist) {
-      e0 = s_pc[i];
-      e1 = s_rk[i];
-      e2 = s_dd[i];
-    }
-    x[s] = __uint_as_float(e0.x);
-    y[s] = __uint_as_float(e0.y);
-    z[s] = __uint_as_float(e0.z);
-    d[s] = __uint_as_float(e2);
-    lo[s] = e1.x;
-    row[s] = e1.y;
-    c11[s] = e0.w;
-    cc[s] = (e0.w & 1023u) | (((e0.w >> 11) & 1023u) << 10) | ((e0.w >> 22) << 20);
-  }
-  if (WHOLE) {  // the list's cell box (every entry's cell lies in it)
-    uint32_t bmax[3] = {0u, 0u, 0u}, bmin[3] = {0u, 0u, 0u};  // bmin: 1023 - the smallest
-#pragma unroll
-    for (uint32_t s = 0; s < kOwnSlots; ++s) {
-      if (s * kRunThreads + tid < nlist) {
-#pragma unroll
-        for (uint32_t a = 0; a < 3; ++a) {
-          const uint32_t v = (cc[s] >> (10 * a)) & 1023u;
-          bmax[a] = max(bmax[a], v);
-          bmin[a] = max(bmin[a], 1023u - v);
-        }
-      }
-    }
-#pragma unroll
-    for (uint32_t a = 0; a < 3; ++a) {
-      bmax[a] = wave_max_u32(bmax[a]);
-      bmin[a] = wave_max_u32(bmin[a]);
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (uint32_t a = 0; a < 3; ++a) {
-        atomicMax(&s_lb[a], bmax[a]);
-        atomicMax(&s_lb[3 + a], bmin[a]);
-      }
-    }
-  }
-  uint32_t it = *gptr(c.iter);
-  const uint32_t m = c.m;
-  NSFPS_GLOBAL int32_t *const out = gptr(c.out);
-  NSFPS_GLOBAL float4 *const pick_p = gptr(c.pick_p);
-  NSFPS_GLOBAL uint2 *const pick_c = gptr(c.pick_c);
-  NSFPS_GLOBAL uint32_t *const err = &rs.err;
-  uint32_t np = 0;
-  bool done = false;
-  // The first hot set's histogram: every key is <= kref0 (keys only decrease).
-  // Later ones are counted right after each hot set's walk.
-  uint64_t kref = kref0 > bkey ? kref0 : bkey;
-  uint32_t S = sel_shift(kref, bkey);
-  hist_live(d, lo, bkey, kref, S, s_sel[0], err);
-  __syncthreads();
-  // WHOLE: the list box's corners in pack11 form (an empty list leaves them
-  // crossed, and no cube then holds them both)
-  uint32_t lb_lo = 0, lb_hi = 0;
-  if (WHOLE) {
-    lb_lo = pack11(pack_cell(1023u - s_lb[3], 1023u - s_lb[4], 1023u - s_lb[5]));
-    lb_hi = pack11(pack_cell(s_lb[0], s_lb[1], s_lb[2]));
-  }
-  // coarse grid, kept in vector registers (the scalar file is full in the walk)
-  const uint32_t gsh = s_geo[0], gx = s_geo[1], gy = s_geo[2];
-  const uint32_t gsx = gsh & 255u, gsy = (gsh >> 8) & 255u, gsz = gsh >> 16;
-  NSFPS_RMARK(kRpLoad);
-  if (PROF) pf[kRpRtLoad] = __builtin_amdgcn_s_memrealtime() - rt0;
-  while (true) {
-    uint64_t key[kOwnSlots];
-    bool live[kOwnSlots];
-#pragma unroll
-    for (uint32_t s = 0; s < kOwnSlots; ++s) {
-      key[s] = ((uint64_t)__float_as_uint(d[s]) << 32) | lo[s];
-      live[s] = lo[s] != 0u && key[s] >= bkey;
-    }
-    // ---- hot threshold.  Histogram 0 (window kref, S) holds every live key;
-    // windows of kSelBins bins are refined 8 bits at a time; buffer i % 3 of
-    // step i was zeroed a step (or a hot set) before, and every wave scans it
-    // itself: one barrier per refinement step.
-    uint64_t hth = bkey;
-    uint32_t nlive = 0;
-    {
-      uint64_t wref = kref;
-      uint32_t wS = S, cap = kHot;
-      for (uint32_t step = 0;; ++step) {
-        const uint4 hv = reinterpret_cast<const uint4 *>(s_sel[step % 3])[lane];
-        const uint32_t tot = hv.x + hv.y + hv.z + hv.w;
-        const uint32_t incl = wave_incl_scan(tot);
-        if (step == 0) {
-          nlive = rdlane(incl, 63);
-          if (nlive <= kHot) break;  // every live entry is hot (or none is left)
-        }
-        const uint64_t over = __ballot(incl > cap);  // running totals only grow
-        if (!over) {  // cannot happen (a refined window holds more than cap keys)
-          *err = 4;
-          nlive = 0;
-          break;
-        }
-        const uint32_t c0 = incl - tot, c1 = c0 + hv.x, c2 = c1 + hv.y, c3 = c2 + hv.z;
-        const uint32_t jj = c1 > cap ? 0u : c2 > cap ? 1u : c3 > cap ? 2u : 3u;
-        const uint32_t bf = c1 > cap ? c0 : c2 > cap ? c1 : c3 > cap ? c2 : c3;
-        const uint32_t L = (uint32_t)__builtin_ctzll(over);
-        const uint32_t bs = 4 * L + rdlane(jj, L), before = rdlane(bf, L);
-        if (before >= cap / 2 || wS == 0) {
-          hth = wref - ((uint64_t)bs << wS) + 1;
-          break;
-        }
-        wref -= (uint64_t)bs << wS;
-        cap -= before;
-        wS = wS >= 8u ? wS - 8u : 0u;
-        uint32_t *H = s_sel[(step + 1) % 3];
-#pragma unroll
-        for (uint32_t s = 0; s < kOwnSlots; ++s) {
-          if (live[s] && key[s] <= wref) {
-            const uint64_t bb = (wref - key[s]) >> wS;
-            if (bb < kSelBins) atomicAdd(&H[(uint32_t)bb], 1u);
-          }
-        }
-        if (tid < kSelBins) s_sel[(step + 2) % 3][tid] = 0;
-        __syncthreads();
-      }
-      hth = hth > bkey ? hth : bkey;
-    }
-    if (nlive == 0) break;  // every key is below B: the run ends
-    NSFPS_RMARK(kRpSelect);
-    // ---- hot copies -> LDS, placed by an LDS counter; then one wave computes
-    // every copy's cube (one pass over the cube code rather than one per wave
-    // holding a hot entry).  Unused slots were cleared during the previous
-    // hot set's walk (key 0).
-    {
-      uint64_t bal[kOwnSlots];
-      uint32_t tot = 0;
-#pragma unroll
-      for (uint32_t s = 0; s < kOwnSlots; ++s) {
-        bal[s] = __ballot(live[s] && key[s] >= hth);
-        tot += (uint32_t)__popcll(bal[s]);
-      }
-      uint32_t base = 0;
-      if (lane == 0 && tot) base = atomicAdd(&s_nhot, tot);
-      base = rdlane(base, 0);
-      // raw copies: {cell, ~rank, distance} and {x, y, z, row}
-#pragma unroll
-      for (uint32_t s = 0; s < kOwnSlots; ++s) {
-        const uint32_t hi = base + lanes_below(bal[s]);
-        base += (uint32_t)__popcll(bal[s]);
-        if ((bal[s] >> lane) & 1u) {
-          if (hi < kHot) {
-            s_hx[hi] = make_uint4(cc[s], lo[s], __float_as_uint(d[s]), 0u);
-            s_hp[hi] = make_uint4(__float_as_uint(x[s]), __float_as_uint(y[s]),
-                                  __float_as_uint(z[s]), row[s]);
-            if (ALIAS) s_hpos[hi] = s * kRunThreads + tid;
-          } else {  // cannot happen (at most kHot keys are >= the hot threshold)
-            *err = 2;
-          }
-        }
-      }
-      if (tid < 2 * kWords) s_big[tid] = 0;
-      if (WHOLE && tid < 2 * kWords) s_bigw[WHOLE ? tid : 0] = 0;
-      if (tid == 0) {
-#pragma unroll
-        for (uint32_t w = 0; w < kWords; ++w) {
-          s_lowm[0][w] = 0;
-          s_lowc[0][w] = 0;
-        }
-        s_kmax[0] = 0;
-        s_kmr = 0;
-      }
-      __syncthreads();
-      if (tid < min(s_nhot, kHot)) {  // the first kHot / 64 waves, a copy a lane
-        const uint4 hx = s_hx[tid];
-        const float D = __uint_as_float(hx.z);
-        const SmallHalves sh(c.r);
-        uint32_t h;
-        if (sh.covers(D)) h = sh.packed(D);
-        else h = packed_halves(c.r, D);
-        uint32_t lo_c, hi_c;
-        cube_corners(hx.x, h, b0, b1, b2, lo_c, hi_c);
-        s_hq[0][hot_slot<HOT>(tid)] = make_uint4(pack11(lo_c), pack11(hi_c) | kGuards, hx.y, hx.z);
-        s_hx[tid] = make_uint4(hx.x, pack11(hx.x) | kGuards, pack11(hx.x), h);
-      }
-      __syncthreads();
-    }
-    NSFPS_RMARK(kRpGather);
-    // ---- phases: thread (j, q) works for hot copy j against copies
-    // kCmp q .. kCmp q + kCmp - 1.  A copy's group keeps what the walk needs
-    // once the copy is accepted: its sample index and cube.
-    const uint32_t hj = tid / kCopyLanes, hq = tid % kCopyLanes;
-    const uint32_t room = m - it;  // samples left (>= 1)
-    // Per phase, two barriers: after the ranks (the accepted prefix is known),
-    // and after the next buffer of hot copies is written.
-    uint32_t npk = 0, stop = 0, ph = 0;
-    bool my_acc = false;
-    uint64_t my_key = 0;  // the copy's key at the last phase (0: none, or accepted)
-    uint32_t my_out = 0, my_qc = 0, my_hh = 0;
-    // ALIAS: the cells of copy j's bucket (pack11; kNoCell's packing never
-    // lies in a clipped box).  Unused slots read some entry's cells: they
-    // have key 0 and are never compared.
-    uint32_t ja[kMaxAlias];
-    if (ALIAS) {
-      const uint32_t pj = s_hpos[hj] & (kListCap - 1u);
-#pragma unroll
-      for (uint32_t a = 0; a < kMaxAlias; ++a)
-        ja[a] = a < na ? s_al[pj * kMaxAlias + a] : pack11(kNoCell);
-    }
-    // 1 when (a cell of the bucket of) copy j lies in the box of pack11
-    // corners lo, hig; two cells per bucket (grids near powers of two) take
-    // two tests, more take all kMaxAlias (padding never lies in a box)
-    const bool na2 = na == 2;
-    const auto j_in = [&](uint32_t cg, uint32_t c11, uint32_t lo, uint32_t hig) -> uint32_t {
-      if (!ALIAS) return in_box11(cg, c11, lo, hig);
-      uint32_t r = in_box11(ja[0] | kGuards, ja[0], lo, hig) | in_box11(ja[1] | kGuards, ja[1], lo, hig);
-      if (!na2) {
-#pragma unroll
-        for (uint32_t a = 2; a < kMaxAlias; ++a) r |= in_box11(ja[a] | kGuards, ja[a], lo, hig);
-      }
-      return r;
-    };
-    while (true) {
-      const uint4 me = s_hq[ph][hot_slot<HOT>(hj)];
-      const uint4 mx = s_hx[hj];
-      const uint64_t mkey = ((uint64_t)me.w << 32) | me.z;
-      my_key = mkey;
-      const bool remj = mkey != 0;  // copies taken earlier, and unused slots, have key 0
-      // bit u of cand: copy kCmp q + u is remaining, ranked above j, and its
-      // cube holds j.  The kCmp copies of this lane are read 8 at a time, all
-      // loads of a chunk issued before any use.
-      uint32_t cnt = 0, cand = 0;
-#pragma unroll
-      for (uint32_t c0 = 0; c0 < kCmp; c0 += 8) {
-        uint4 og[8];
-#pragma unroll
-        for (uint32_t v = 0; v < 8; ++v) og[v] = s_hq[ph][kCopyLanes * (c0 + v) + hq];  // copy kCmp hq + c0 + v
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (uint32_t v = 0; v < 8; ++v) {
-          const uint32_t gt = (uint32_t)((((uint64_t)og[v].w << 32) | og[v].z) > mkey);
-          cnt += gt;
-          cand |= (gt & j_in(mx.y, mx.z, og[v].x, og[v].y)) << (c0 + v);
-        }
-      }
-      uint32_t low = 0;
-      if (cand) {  // rare: the exact distance decides
-        const uint4 pj = s_hp[hj];
-        for (uint32_t cm = cand; cm; cm &= cm - 1) {
-          const uint32_t u = (uint32_t)__builtin_ctz(cm);
-          const uint4 pi = s_hp[hq * kCmp + u];
-          const float dd = sqdist(__uint_as_float(pj.x), __uint_as_float(pj.y),
-                                  __uint_as_float(pj.z), __uint_as_float(pi.x),
-                                  __uint_as_float(pi.y), __uint_as_float(pi.z));
-          low |= dd < __uint_as_float(me.w) ? 1u : 0u;
-        }
-      }
-      const uint32_t rank = group_sum<kCopyLanes>(cnt);
-      const bool lowered = group_sum<kCopyLanes>(low) != 0;
-      const bool rep = remj && hq == 0;
-      const bool ge = mkey >= hth;
-      if (rep) s_rank[hj] = rank;
-      if (hq == 0 && !remj) s_rank[hj] = kHot;  // never accepted
-      if (rep && lowered) {
-        atomicOr(&s_lowm[ph][rank >> 6], 1ull << (rank & 63u));
-        atomicOr(&s_lowc[ph][hj >> 6], 1ull << (hj & 63u));
-      }
-      const uint32_t wge = (uint32_t)__popcll(__ballot(rep && ge));
-      const uint32_t wnz = (uint32_t)__popcll(__ballot(rep && ge && me.w != 0u));
-      if (lane == 0) {
-        s_wr[ph][wave][0] = wge;
-        s_wr[ph][wave][1] = wnz;
-      }
-      if (tid == 0) {
-#pragma unroll
-        for (uint32_t w = 0; w < kWords; ++w) {
-          s_lowm[ph ^ 1][w] = 0;
-          s_lowc[ph ^ 1][w] = 0;
-        }
-        s_kmax[ph ^ 1] = 0;
-      }
-      __syncthreads();
-      NSFPS_RMARK(kRpRank);
-      // copies >= the hot threshold with distance > 0 are ranks 0 .. nnz - 1
-      unsigned long long lowm[kWords], lowany = 0;
-#pragma unroll
-      for (uint32_t w = 0; w < kWords; ++w) {
-        lowm[w] = s_lowm[ph][w];
-        lowany |= lowm[w];
-      }
-      uint32_t nge = 0, nnz = 0;
-#pragma unroll
-      for (uint32_t w = 0; w < kRunWaves; ++w) {
-        nge += s_wr[ph][w][0];
-        nnz += s_wr[ph][w][1];
-      }
-      // A lowered copy j bounds the samples of the phase by K_j, its key once
-      // every copy above it that is not lowered is a sample (more samples
-      // only lower it further): ranks at or below K_j wait for the next phase.
-      uint32_t sstop = kHot;
-      if (lowany) {
-        if (remj && lowered) {  // the whole group of a lowered copy
-          const uint32_t lb = hq * kCmp;  // this lane's copies' bits
-          const uint32_t lowc = (uint32_t)(s_lowc[ph][lb >> 6] >> (lb & 63u));
-          uint32_t nk = me.w;
-          uint32_t nm = cand & ~lowc & HotSet<HOT>::kCmpMask;
-          if (nm) {
-            const uint4 pj = s_hp[hj];
-            for (; nm; nm &= nm - 1) {
-              const uint32_t u = (uint32_t)__builtin_ctz(nm);
-              const uint4 pi = s_hp[hq * kCmp + u];
-              const float dd = sqdist(__uint_as_float(pj.x), __uint_as_float(pj.y),
-                                      __uint_as_float(pj.z), __uint_as_float(pi.x),
-                                      __uint_as_float(pi.y), __uint_as_float(pi.z));
-              nk = min(nk, __float_as_uint(dd));  // non-negative floats order like their bits
-            }
-          }
-          const uint64_t K = ((uint64_t)group_min<kCopyLanes>(nk) << 32) | me.z;
-          if (hq == 0) atomicMax(&s_kmax[ph], (unsigned long long)K);
-        }
-        __syncthreads();
-        // the first rank at or below some K_j: the least number of copies
-        // above a K_j is the number above the largest, which every wave
-        // counts over the copies itself
-        const unsigned long long kmax = s_kmax[ph];
-        sstop = 0;
-#pragma unroll
-        for (uint32_t t = 0; t < kHot / 64; ++t) {
-          const uint4 o = s_hq[ph][64 * t + lane];
-          sstop += (uint32_t)__popcll(__ballot((((uint64_t)o.w << 32) | o.z) > kmax));
-        }
-      }
-      // the samples: copies not lowered, ranked below min(stop, nnz), the
-      // first room - npk of them, in rank order
-      const uint32_t seff = min(sstop, nnz);
-      uint64_t accr[kWords];  // by rank
-      uint32_t P = 0;
-#pragma unroll
-      for (uint32_t w = 0; w < kWords; ++w) {
-        const uint32_t r0 = 64 * w;
-        const uint64_t f = seff >= r0 + 64 ? ~0ull : seff > r0 ? (1ull << (seff - r0)) - 1ull : 0ull;
-        accr[w] = f & ~lowm[w];
-        P += (uint32_t)__popcll(accr[w]);
-      }
-      while (P > room - npk) {  // the last samples of the call: the highest ranks go
-#pragma unroll
-        for (int w = (int)kWords - 1; w >= 0; --w) {
-          if (accr[w]) {
-            accr[w] &= ~(1ull << (63 - __clzll(accr[w])));
-            break;
-          }
-        }
-        --P;
-      }
-      // ranks below r among the accepted, and whether r is accepted
-      const auto acc_below = [&](uint32_t r) -> uint32_t {
-        uint32_t b = 0;
-#pragma unroll
-        for (uint32_t w = 0; w < kWords; ++w) {
-          const uint32_t r0 = 64 * w;
-          b += r >= r0 + 64 ? (uint32_t)__popcll(accr[w])
-               : r > r0     ? (uint32_t)__popcll(accr[w] & ((1ull << (r - r0)) - 1ull))
-                            : 0u;
-        }
-        return b;
-      };
-      const auto acc_has = [&](uint32_t r) -> bool {
-        return (accr[(r >> 6) & (kWords - 1u)] >> (r & 63u)) & 1u;
-      };
-      if (P == 0) {  // rank 0: below the hot threshold, or distance 0
-        stop = (nge == 0) ? 1u : 2u;
-        break;
-      }
-      const bool acc = remj && rank < kHot && acc_has(rank);
-      if (acc) {
-        my_acc = true;
-        my_key = 0;
-        my_out = npk + acc_below(rank);
-        my_qc = mx.x;
-        my_hh = mx.w;
-      }
-      npk += P;
-      if (npk >= room) {  // the last sample needs no update
-        stop = 2;
-        break;
-      }
-      if (P >= nnz && nnz < nge) {  // the next copy has distance 0: src/yuezu_fps.cpp:705-706
-        stop = 2;
-        break;
-      }
-      // few copies left: they go back to the next selection (always so at
-      // kPhaseMin = kHot, at most kHot copies being >= the hot threshold)
-      if (kPhaseMin >= kHot || nge - P < kPhaseMin) {
-        stop = P >= nge ? 1u : 0u;
-        break;
-      }
-      // the accepted cubes on the remaining copies
-      const bool remj2 = remj && !acc;
-      uint32_t mnb = 0xffffffffu;
-      if (remj2) {
-        uint32_t rk[kCmp];
-#pragma unroll
-        for (uint32_t v = 0; v < kCmp / 4; ++v) {
-          const uint4 r4 = reinterpret_cast<const uint4 *>(s_rank)[hq * (kCmp / 4) + v];
-          rk[4 * v] = r4.x;
-          rk[4 * v + 1] = r4.y;
-          rk[4 * v + 2] = r4.z;
-          rk[4 * v + 3] = r4.w;
-        }
-        uint32_t cand2 = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < kCmp; ++u) {
-          const uint4 o = s_hq[ph][kCopyLanes * u + hq];
-          cand2 |= ((rk[u] < kHot ? (uint32_t)acc_has(rk[u]) : 0u) & j_in(mx.y, mx.z, o.x, o.y)) << u;
-        }
-        if (cand2) {  // rare: the exact distances
-          const uint4 pj = s_hp[hj];
-          while (cand2) {
-            const uint32_t u = (uint32_t)__builtin_ctz(cand2);
-            cand2 &= cand2 - 1;
-            const uint4 pi = s_hp[hq * kCmp + u];
-            const float dd = sqdist(__uint_as_float(pj.x), __uint_as_float(pj.y),
-                                    __uint_as_float(pj.z), __uint_as_float(pi.x),
-                                    __uint_as_float(pi.y), __uint_as_float(pi.z));
-            mnb = min(mnb, __float_as_uint(dd));  // non-negative floats order like their bits
-          }
-        }
-      }
-      mnb = group_min<kCopyLanes>(mnb);
-      // the next buffer: accepted copies get key 0, lowered ones new cubes
-      if (hq == 0) {
-        uint4 nv = me;
-        if (acc) {
-          nv.z = 0u;
-          nv.w = 0u;
-        } else if (remj && mnb < me.w) {
-          const uint32_t h = packed_halves(c.r, __uint_as_float(mnb));
-          uint32_t lo_c, hi_c;
-          cube_corners(mx.x, h, b0, b1, b2, lo_c, hi_c);
-          nv = make_uint4(pack11(lo_c), pack11(hi_c) | kGuards, me.z, mnb);
-          s_hx[hj].w = h;
-        }
-        s_hq[ph ^ 1][hot_slot<HOT>(hj)] = nv;
-      }
-      __syncthreads();
-      ph ^= 1;
-      NSFPS_RMARK(kRpPhases);
-      if (PROF) pf[kRpPhaseCount] += 1;
-    }
-    NSFPS_RMARK(kRpPhases);
-    // ---- the hot run's samples -> global memory and every list entry.
-    // The group of an accepted copy walks the coarse rows its cube spans,
-    // min-ing distances into LDS.  A cube over more than kWalkRows rows, or a
-    // lane meeting more than kWalkLaneEntries entries in its rows, flags the
-    // sample instead; flagged samples are applied below by every thread to its
-    // own entries (applying a sample twice changes nothing).  Meanwhile the
-    // next hot set's copy buffer and first histogram are cleared, and the
-    // largest key of a copy left unaccepted bounds the next histogram.
-    {
-      const uint32_t q = hq;
-      if (tid < kHot) s_hq[0][tid] = make_uint4(0u, 0u, 0u, 0u);
-      if (tid < kSelBins) s_sel[0][tid] = 0;
-      if (q == 0 && my_key != 0) atomicMax(&s_kmr, (unsigned long long)my_key);
-      if (my_acc) {
-        const uint4 rp = s_hp[hj];
-        const uint32_t qc = my_qc, hh = my_hh;
-        uint32_t lo_c, hi_c;
-        cube_corners(qc, hh, b0, b1, b2, lo_c, hi_c);
-        const uint32_t lo11 = pack11(lo_c), hi11g = pack11(hi_c) | kGuards;
-        if (q == 0) {
-          out[it + my_out] = (int32_t)rp.w;
-          pick_p[np + my_out] = make_float4(__uint_as_float(rp.x), __uint_as_float(rp.y),
-                                            __uint_as_float(rp.z), 0.f);
-          pick_c[np + my_out] = make_uint2(lo11, hi11g);
-          s_rp[hj] = rp;
-          s_rc[hj] = make_uint2(lo11, hi11g);
-          if (ALIAS) {
-            s_sbox[my_out] = make_uint2(lo11, hi11g);
-            s_spos[my_out] = make_float4(__uint_as_float(rp.x), __uint_as_float(rp.y),
-                                         __uint_as_float(rp.z), 0.f);
-          }
-        }
-        const uint32_t x0 = (lo_c & 1023u) >> gsx, x1 = (hi_c & 1023u) >> gsx;
-        const uint32_t y0 = ((lo_c >> 10) & 1023u) >> gsy, y1 = ((hi_c >> 10) & 1023u) >> gsy;
-        const uint32_t z0 = (lo_c >> 20) >> gsz, z1 = (hi_c >> 20) >> gsz;
-        const uint32_t ny = y1 - y0 + 1, nrows = ny * (z1 - z0 + 1);
-        bool big = nrows > WalkLimits<HOT, ROWS>::kRows;
-        if (!big) {
-          // row rr = rz * ny + ry; rz = floor((rr + 0.5) / ny) holds with an
-          // approximate reciprocal: rr < 64 leaves a margin of 0.5 / ny
-          const float rny = __builtin_amdgcn_rcpf((float)ny);
-          const float px = __uint_as_float(rp.x), py = __uint_as_float(rp.y),
-                      pz = __uint_as_float(rp.z);
-          // four entries per step, their reads in flight together (a short
-          // last step repeats an entry: min is idempotent); one 16-byte read
-          // each, and the min is unconditional (a no-op outside the cube), so
-          // the cell is not read ahead of the coordinates
-          const auto walk4 = [&](const uint32_t(&ee)[4]) {
-            uint4 pe[4];
-#pragma unroll
-            for (uint32_t t = 0; t < 4; ++t) pe[t] = s_pc[ee[t]];
-#pragma unroll
-            for (uint32_t t = 0; t < 4; ++t) {
-              const uint32_t dt =
-                  __float_as_uint(sqdist(__uint_as_float(pe[t].x), __uint_as_float(pe[t].y),
-                                         __uint_as_float(pe[t].z), px, py, pz));
-              // non-negative floats order like their bits
-              atomicMin(&s_dd[ee[t]],
-                        in_box11(pe[t].w | kGuards, pe[t].w, lo11, hi11g) ? dt : 0xffffffffu);
-            }
-          };
-          if (!ALIAS) {
-            // the lane's rows (rr = q, q + kCopyLanes, ...): their entry
-            // ranges read up front (one LDS wait; a lane with fewer rows reads
-            // row 0's again and counts it empty), then their entries walked
-            // as one list.  Per call, against row by row (whose last step in
-            // each row mostly repeats): uniform cube 2.6 % and LiDAR scan
-            // 5.5 % faster, clustered cloud (full rows) 2.5 % slower.
-            constexpr uint32_t kLaneRows = (WalkLimits<HOT, ROWS>::kRows + kCopyLanes - 1) / kCopyLanes;
-            uint32_t rs[kLaneRows], rn[kLaneRows], ne = 0;
-#pragma unroll
-            for (uint32_t t = 0; t < kLaneRows; ++t) {
-              const bool ok = q + t * kCopyLanes < nrows;
-              const uint32_t rr = ok ? q + t * kCopyLanes : 0u;
-              const uint32_t rz = (uint32_t)(((float)rr + 0.5f) * rny), ry = rr - rz * ny;
-              const uint32_t rw = ((z0 + rz) * gy + y0 + ry) * gx;
-              const uint32_t e0 = s_cell[rw + x0], e1 = s_cell[rw + x1 + 1];
-              rs[t] = e0;
-              rn[t] = ok ? e1 - e0 : 0u;
-              ne += rn[t];
-            }
-            // more entries than the lane's budget: the sample is flagged (the
-            // same samples as a row-by-row test: running totals only grow)
-            if (ne > WalkLimits<HOT, ROWS>::kLaneEntries) {
-              big = true;
-            } else {
-              for (uint32_t f = 0; f < ne; f += 4) {
-                uint32_t ee[4];
-#pragma unroll
-                for (uint32_t t = 0; t < 4; ++t) {  // list position -> entry
-                  const uint32_t ff = f + t < ne ? f + t : ne - 1;
-                  uint32_t e = rs[0] + ff, acc = rn[0];
-#pragma unroll
-                  for (uint32_t u = 1; u < kLaneRows; ++u) {
-                    e = ff >= acc ? rs[u] + (ff - acc) : e;
-                    acc += rn[u];
-                  }
-                  ee[t] = e;
-                }
-                walk4(ee);
-              }
-            }
-          } else {
-            // shared buckets: row by row, each row's entries and then the
-            // other-cell records of its coarse cells (the budget counts both)
-            uint32_t budget = kWalkLaneEntries;
-            for (uint32_t rr = q; rr < nrows; rr += kCopyLanes) {
-              const uint32_t rz = (uint32_t)(((float)rr + 0.5f) * rny), ry = rr - rz * ny;
-              const uint32_t rw = ((z0 + rz) * gy + y0 + ry) * gx;
-              const uint32_t e0 = s_cell[rw + x0], e1 = s_cell[rw + x1 + 1];
-              const uint32_t f0 = s_xc[rw + x0], f1 = s_xc[rw + x1 + 1];
-              if (e1 - e0 + (f1 - f0) > budget) {
-                big = true;
-                break;
-              }
-              budget -= e1 - e0 + (f1 - f0);
-              for (uint32_t e = e0; e < e1; e += 4) {
-                uint32_t ee[4];
-#pragma unroll
-                for (uint32_t t = 0; t < 4; ++t) ee[t] = e + t < e1 ? e + t : e1 - 1;
-                walk4(ee);
-              }
-              for (uint32_t f = f0; f < f1; ++f) {
-                const uint4 pa = s_xp[f];
-                const uint32_t ea = s_xe[f];
-                const uint32_t da =
-                    __float_as_uint(sqdist(__uint_as_float(pa.x), __uint_as_float(pa.y),
-                                           __uint_as_float(pa.z), px, py, pz));
-                atomicMin(&s_dd[ea], in_box11(pa.w | kGuards, pa.w, lo11, hi11g) ? da : 0xffffffffu);
-              }
-            }
-          }
-        }
-        if (big) {
-          // WHOLE: a cube holding the list box holds every entry's cell
-          const bool all = WHOLE && (in_box11(lb_lo | kGuards, lb_lo, lo11, hi11g) &
-                                     in_box11(lb_hi | kGuards, lb_hi, lo11, hi11g)) != 0;
-          if (all) atomicOr(&s_bigw[WHOLE ? hj >> 5 : 0], 1u << (hj & 31u));
-          else atomicOr(&s_big[hj >> 5], 1u << (hj & 31u));
-        }
-      }
-      NSFPS_RMARK(kRpWalk);
-      __syncthreads();  // the walks' updates are in LDS
-      NSFPS_RMARK(kRpWalkWait);
-      if (ALIAS) {
-        // the entries whose other cells did not fit the second index (the
-        // walk reached them by their own cell alone), against every sample
-        // of the hot set: a thread per entry; lane k of every wave holds
-        // sample k's cube corners, which the loop reads lane by lane (the
-        // walk is done, so the thread owns the entry's distance)
-        const uint32_t nal = uniform(s_nal), nk = uniform(npk);
-        const uint2 bx = s_sbox[lane < nk ? lane : 0u];
-        if (PROF) pf[kRpAliasN] += nal;
-        for (uint32_t ia = tid; ia < nal; ia += kRunThreads) {
-          const uint32_t pe = s_alist[ia];
-          const uint4 pp = s_pc[pe];
-          uint32_t dm = s_dd[pe];
-          // sample k's cube holds another cell of the bucket (rare): its distance
-          const auto take = [&](uint32_t k) {
-            const float4 q = s_spos[k];
-            const float dd = sqdist(__uint_as_float(pp.x), __uint_as_float(pp.y),
-                                    __uint_as_float(pp.z), q.x, q.y, q.z);
-            dm = min(dm, __float_as_uint(dd));  // non-negative floats order like their bits
-          };
-          // every cell of the bucket (its own again: min is idempotent)
-          uint32_t eo[kMaxAlias];
-#pragma unroll
-          for (uint32_t a = 0; a < kMaxAlias; ++a)
-            eo[a] = a < na ? s_al[pe * kMaxAlias + a] : pack11(kNoCell);
-          for (uint32_t k = 0; k < nk; ++k) {
-            const uint32_t lo = rdlane(bx.x, k), hig = rdlane(bx.y, k);
-            uint32_t in = 0;
-#pragma unroll
-            for (uint32_t a = 0; a < kMaxAlias; ++a)
-              in |= in_box11(eo[a] | kGuards, eo[a], lo, hig);
-            if (in) take(k);
-          }
-          s_dd[pe] = dm;
-        }
-        __syncthreads();
-        NSFPS_RMARK(kRpAlias);
-      }
-#pragma unroll
-      for (uint32_t s = 0; s < kOwnSlots; ++s)
-        if (s * kRunThreads + tid < nlist) d[s] = __uint_as_float(s_dd[s * kRunThreads + tid]);
-      NSFPS_RMARK(kRpApply);
-      uint64_t bigm[kWords], bigw[kWords], bany = 0;
-#pragma unroll
-      for (uint32_t w = 0; w < kWords; ++w) {
-        bigm[w] = ((uint64_t)uniform(s_big[2 * w + 1]) << 32) | uniform(s_big[2 * w]);
-        bigw[w] = WHOLE ? ((uint64_t)uniform(s_bigw[WHOLE ? 2 * w + 1 : 0]) << 32) |
-                              uniform(s_bigw[WHOLE ? 2 * w : 0])
-                        : 0ull;
-        bany |= bigm[w] | bigw[w];
-      }
-      if (bany) {
-        // branch-free (the distance is always computed, the box test masks
-        // it), two samples a trip so that their LDS reads overlap; a lone
-        // last sample is applied twice (min is idempotent)
-        const auto take = [&](const uint4 a0, const uint2 bx) {
-#pragma unroll
-          for (uint32_t s = 0; s < kOwnSlots; ++s) {
-            uint32_t in = in_box11(c11[s] | kGuards, c11[s], bx.x, bx.y);
-            if (ALIAS) {  // every cell of the bucket (the own cell among them)
-              const uint32_t i = s * kRunThreads + tid;
-              for (uint32_t a = 0; a < na; ++a) {
-                const uint32_t e = s_al[i * kMaxAlias + a];
-                in |= in_box11(e | kGuards, e, bx.x, bx.y);
-              }
-            }
-            const float dd = sqdist(x[s], y[s], z[s], __uint_as_float(a0.x),
-                                    __uint_as_float(a0.y), __uint_as_float(a0.z));
-            // non-negative floats order like their bits; outside the cube the
-            // distance becomes all ones, which never wins
-            d[s] = __uint_as_float(min(__float_as_uint(d[s]), __float_as_uint(dd) | (in - 1u)));
-          }
-        };
-        // WHOLE: a sample whose cube holds the list box holds every entry's
-        // cell, and takes the distances with no cell test
-        const auto take_all = [&](const uint4 a0) {
-#pragma unroll
-          for (uint32_t s = 0; s < kOwnSlots; ++s) {
-            const float dd = sqdist(x[s], y[s], z[s], __uint_as_float(a0.x),
-                                    __uint_as_float(a0.y), __uint_as_float(a0.z));
-            d[s] = __uint_as_float(min(__float_as_uint(d[s]), __float_as_uint(dd)));
-          }
-        };
-#pragma unroll
-        for (uint32_t w = 0; w < kWords; ++w) {
-          uint64_t bm = bigw[w];
-          while (WHOLE && bm) {
-            const uint32_t ka = 64 * w + (uint32_t)__builtin_ctzll(bm);
-            bm &= bm - 1;
-            const uint32_t kc = bm ? 64 * w + (uint32_t)__builtin_ctzll(bm) : ka;
-            bm &= bm - 1;
-            const uint4 a0 = s_rp[ka], a1 = s_rp[kc];
-            take_all(a0);
-            take_all(a1);
-          }
-          bm = bigm[w];
-          while (bm) {
-            const uint32_t ka = 64 * w + (uint32_t)__builtin_ctzll(bm);
-            bm &= bm - 1;
-            const uint32_t kc = bm ? 64 * w + (uint32_t)__builtin_ctzll(bm) : ka;
-            bm &= bm - 1;
-            const uint4 a0 = s_rp[ka], a1 = s_rp[kc];
-            const uint2 b0 = s_rc[ka], b1 = s_rc[kc];
-            take(a0, b0);
-            take(a1, b1);
-          }
-        }
-#pragma unroll
-        for (uint32_t s = 0; s < kOwnSlots; ++s)
-          if (s * kRunThreads + tid < nlist) s_dd[s * kRunThreads + tid] = __float_as_uint(d[s]);
-      }
-      NSFPS_RMARK(kRpBig);
-    }
-    it += npk;
-    np += npk;
-    if (PROF) pf[kRpHotRounds] += 1;
-    if (stop == 2) {
-      done = true;
-      break;
-    }
-    if (hth == bkey && stop == 1) break;  // every live entry was hot: all below B now
-    // ---- the next hot set's first histogram.  Live keys are below the hot
-    // threshold, or belong to a copy left unaccepted (at most its last key).
-    {
-      const uint64_t kmr = s_kmr;
-      kref = hth > bkey ? hth - 1 : bkey;
-      kref = kmr > kref ? kmr : kref;
-      S = sel_shift(kref, bkey);
-      hist_live(d, lo, bkey, kref, S, s_sel[0], err);
-      if (tid < kSelBins) s_sel[1][tid] = 0;
-      if (tid == 0) s_nhot = 0;
-      __syncthreads();
-    }
-    NSFPS_RMARK(kRpPublish);
-  }
-  if (tid == 0) {
-    *gptr(c.iter) = it;
-    rs.npicks = np;
-    rs.kref0 = bkey - 1;  // every key is below the threshold now
-    rs.s0 = rs.s0_next;
-    rs.nlist = 0;
-    rs.rounds += 1;
-    if (done) *gptr(c.done) = 1;
-  }
-  // the histograms this round's selection read are cleared for the next
-  // round's update pass (16-byte stores: three a thread)
-  NSFPS_GLOBAL uint4 *const hz = reinterpret_cast<NSFPS_GLOBAL uint4 *>(hist_set(c));
-  for (uint32_t j = tid; j < kHists * kHistBins / 4; j += kRunThreads) hz[j] = make_uint4(0u, 0u, 0u, 0u);
-  if (PROF && tid == 0) {
-    NSFPS_RMARK(kRpTail);
-    pf[kRpPicks] = np;
-    pf[kRpRounds] = 1;
-    pf[kRpRtTotal] = __builtin_amdgcn_s_memrealtime() - rt0;
-    NSFPS_GLOBAL uint64_t *pw = gptr(c.prof);
-    for (uint32_t i = 0; i < kRpWords; ++i) pw[i] += pf[i];
-    for (uint32_t i = kRpWords; i < kRpLocal; ++i) pw[kRpExtraAt + i - kRpWords] += pf[i];
-  }
-#undef NSFPS_RMARK
 }
 
-template <bool PROF, bool ALIAS, uint32_t HOT, uint32_t ROWS, bool WHOLE>
-__global__ __launch_bounds__(kRunThreads) void k_run(const CloudDev *__restrict__ clouds) {
-  run_list<PROF, ALIAS, HOT, ROWS, WHOLE>(clouds[blockIdx.x]);
+// The samples' places: sample i's is the number of samples with larger keys.
+// Samples of rounds whose smallest threshold so far is above its key all
+// precede it, those of rounds whose largest key is below it all follow; in
+// the rounds between (sorted by key) binary searches find how many precede
+// it.  Bound by the latency of their reads: kOrderLanes lanes per sample take
+// a round each (1,000 samples: 18 us with one lane a sample, 5 so).
+constexpr uint32_t kOrderThreads = 256;
+constexpr uint32_t kOrderLanes = 16;
+__global__ __launch_bounds__(kOrderThreads) void k_order(const CloudDev *__restrict__ clouds) {
+  const CloudDev &c = clouds[blockIdx.y];
+  if (!*gptr(c.done)) return;
+  const NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
+  constexpr uint32_t kPer = kOrderThreads / kOrderLanes;  // samples of a workgroup
+  const uint32_t T = min(rs.ntaken, c.n), nlog = rs.nlog, m = c.m;
+  const uint32_t sub = threadIdx.x % kOrderLanes;
+  const NSFPS_GLOBAL uint32_t *const sd = gptr(c.smp_d), *const sl = gptr(c.smp_lo);
+  for (uint32_t i = blockIdx.x * kPer + threadIdx.x / kOrderLanes; i < T; i += gridDim.x * kPer) {
+    const uint64_t k = ((uint64_t)sd[i] << 32) | sl[i];
+    uint32_t r = 0;
+    if (i) {  // sample 0 (input row 0) has the largest key and is in no round
+      uint32_t a0 = 0, a1 = nlog, e0 = 0, e1 = nlog;
+      while (a0 < a1) {  // the first round whose smallest threshold so far is <= k
+        const uint32_t mid = (a0 + a1) / 2;
+        if (gptr(c.log_bmin)[mid] <= k) a1 = mid;
+        else a0 = mid + 1;
+      }
+      while (e0 < e1) {  // the first round whose largest key is < k
+        const uint32_t mid = (e0 + e1) / 2;
+        if (gptr(c.log_ktop)[mid] < k) e1 = mid;
+        else e0 = mid + 1;
+      }
+      if (sub == 0) r = a0 < nlog ? gptr(c.log_start)[a0] : T;
+      for (uint32_t q = a0 + sub; q < e0; q += kOrderLanes) {
+        const uint32_t b = gptr(c.log_start)[q], e = q + 1 < nlog ? gptr(c.log_start)[q + 1] : T;
+        if (e - b > kListCap) {  // not sorted
+          for (uint32_t j = b; j < e; ++j) r += (((uint64_t)sd[j] << 32) | sl[j]) > k ? 1u : 0u;
+        } else if (i >= b && i < e) {
+          r += i - b;
+        } else {
+          uint32_t lo = b, hi = e;
+          while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            const uint32_t d = sd[mid];
+            if (d > (uint32_t)(k >> 32) || (d == (uint32_t)(k >> 32) && sl[mid] > (uint32_t)k)) lo = mid + 1;
+            else hi = mid;
+          }
+          r += lo - b;
+        }
+      }
+    }
+#pragma unroll
+    for (uint32_t off = kOrderLanes / 2; off; off >>= 1) r += __shfl_xor(r, off, kOrderLanes);
+    if (sub == 0 && r < m) gptr(c.out)[r] = (int32_t)gptr(c.smp_row)[i];
+  }
 }
-
 
 // ------------------------------------------------------------------ setup
 
 // First round: the only pick is input row 0 (the first sample) with a cube
 // over the whole grid.
 __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__restrict__ clouds,
-                                                           bool split) {
+                                                           uint32_t split) {
   const CloudDev &c = clouds[blockIdx.x];
   const uint32_t tid = threadIdx.x;
   // split: each node's key moves into its first part (the other parts and
@@ -1990,16 +1213,24 @@ __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__re
     rs.bkey = 0;
     rs.s0 = kMaxShift;
     rs.s0_next = kMaxShift;
-    rs.npicks = 1;
-    rs.nlist = 0;
+    rs.nb = rs.nb_next = kHistBins;
+    rs.nl[0] = 0;
+    rs.nl[1] = 1;  // read by round 0
+    rs.ntaken = 1;
+    rs.nlog = 0;
+    rs.cap = min(kListMin, c.list_cap);
+    rs.bmin = ~0ull;
+    rs.ktop = ~0ull;
     rs.rounds = 0;
     rs.err = 0;
     rs.forced = 0;
     const float4 p0 = *gptr(c.root_pos);
-    gptr(c.pick_p)[0] = make_float4(p0.x, p0.y, p0.z, INFINITY);
-    gptr(c.pick_c)[0] = make_uint2(
+    gptr(c.smp_d)[0] = gptr(c.smp_lo)[0] = 0xffffffffu;
+    gptr(c.smp_row)[0] = 0;
+    gptr(c.list_f)[0] = 0;
+    gptr(c.list_p)[0] = make_float4(p0.x, p0.y, p0.z, INFINITY);
+    gptr(c.list_c)[0] = make_uint2(
         0u, pack11(pack_cell(c.r.blocks[0] - 1, c.r.blocks[1] - 1, c.r.blocks[2] - 1)) | kGuards);
-    gptr(c.out)[0] = 0;
     *gptr(c.iter) = 1;
     *gptr(c.done) = c.m <= 1 ? 1u : 0u;
   }
@@ -2012,72 +1243,64 @@ __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__re
 hipError_t preload_runs_kernels() {
   constexpr uint32_t S = kUpdateSplit;
   return func_attributes(
-      k_runs_init, k_refine, k_gather<false, false>, k_gather<false, true>,
-      k_run<false, false, 64, kWalkRows, false>, k_run<false, false, 64, kWalkRows, true>,
-      k_run<false, false, 128, kWalkRows, false>, k_run<false, false, 128, kDenseWalkRows, false>,
-      k_run<false, true, 64, kWalkRows, false>, k_update<false, false, false, 1, false>, k_update<false, false, false, S, false>,
-      k_update<false, false, true, 1, false>, k_update<false, false, true, S, false>,
-      k_update<false, true, false, 1, false>, k_update<false, true, false, S, false>,
-      k_update<false, true, true, 1, false>, k_update<false, true, true, S, false>,
-      k_update<false, false, false, 1, true>, k_update<false, false, false, S, true>,
-      k_update<false, false, true, 1, true>, k_update<false, false, true, S, true>);
+      k_runs_init, k_refine, k_gather<false>, k_accept, k_sort_rounds, k_order,
+      k_update<false, false, 1, false>, k_update<false, false, S, false>,
+      k_update<false, true, 1, false>, k_update<false, true, S, false>,
+      k_update<false, false, 1, true>, k_update<false, false, S, true>);
 }
 
-hipError_t launch_runs_init(const CloudDev *d_clouds, uint32_t nclouds, bool split,
+hipError_t launch_runs_init(const CloudDev *d_clouds, uint32_t nclouds, uint32_t split,
                             hipStream_t st) {
   k_runs_init<<<nclouds, kPassThreads, 0, st>>>(d_clouds, split);
   return hipGetLastError();
 }
 
-// The classic round's update, gather and run kernels of one variant; hot:
-// the run kernel's hot-set size where cells do not share buckets (64 or 128);
-// dense: 128-copy sets walk at most kDenseWalkRows rows.
-template <bool PROF, bool ALIAS, bool LB, uint32_t SPLIT, bool MIXED>
-void launch_classic(const CloudDev *d_clouds, uint32_t nclouds, dim3 grid, dim3 sparse,
-                    uint32_t passes, uint32_t hot, bool dense, bool whole, hipStream_t st) {
-  k_update<PROF, ALIAS, LB, SPLIT, MIXED>
-      <<<dim3(grid.x * SPLIT, grid.y), kPassThreads, 0, st>>>(d_clouds);
+// Round `round` of one variant: update (and one workgroup recording the last
+// round's samples), gather and accept passes.
+template <bool PROF, bool ALIAS, uint32_t SPLIT, bool MIXED>
+void launch_round(const CloudDev *d_clouds, uint32_t nclouds, dim3 grid, dim3 sparse,
+                  uint32_t passes, uint32_t list_cap, uint32_t round, hipStream_t st) {
+  k_update<PROF, ALIAS, SPLIT, MIXED>
+      <<<dim3(grid.x * SPLIT + 1, grid.y), kPassThreads, 0, st>>>(d_clouds, round);
   for (uint32_t p = 1; p <= passes; ++p)
     k_refine<<<sparse, kPassThreads, 0, st>>>(d_clouds, p, passes);
-  k_gather<PROF, ALIAS><<<sparse, kPassThreads, 0, st>>>(d_clouds, passes);
-  if (!ALIAS && hot == 128 && dense)
-    k_run<PROF, false, 128, kDenseWalkRows, false><<<nclouds, kRunThreads, 0, st>>>(d_clouds);
-  else if (!ALIAS && hot == 128)
-    k_run<PROF, false, 128, kWalkRows, false><<<nclouds, kRunThreads, 0, st>>>(d_clouds);
-  else if (!ALIAS && whole)
-    k_run<PROF, false, 64, kWalkRows, true><<<nclouds, kRunThreads, 0, st>>>(d_clouds);
-  else
-    k_run<PROF, ALIAS, 64, kWalkRows, false><<<nclouds, kRunThreads, 0, st>>>(d_clouds);
+  k_gather<PROF><<<sparse, kPassThreads, 0, st>>>(d_clouds, passes, round & 1u);
+  const uint32_t ncube = (list_cap + kAcceptThreads - 1) / kAcceptThreads;
+  const uint32_t xgs = list_cap / kAcceptX;
+  k_accept<<<dim3(ncube + xgs * (list_cap / kAcceptChunk) / kAcceptWaves, nclouds),
+             kAcceptThreads, 0, st>>>(d_clouds, round & 1u, ncube);
+}
+
+hipError_t launch_order(const CloudDev *d_clouds, uint32_t nclouds, uint32_t m, hipStream_t st) {
+  // some more samples than m are settled
+  const uint32_t want = (uint32_t)(((uint64_t)m + m / 8) * kOrderLanes / kOrderThreads) + 2;
+  k_sort_rounds<<<dim3(m < 64u ? m : nclouds > 1 ? 64u : 256u, nclouds), kSortThreads, 0, st>>>(d_clouds);
+  k_order<<<dim3(want < 8192u ? want : 8192u, nclouds), kOrderThreads, 0, st>>>(d_clouds);
+  return hipGetLastError();
 }
 
 hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t max_nl1,
                          uint32_t rounds, uint32_t passes, bool profile, bool alias,
-                         bool leaf_bound, bool split, bool mixed, uint32_t hot, bool dense,
-                         bool whole, hipStream_t st) {
+                         bool split, bool mixed, uint32_t list_cap, uint32_t first,
+                         hipStream_t st) {
   if (alias && mixed) return hipErrorInvalidValue;  // leaves of several buckets: one cell each
-  if (hot != 64 && hot != 128) return hipErrorInvalidValue;
+  if (list_cap != kListShort && list_cap != kListCap) return hipErrorInvalidValue;
   const dim3 grid(max_nl1, nclouds);
   const dim3 sparse(max_nl1 < kSparseGroups ? max_nl1 : kSparseGroups, nclouds);
-  using Launch = void (*)(const CloudDev *, uint32_t, dim3, dim3, uint32_t, uint32_t, bool, bool,
+  using Launch = void (*)(const CloudDev *, uint32_t, dim3, dim3, uint32_t, uint32_t, uint32_t,
                           hipStream_t);
   constexpr uint32_t S = kUpdateSplit;
-  // [profile][cells: one per leaf, shared buckets, several per leaf][leaf_bound][split]
-  static constexpr Launch kClassic[2][3][2][2] = {
-      {{{launch_classic<false, false, false, 1, false>, launch_classic<false, false, false, S, false>},
-        {launch_classic<false, false, true, 1, false>, launch_classic<false, false, true, S, false>}},
-       {{launch_classic<false, true, false, 1, false>, launch_classic<false, true, false, S, false>},
-        {launch_classic<false, true, true, 1, false>, launch_classic<false, true, true, S, false>}},
-       {{launch_classic<false, false, false, 1, true>, launch_classic<false, false, false, S, true>},
-        {launch_classic<false, false, true, 1, true>, launch_classic<false, false, true, S, true>}}},
-      {{{launch_classic<true, false, false, 1, false>, launch_classic<true, false, false, S, false>},
-        {launch_classic<true, false, true, 1, false>, launch_classic<true, false, true, S, false>}},
-       {{launch_classic<true, true, false, 1, false>, launch_classic<true, true, false, S, false>},
-        {launch_classic<true, true, true, 1, false>, launch_classic<true, true, true, S, false>}},
-       {{launch_classic<true, false, false, 1, true>, launch_classic<true, false, false, S, true>},
-        {launch_classic<true, false, true, 1, true>, launch_classic<true, false, true, S, true>}}}};
-  const Launch classic = kClassic[profile][alias ? 1 : mixed ? 2 : 0][leaf_bound][split];
+  // [profile][cells: one per leaf, shared buckets, several per leaf][split]
+  static constexpr Launch kRound[2][3][2] = {
+      {{launch_round<false, false, 1, false>, launch_round<false, false, S, false>},
+       {launch_round<false, true, 1, false>, launch_round<false, true, S, false>},
+       {launch_round<false, false, 1, true>, launch_round<false, false, S, true>}},
+      {{launch_round<true, false, 1, false>, launch_round<true, false, S, false>},
+       {launch_round<true, true, 1, false>, launch_round<true, true, S, false>},
+       {launch_round<true, false, 1, true>, launch_round<true, false, S, true>}}};
+  const Launch one = kRound[profile][alias ? 1 : mixed ? 2 : 0][split];
   for (uint32_t r = 0; r < rounds; ++r)
-    classic(d_clouds, nclouds, grid, sparse, passes, hot, dense, whole, st);
+    one(d_clouds, nclouds, grid, sparse, passes, list_cap, first + r, st);
   return hipGetLastError();
 }
 

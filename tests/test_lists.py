@@ -1,0 +1,58 @@
+"""The rounds engine's lists and final order at their edges (nsfps_runs.hip):
+both list lengths, nodes with more samples a round than fit the LDS at once,
+ties, chains of conflicts, nearly all points sampled, shared buckets, split
+update passes and batched clouds, against the oracle.  Indices: no tolerance."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+UNIT = (-1.0, 1.0, -1.0, 1.0, -1.0, 1.0)
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from ns_fps_amd.capi import Lib
+    L = Lib()
+    if L.device_count() < 1:
+        pytest.fail("no HIP device visible: GPU tests need an MI355X")
+    return L
+
+
+def cloud(kind, n):
+    rs = np.random.RandomState(n % 1000003)
+    if kind == "cube":
+        P = rs.uniform(-1, 1, (n, 3))
+    elif kind == "lattice":  # ties in every distance
+        side = int(np.ceil(n ** (1 / 3)))
+        P = np.stack(np.meshgrid(*[np.arange(side)] * 3), -1).reshape(-1, 3) * (2 / side) - 1
+        P = P[rs.permutation(len(P))[:n]]
+    elif kind == "dups":
+        P = np.repeat(rs.uniform(-1, 1, ((n + 7) // 8, 3)), 8, 0)[rs.permutation(n)]
+    elif kind == "plane":
+        P = rs.uniform(-1, 1, (n, 3)) * [1, 1, 0]
+    else:  # rings of halving radius: each sample's rivals are its neighbours
+        r = 2.0 ** -(np.arange(n) % 40)
+        a = rs.uniform(0, 2 * np.pi, n)
+        P = np.stack([r * np.cos(a), r * np.sin(a), r * rs.uniform(-0.1, 0.1, n)], 1)
+    return np.ascontiguousarray(P, np.float32)
+
+
+@pytest.mark.parametrize("kind,n,m,blocks", [
+    ("cube", 2, 1, (4, 4, 4)), ("cube", 70, 69, (4, 4, 4)), ("cube", 1025, 1024, (8, 8, 8)),
+    ("cube", 32768, 3000, (16, 16, 16)), ("cube", 32769, 3000, (16, 16, 16)),
+    ("cube", 40000, 39999, (1, 1, 1)), ("cube", 60000, 30000, (2, 2, 2)),
+    ("cube", 50000, 9000, (17, 17, 17)), ("cube", 90000, 20000, (30, 30, 30)),
+    ("lattice", 64000, 9000, (16, 16, 16)), ("lattice", 40000, 39990, (8, 8, 8)),
+    ("dups", 48000, 20000, (16, 16, 16)), ("plane", 70000, 9000, (32, 32, 2)),
+    ("rings", 40000, 9000, (32, 32, 4)), ("rings", 3000, 2990, (4, 4, 4)),
+])
+def test_lists_match_the_oracle(lib, oracle, monkeypatch, kind, n, m, blocks):
+    P = cloud(kind, n)
+    monkeypatch.setenv("NSFPS_SMALL", "0")
+    want = oracle.fps(P, m, (*UNIT, *blocks))
+    assert np.array_equal(lib.fps(P, m, (*UNIT, *blocks)), want)
+    if n <= 1025:
+        got = lib.fps_batched(np.stack([P] * 9), m, [(*UNIT, *blocks)] * 9)
+        assert all(np.array_equal(g, want) for g in got)
