@@ -33,7 +33,7 @@ constexpr uint32_t kListCap = 4096;
 // before, at least kListMin and at most the cloud's list_cap entries: the
 // first rounds of a cloud settle few, however long their lists.
 constexpr uint32_t kListMin = 1024;
-constexpr uint32_t kListGrow = 4;
+constexpr uint32_t kListGrow = 8;
 // list_cap of small clouds (host's kShortListPoints)
 constexpr uint32_t kListShort = 512;
 // rounds in the log that orders the samples, for up to 131,072 samples (more

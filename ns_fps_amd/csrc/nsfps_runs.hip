@@ -32,11 +32,11 @@
 // What bounds it: the rounds' launches (three of 5 to 17 us each; the points
 // that a round touches are read from cache) times the rounds.  They are few:
 // samples settle as soon as the few larger keys near them have, so a round of
-// 4,096 listed points settles some 800 to 1,300.  Per call on one MI355X, device-resident,
+// 4,096 listed points settles some 900 to 2,200.  Per call on one MI355X, device-resident,
 // against lists sampled one after another by one workgroup: 120,000-point
-// scan -> 16,384 (55 rounds) 3.65 -> 1.38 ms, 1M-point cube -> 65,536 (82)
-// 7.02 -> 2.56, the same on 30^3 cells 10.6 -> 3.95, 8M clustered points ->
-// 524,288 (292) 59 -> 17.9, 1M -> 524,288 (236) 38 -> 7.2.  Clouds in few
+// scan -> 16,384 (50 rounds) 3.65 -> 1.30 ms, 1M-point cube -> 65,536 (75)
+// 7.02 -> 2.56, the same on 30^3 cells 10.6 -> 3.83, 8M clustered points ->
+// 524,288 (243) 59 -> 16.0, 1M -> 524,288 (236) 38 -> 7.2.  Clouds in few
 // samples gain least: 17,000 -> 64 0.34 -> 0.37 ms, 14 rounds for 7.
 //
 // The cube test compares cell coordinates.  Where cells share buckets (block
@@ -793,17 +793,21 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
       // the first rounds start from windows over the whole key range and are
       // forced as a rule; later forced rounds ask for refinement passes
       rs.forced += forced && rs.rounds >= 2 ? 1u : 0u;
-      // next round: bins of 1/1024 to 1/2048 of this round's key span, over
-      // 1.75 spans (the next threshold lies about half a span below this one;
-      // every leaf with a key in the window is read); where the list came out
-      // short, over two to four times the whole window down to the threshold
+      // next round: bins of 1/512 to 1/1024 of this round's key span, over 3
+      // spans (a window that ends above the next threshold leaves the list
+      // short; most leaves with a key in it are read anyway, for a sample
+      // reaches them); where the list came out short, over four to eight
+      // times the whole window down to the threshold.  8M clustered points:
+      // 1.75 spans 292 rounds, 17.8 ms; 2: 261, 16.5; 3: 247, 16.1; 4: 246,
+      // 16.2 (1M cube 2.57, 2.55, 2.62, 2.68; with kListGrow 8 for 4, 3 spans
+      // 2.56 and 16.0).
       const bool grow = 2 * s.total < rs.cap;
       const uint64_t span = (grow ? rs.kref0 : ktop) - bkey + 1;
       uint32_t nx = bit_length(span);
-      nx = nx > 11u ? nx - 11u : 0u;
+      nx = nx > 10u ? nx - 10u : 0u;
       nx = nx < kMaxShift ? nx : kMaxShift;
       rs.s0_next = nx;
-      rs.nb_next = grow ? kHistBins : min((uint32_t)(span >> nx) * 7 / 4 + 1, kHistBins);
+      rs.nb_next = grow ? kHistBins : min((uint32_t)(span >> nx) * 3 + 1, kHistBins);
       if (fin) {
         *gptr(c.iter) = min(T, m);
         *gptr(c.done) = 1;
