@@ -140,7 +140,7 @@ def roofline_of(wname, sample_ms, engine):
     return {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 6),
             "traffic": profile_traffic("sampling", wname),
-            "kernel": "sampling pass (k_update+k_refine+k_gather+k_run rounds)"
+            "kernel": "sampling pass (k_update+k_refine+k_gather+k_accept rounds)"
             if engine == "runs" else "sampling pass (k_wide_update+k_late_loop)",
             "alg_bytes_per_launch": alg, "kernel_ms": round(sample_ms, 3)}
 

@@ -42,25 +42,13 @@ SOURCES = ("nsfps_build.hip", "nsfps_sample.hip", "nsfps_runs.hip", "nsfps_small
 # forward an option with an argument to the device pass alone
 # (-Xarch_device refuses it), so that host-pass warning is filtered from the
 # build output and the device assembly is checked instead (check_no_packed_fp32).
-# The backend's atomic optimizer is off: by default it turns an atomic whose
-# address is the same in every lane into a loop over the active lanes (a
-# read-lane and a scalar step each) ahead of one atomic, and in these kernels
-# such atomics have few active lanes on the run kernel's critical path (the
-# largest key left unaccepted, the lowered copies' masks and bounds).  With
-# one LDS atomic per lane instead, per call on one MI355X, bit-exact: 1M-point
-# uniform cube 7.20-7.22 -> 6.99-7.01 ms, quickstart 0.71 -> 0.65-0.66,
-# LiDAR scan 3.91 -> 3.77-3.80, batched clouds 2.05 -> 1.93-1.98, clustered
-# cloud 60.2-60.3 -> 59.5.  Its DPP form (a reduction across lanes in place of
-# the loop) measured in between: uniform cube 7.16-7.23, quickstart 0.67-0.69.
-# The machine scheduler favours instruction-level parallelism (max-ilp): the
-# run kernel is latency-bound with two waves per SIMD.  Per call, two runs on
-# each of two boxes, bit-exact, against the default strategy: uniform cube
-# 7.01-7.02 -> 6.96-7.00 ms, LiDAR scan 3.77-3.79 -> 3.67-3.69, batched
-# clouds 1.99-2.00 -> 1.89-1.94, clustered cloud 59.5-59.8 -> 58.3-58.6,
-# quickstart 0.66-0.68 -> 0.65-0.66.  The others measured: max-memory-clause
-# slower everywhere (uniform cube 7.04-7.05), iterative-ilp and
-# iterative-maxocc in between (uniform cube 6.95-6.97 and 7.00-7.01,
-# clustered 58.7 and 58.9-59.0).
+# The backend's atomic optimizer is off (by default it turns an atomic whose
+# address is the same in every lane into a loop over the active lanes, a
+# read-lane and a scalar step each, ahead of one atomic) and the machine
+# scheduler favours instruction-level parallelism.  Per call on one MI355X,
+# with both against the default optimizer and the default scheduler, two runs
+# each: 1M-point uniform cube 2.57-2.58, 2.58, 2.57-2.59 ms; 64 clouds of
+# 20,000 points 2.07-2.12, 2.15, 2.12-2.17; clustered cloud 17.8, 17.9, 17.8.
 DEVICE_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-ffp-contract=off", "-fno-fast-math",
