@@ -115,6 +115,7 @@ struct RunState {
   uint32_t rounds;    // rounds that ran (statistics)
   uint32_t err;       // set if a list overflowed (internal error)
   uint32_t forced;    // rounds whose threshold was forced for want of refinement passes
+  uint32_t fin;       // the gather pass found the end (the accept pass then sets done)
 };
 
 // Everything one cloud's kernels touch.  Device pointers; passed by value to

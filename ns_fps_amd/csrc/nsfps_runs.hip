@@ -710,8 +710,13 @@ __device__ __forceinline__ uint32_t bit_length(uint64_t v) { return v ? 64u - __
 // maximum key itself: a run of one sample.  Few workgroups, each striding over
 // the level-1 nodes; most nodes hold no key above the threshold.  PROF: counts
 // the hot leaves whose points it reads and those points.  Its first workgroup
-// also ends the sampling: when m samples have keys above every key left, or
-// only points at distance 0 are left (src/yuezu_fps.cpp:705-706).
+// also finds the sampling's end: when m samples have keys above every key
+// left, or only points at distance 0 are left (src/yuezu_fps.cpp:705-706).
+// It leaves that in rs.fin, which no workgroup of this launch tests; the
+// accept pass tests fin and writes done, which none of its own tests.  With
+// one word for both, waves of one workgroup could read it before and after
+// the write, and those that went on would scan LDS words that the others
+// never wrote.
 template <bool PROF>
 __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restrict__ clouds,
                                                          uint32_t passes, uint32_t par) {
@@ -810,7 +815,7 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
       rs.nb_next = grow ? kHistBins : min((uint32_t)(span >> nx) * 3 + 1, kHistBins);
       if (fin) {
         *gptr(c.iter) = min(T, m);
-        *gptr(c.done) = 1;
+        rs.fin = 1;
       }
     }
     if (fin) return;
@@ -984,7 +989,7 @@ __global__ __launch_bounds__(kAcceptThreads) void k_accept(const CloudDev *__res
   const bool cubes = blockIdx.x < ncube;
   const uint32_t w = uniform(cubes ? 0u : (blockIdx.x - ncube) * kAcceptWaves + (tid >> 6));
   const uint32_t x0 = (w % xgs) * kAcceptX + lane, q0 = (w / xgs) * kAcceptChunk;
-  const uint32_t nl = min(rs.nl[par], kListCap), done = *gptr(c.done);
+  const uint32_t nl = min(rs.nl[par], kListCap), fin = rs.fin;
   // entries past the list are stale and unused
   float4 X[2];
   uint32_t XR[2];
@@ -993,7 +998,10 @@ __global__ __launch_bounds__(kAcceptThreads) void k_accept(const CloudDev *__res
     X[t] = gptr(c.list_p)[x0 + 64 * t];
     XR[t] = gptr(c.list_r)[x0 + 64 * t].x;
   }
-  if (done) return;
+  if (fin) {  // found by the gather pass, of this round or an earlier one
+    if (blockIdx.x == 0 && tid == 0) *gptr(c.done) = 1;
+    return;
+  }
   // the histograms this round's selection read are cleared for the next
   // round's update pass
   NSFPS_GLOBAL uint4 *const hz = reinterpret_cast<NSFPS_GLOBAL uint4 *>(hist_set(c));
@@ -1236,7 +1244,7 @@ __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__re
     gptr(c.list_c)[0] = make_uint2(
         0u, pack11(pack_cell(c.r.blocks[0] - 1, c.r.blocks[1] - 1, c.r.blocks[2] - 1)) | kGuards);
     *gptr(c.iter) = 1;
-    *gptr(c.done) = c.m <= 1 ? 1u : 0u;
+    *gptr(c.done) = rs.fin = c.m <= 1 ? 1u : 0u;
   }
   for (uint32_t j = tid; j < kHists * kHistBins; j += kPassThreads) gptr(c.hist)[j] = 0;
 }
