@@ -94,7 +94,8 @@ enum : uint32_t {
 // update pass a workgroup reads its siblings' parts while they may write
 // them: the parts are read and written as relaxed agent-scope atomics (each
 // 64-bit word whole, no order needed: either value of a part bounds its
-// quarter's points, distances only falling).
+// quarter's points, distances only falling).  There one wave reads the key
+// for its whole workgroup, which leaves ahead of a barrier by it.
 __device__ __forceinline__ uint64_t node_key(const CloudDev &c, uint32_t g) {
   NSFPS_GLOBAL uint64_t *const pp = gptr(c.l1_part) + (size_t)g * kUpdateSplit;
   uint64_t k = gptr(c.l1_key)[g];
@@ -329,6 +330,7 @@ __global__ __launch_bounds__(kPassThreads) __attribute__((amdgpu_num_sgpr(60), a
   __shared__ uint2 s_pc[kPickLds];  // the picks' cube corners: pack11(lo), pack11(hi) | kGuards
   __shared__ uint16_t s_more[kListCap - kPickLds];  // the node's picks past kPickLds
   __shared__ uint64_t s_lk[kFan];
+  __shared__ uint64_t s_nkey;  // SPLIT: the node's key as wave 0 read it
   __shared__ uint32_t s_np;
   __shared__ uint32_t s_ct[4];  // PROF: leaves and points read by the workgroup, and of them touched
   __shared__ uint32_t s_wt[PROF ? 3 * kPassWaves : 1];  // PROF: per-wave clocks
@@ -365,8 +367,11 @@ __global__ __launch_bounds__(kPassThreads) __attribute__((amdgpu_num_sgpr(60), a
   const uint32_t S = rs.s0;
   const uint32_t gn = g < c.nl1 ? g : 0u;  // read unconditionally, used only if g < nl1
   // split: a sibling workgroup may have written its part already; either value
-  // bounds this workgroup's points (distances only fall)
-  const uint64_t nkey = SPLIT == 1 ? gptr(c.l1_key)[gn] : node_key(c, gn);
+  // bounds this workgroup's points (distances only fall), but every wave has
+  // to take the same one (s_nkey)
+  uint64_t nkey = 0;
+  if (SPLIT == 1) nkey = gptr(c.l1_key)[gn];
+  else if (wave == 0) nkey = node_key(c, gn);
   uint32_t clo, chi;
   uint64_t uta = 0, utb = 0, utc = 0, utd = 0;
   // the node's box of points (x > its hi x: no points)
@@ -399,8 +404,10 @@ __global__ __launch_bounds__(kPassThreads) __attribute__((amdgpu_num_sgpr(60), a
   const uint32_t clo11 = pack11(clo), chi11g = pack11(chi) | kGuards;
   for (uint32_t j = tid; j < kHistBins; j += kPassThreads) s_hist[j] = 0;
   if (tid == 0) s_np = 0;
+  if (SPLIT > 1 && tid == 0) s_nkey = nkey;
   if (PROF && tid < 4) s_ct[tid] = 0;
   __syncthreads();
+  if (SPLIT > 1) nkey = uni(s_nkey);
   if (PROF) utb = __builtin_amdgcn_s_memrealtime();
   // every thread's list entries are read together (entries past the list are
   // stale and unused)

@@ -43,3 +43,19 @@ def test_no_launch_writes_a_word_that_it_tests(word):
     testers = [k for k, b in found.items() if re.search(word + r"(?!\s*=[^=])", b)]
     assert writers and testers
     assert not set(writers) & set(testers), (writers, testers)
+
+
+def test_one_wave_reads_the_node_key_that_siblings_write():
+    """The split update pass returns on the node's key ahead of a barrier
+    while sibling workgroups write parts of it: wave 0 alone reads it there,
+    and every wave takes its value from LDS after a barrier."""
+    body = bodies()["k_update"]
+    reads = [m.start() for m in re.finditer(r"node_key\(", body)]
+    assert len(reads) == 1
+    assert re.search(r"if \(wave == 0\) nkey = node_key\(c, gn\);", body)
+    publish = re.search(r"tid == 0\) s_nkey = nkey;.*?__syncthreads\(\);\s*if \(SPLIT > 1\) nkey = uni\(s_nkey\);",
+                        body, re.S)
+    assert publish and reads[0] < publish.start()
+    # nothing looks at the value before it is shared, but the wait for the reads
+    between = re.sub(r"pin_sgpr\([^;]*;", "", body[reads[0]:publish.start()])
+    assert between.count("nkey") == 0
