@@ -218,7 +218,7 @@ struct SmallDev {
   uint16_t *rows;    // input row of each rank
   SmallStatus *st;
   uint32_t bbox;     // 1: the range is compute_bbox of the points with r's block counts
-  uint32_t pad;
+  uint32_t any_bad;  // devs[0]: some cloud of the call is bad (0 when the sort starts)
   RangeDev r;
 };
 

@@ -165,7 +165,7 @@ constexpr uint32_t kSpatialBits = 16;  // two passes of the sort
 // registers until they are stored in place (read again in order instead, three
 // scattered words a point, the kernel took 70 us for 16,384 points).
 template <uint32_t R, bool ONE>
-__device__ __forceinline__ void sort_cloud(const SmallDev &c, SmallDev *dst) {
+__device__ __forceinline__ void sort_cloud(const SmallDev &c, SmallDev *dst, SmallDev *first_dev) {
   __shared__ uint32_t s_el[kSmThreads * R];
   __shared__ uint16_t s_rank[kSmThreads * R], s_pos[kSmThreads * R];  // by row
   __shared__ uint32_t s_cnt[kSmWaves][256];
@@ -244,6 +244,9 @@ __device__ __forceinline__ void sort_cloud(const SmallDev &c, SmallDev *dst) {
       dst->pts = c.pts;
       dst->rows = c.rows;
       dst->st = c.st;
+      dst->any_bad = s_bad;
+    } else if (s_bad) {
+      atomicOr(&first_dev->any_bad, s_bad);
     }
     gptr(c.st)->bad = s_bad;
     gptr(c.st)->len = 0;
@@ -346,11 +349,11 @@ __device__ __forceinline__ void sort_cloud(const SmallDev &c, SmallDev *dst) {
 // devs[0] for the sampling); otherwise devs[blockIdx.x].
 template <uint32_t R>
 __global__ __launch_bounds__(kSmThreads) void k_small_sort1(SmallDev one, SmallDev *devs) {
-  sort_cloud<R, true>(one, devs);
+  sort_cloud<R, true>(one, devs, devs);
 }
 template <uint32_t R>
 __global__ __launch_bounds__(kSmThreads) void k_small_sort(SmallDev *devs) {
-  sort_cloud<R, false>(devs[blockIdx.x], devs + blockIdx.x);
+  sort_cloud<R, false>(devs[blockIdx.x], devs + blockIdx.x, devs);
 }
 
 // ----------------------------------------------------------------- sample
@@ -450,7 +453,8 @@ __global__ __launch_bounds__(kSmThreads) void k_small_sample(const SmallDev *__r
   const uint32_t n = c.n, m = m_over ? m_over : c.m;
   NSFPS_GLOBAL SmallStatus &st = *gptr(c.st);
   const NSFPS_GLOBAL float4 *const pts = gptr(c.pts);
-  if (st.bad) return;  // uniform
+  // a call with a cloud that it refuses writes no row of any (uniform)
+  if (gptr(devs)->any_bad) return;
   const uint32_t pos0 = st.pos0, rank0 = st.rank0;
   const uint32_t lpw = ((n + 63u) / 64u + kSmWaves - 1) / kSmWaves;  // leaves per wave, <= S
   if (tid < sizeof(RangeDev) / 4)

@@ -109,6 +109,34 @@ def test_small_clouds_report_what_the_general_engine_reports(lib, monkeypatch):
     assert all(len(v) == 1 for v in said.values()), said
 
 
+@pytest.mark.parametrize("small", ["0", "1"])
+@pytest.mark.parametrize("what", ["nan", "flat"])
+@pytest.mark.parametrize("at", [0, 5, 7])
+def test_a_batch_with_a_refused_cloud_writes_no_row(lib, hip, oracle, monkeypatch, small, what, at):
+    from ns_fps_amd.capi import NsfpsError
+    P = np.stack([cloud("cube", 300 + b)[:300] for b in range(8)])
+    good = P.copy()
+    if what == "nan":
+        P[at, 123, 2] = np.nan
+    else:
+        P[at] = 1e9
+    monkeypatch.setenv("NSFPS_SMALL", small)
+    before = np.arange(8 * 60, dtype=np.int32)
+    d_xyz, d_out, d_good = hip.upload(P), hip.upload(before), hip.upload(good)
+    try:
+        with pytest.raises(NsfpsError):
+            lib.fps_batched_device(d_xyz, 8, 300, 60, d_out)
+        assert np.array_equal(hip.download(d_out, 8 * 60, np.int32), before)
+        # and the call after it is sampled
+        lib.fps_batched_device(d_good, 8, 300, 60, d_out)
+        rows = hip.download(d_out, 8 * 60, np.int32).reshape(8, 60)
+        for b in range(8):
+            assert np.array_equal(rows[b], oracle.fps(good[b], 60, None)), b
+    finally:
+        for d in (d_xyz, d_out, d_good):
+            hip.free(d)
+
+
 @pytest.mark.parametrize("kind", ["launch", "copy", "sync", "any"])
 def test_every_operation_of_a_small_call_fails_cleanly(lib, oracle, monkeypatch, kind):
     from ns_fps_amd.capi import NsfpsError
