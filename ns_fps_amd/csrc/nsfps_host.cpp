@@ -1186,7 +1186,7 @@ nsfps_status finish_cloud(CloudPlan &p, const uint32_t *lorig, const uint32_t *p
 }
 
 // bd: host copies of the many-cloud build parameters, sources of
-// asynchronous copies; the caller keeps them until the stream is synchronised.
+// asynchronous copies (CallLayout's h_bd).
 nsfps_status build_clouds(std::vector<CloudPlan> &plans, const CallBuffers &cb, const Scratch &s,
                           std::vector<BuildDev> &bd, hipStream_t st) {
   const size_t nc = plans.size();
@@ -1604,13 +1604,18 @@ struct Ws {
 
 // Where one call's buffers live: per cloud (layout_cloud), for the call
 // (layout_call), the sorts' scratch, and the per-cloud descriptors and status
-// words the sampling kernels read.
+// words the sampling kernels read.  With the host sources of the call's
+// asynchronous copies: it is destroyed only after the call's stream has been
+// waited for, whichever way the call ends.
 struct CallLayout {
   CallBuffers cb{};
   Scratch sc{};
   CloudDev *d_clouds = nullptr;
   CloudStatus *d_status = nullptr;
   uint32_t nsort = 0, tmax = 0;
+  std::vector<BuildDev> h_bd;
+  std::vector<CloudDev> h_devs;
+  std::vector<SmallDev> h_small;
 };
 
 // Lays the call out over bp (a null base measures it).
@@ -1702,7 +1707,7 @@ void layout_small(Bump &bp, const std::vector<CloudPlan> &plans, SmallLayout &L)
 }
 
 // The sort of every cloud, enqueued on st; devs: the clouds' parameters, a
-// source of an asynchronous copy that the caller keeps until st is waited for.
+// source of an asynchronous copy (CallLayout's h_small).
 nsfps_status small_sort(const std::vector<CloudPlan> &plans, const SmallLayout &L,
                         std::vector<SmallDev> &devs, hipStream_t st) {
   const size_t nc = plans.size(), n = plans[0].n;
@@ -1775,7 +1780,7 @@ void small_stats(const std::vector<CloudPlan> &plans, const std::vector<SmallSta
 
 // One call of small clouds over workspace ws, as run_clouds_once.
 nsfps_status run_small(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_host, int32_t *h_out,
-                       uint64_t out_stride, uint64_t *out_lens) {
+                       uint64_t out_stride, uint64_t *out_lens, CallLayout &CL) {
   auto t0 = std::chrono::steady_clock::now();
   const size_t nc = plans.size();
   SmallLayout L;
@@ -1800,9 +1805,8 @@ nsfps_status run_small(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_host, 
   layout_small(bp, plans, L);
   hipStream_t st = ws.st;
   ws.st_used = true;
-  std::vector<SmallDev> devs;
   if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[0], st));
-  nsfps_status rc = small_sort(plans, L, devs, st);
+  nsfps_status rc = small_sort(plans, L, CL.h_small, st);
   if (rc) return rc;
   if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[1], st));
   HIP_TRY(launch_small_sample(L.devs, (uint32_t)nc, plans[0].n, 0, nullptr, st));
@@ -1837,11 +1841,12 @@ nsfps_status run_small(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_host, 
 // the first iterations of a single cloud on the tree engine, then its loop;
 // or the rounds.
 // fin: the runs engine's final statuses (left empty by the tree engine)
-nsfps_status sample_clouds(std::vector<CloudPlan> &plans, const CallLayout &L, const Ws &ws,
+nsfps_status sample_clouds(std::vector<CloudPlan> &plans, CallLayout &L, const Ws &ws,
                            bool runs, uint64_t *rounds, uint64_t *wide_total,
                            PassShape *pass, std::vector<CloudStatus> &fin) {
   hipStream_t st = ws.st;
-  std::vector<CloudDev> devs;
+  std::vector<CloudDev> &devs = L.h_devs;
+  devs.clear();
   uint32_t lds_bytes = 0;
   for (auto &p : plans) {
     devs.push_back(p.dev);
@@ -1961,7 +1966,7 @@ nsfps_status run_clouds(std::vector<CloudPlan> &plans, Ws ws, bool out_on_host, 
                         uint64_t out_stride, uint64_t *out_lens) {
   CallLayout L;
   const nsfps_status rc =
-      small_wanted(plans) ? run_small(plans, ws, out_on_host, h_out, out_stride, out_lens)
+      small_wanted(plans) ? run_small(plans, ws, out_on_host, h_out, out_stride, out_lens, L)
                           : run_clouds_once(plans, ws, out_on_host, h_out, out_stride, out_lens, L);
   if (rc && ws.st_used) {
     (void)hipStreamSynchronize(ws.st);
@@ -2000,8 +2005,7 @@ nsfps_status run_clouds_once(std::vector<CloudPlan> &plans, Ws &ws, bool out_on_
   hipStream_t st = ws.st;
   ws.st_used = true;
   if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[0], st));
-  std::vector<BuildDev> bd_host;  // lives until the stream is synchronised below
-  nsfps_status rc = build_clouds(plans, L.cb, L.sc, bd_host, st);
+  nsfps_status rc = build_clouds(plans, L.cb, L.sc, L.h_bd, st);
   if (rc) return rc;
   if (ws.ev) HIP_TRY(hipEventRecord(ws.ev[1], st));
   uint64_t rounds = 0, wide_total = 0;
@@ -2551,9 +2555,8 @@ nsfps_status nsfps_plan_create(const float *xyz, uint64_t n, const nsfps_range *
       for (auto &ev : P.ev) HIP_TRY(hipEventCreate(&ev));
       Bump bp(P.mem);
       layout_small(bp, P.plans, P.SL);
-      std::vector<SmallDev> devs;
       std::vector<SmallStatus> fin(1);
-      rc = small_sort(P.plans, P.SL, devs, nullptr);
+      rc = small_sort(P.plans, P.SL, P.L.h_small, nullptr);
       if (!rc) rc = readback(fin.data(), P.SL.st, sizeof(SmallStatus), nullptr);
       if (rc) {
         (void)hipStreamSynchronize(nullptr);  // nothing enqueued outlives the plan's memory
@@ -2591,16 +2594,24 @@ nsfps_status nsfps_plan_create(const float *xyz, uint64_t n, const nsfps_range *
     P.lp_0 = bp.take<float4>(pb.leaves_ub);
     P.runs = choose_runs(P.plans);
     hipStream_t st = nullptr;
-    std::vector<BuildDev> bd_host;
-    rc = build_clouds(P.plans, P.L.cb, P.L.sc, bd_host, st);
-    if (rc) return rc;
-    const CloudDev &c = P.plans[0].dev;
-    HIP_TRY(hipMemcpyAsync(P.p4_0, c.P4, (size_t)c.nslots * sizeof(float4),
-                           hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(P.lk_0, c.leaf_key, (size_t)c.nleaves * 8, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(P.lp_0, c.leaf_pos, (size_t)c.nleaves * sizeof(float4),
-                           hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    const auto body = [&]() -> nsfps_status {
+      const nsfps_status built = build_clouds(P.plans, P.L.cb, P.L.sc, P.L.h_bd, st);
+      if (built) return built;
+      const CloudDev &c = P.plans[0].dev;
+      HIP_TRY(hipMemcpyAsync(P.p4_0, c.P4, (size_t)c.nslots * sizeof(float4),
+                             hipMemcpyDeviceToDevice, st));
+      HIP_TRY(hipMemcpyAsync(P.lk_0, c.leaf_key, (size_t)c.nleaves * 8, hipMemcpyDeviceToDevice,
+                             st));
+      HIP_TRY(hipMemcpyAsync(P.lp_0, c.leaf_pos, (size_t)c.nleaves * sizeof(float4),
+                             hipMemcpyDeviceToDevice, st));
+      HIP_TRY(hipStreamSynchronize(st));
+      return NSFPS_OK;
+    };
+    rc = body();
+    if (rc) {
+      (void)hipStreamSynchronize(st);  // nothing enqueued outlives the plan's memory
+      return rc;
+    }
     // the input is not read again
     P.plans[0].h_xyz = nullptr;
     P.plans[0].d_xyz_in = nullptr;
