@@ -108,9 +108,9 @@ __device__ __forceinline__ uint64_t node_key(const CloudDev &c, uint32_t g) {
 }
 
 // Histogram window of a selection pass: nb bins of 2^S keys each, bin 0 ending
-// at kref (S = kMaxShift: all keys).  Lowest key inside the window:
+// at kref.  Lowest key inside the window (kHistBins bins at kMaxShift hold
+// every key: the product wraps to 0, and w to the largest key):
 __device__ __forceinline__ uint64_t window_lo(uint64_t kref, uint32_t S, uint32_t nb = kHistBins) {
-  if (S >= kMaxShift) return 0;
   const uint64_t w = ((uint64_t)nb << S) - 1;
   return kref >= w ? kref - w : 0;
 }

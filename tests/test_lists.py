@@ -56,3 +56,19 @@ def test_lists_match_the_oracle(lib, oracle, monkeypatch, kind, n, m, blocks):
     if n <= 1025:
         got = lib.fps_batched(np.stack([P] * 9), m, [(*UNIT, *blocks)] * 9)
         assert all(np.array_equal(g, want) for g in got)
+
+
+def test_a_window_of_coarse_bins_that_ends_above_the_last_keys(lib, oracle):
+    """Squared distances over more than 60 octaves give the second round's
+    window bins of 2^52 keys; it ends above the keys of the points at distance
+    0, which are far more than a list holds and are not to be listed with the
+    1,015 inside the window."""
+    rs = np.random.RandomState(5)
+    d2 = np.concatenate([[2.0 ** 69], rs.uniform(20.5, 38.0, 1000), rs.uniform(18.1, 19.9, 25)])
+    u = rs.randn(len(d2), 3)
+    far = u / np.linalg.norm(u, axis=1, keepdims=True) * np.sqrt(d2)[:, None]
+    far[0] = [2.0 ** 34.5, 0, 0]
+    P = np.zeros((40000, 3), np.float32)
+    P[1 + rs.permutation(39999)[:len(far)]] = far
+    rng = (-1e11, 1e11, -1e11, 1e11, -1e11, 1e11, 4, 4, 4)
+    assert np.array_equal(lib.fps(P, 1500, rng), oracle.fps(P, 1500, rng))
