@@ -798,14 +798,25 @@ uint64_t padded_slot_limit(uint32_t n) { return std::max<uint64_t>(4ull * n, 655
 // Clouds of at most this many points keep their lists at kListShort entries:
 // longer ones hardly save rounds there (a CPU model: 30 rounds of the
 // 10,000-point quickstart at 1,024 as at 4,096 entries, but 57 against 41 of
-// a 120,000-point scan) and the pairs of many clouds' lists add up: 64 clouds
-// of 20,000 points 2.6 ms per call at 1,024 entries (39 rounds), 2.06 at 512
-// (42), 2.3 at 256 (56).
+// a 120,000-point scan).  17,000 Gaussian points -> 1,024: 626 us per call at
+// 512 entries, 642 at 1,024, 662 at 4,096.
 constexpr uint32_t kShortListPoints = 32768;
+
+// The longest list of a cloud.  All pairs of every cloud's list are tested, so
+// the lists of many clouds are shorter: as many pairs in all as one list of
+// kListCap has.  Per call at one and four times that: 16 clouds of 65,536
+// points -> 4,096 (lists of 1,024 and 2,048) 1.61 and 1.86 ms, 64 (512 and
+// 1,024) 4.15 and 4.35; with lists of kListCap for all of them 2.85 and 9.97.
+// Four clouds -> 16,384 (2,048 and 4,096) 1.51 and 1.77.
+uint32_t list_cap_for(uint32_t n, size_t nclouds) {
+  uint32_t cap = n <= kShortListPoints ? kListShort : kListCap;
+  while (cap > kListShort && (uint64_t)cap * cap * nclouds > (uint64_t)kListCap * kListCap) cap /= 2;
+  return cap;
+}
 
 // Lays out the persistent buffers of one cloud (upper bounds: the padded /
 // dense decision is made on the device data during the build).
-void layout_cloud(Bump &bp, CloudPlan &p) {
+void layout_cloud(Bump &bp, CloudPlan &p, size_t nclouds) {
   const uint32_t n = p.n, T = p.rng.dev.T;
   uint64_t slots = std::max<uint64_t>(n, padded_slot_limit(n));
   uint64_t leaves = std::max<uint64_t>(n / kLeaf + 1 + std::min<uint32_t>(T, n), slots / kLeaf);
@@ -842,7 +853,7 @@ void layout_cloud(Bump &bp, CloudPlan &p) {
   c.list_r = bp.take<uint2>(kListCap);
   c.list_f = bp.take<uint32_t>(kListCap);
   c.list_c = bp.take<uint2>(kListCap);
-  c.list_cap = n <= kShortListPoints ? kListShort : kListCap;
+  c.list_cap = list_cap_for(n, nclouds);
   // every round settles a sample, and usually many; with a full log the later
   // rounds share its last entry.  A plan learns m later: at most n.
   const uint32_t mmax = p.m ? p.m : n;
@@ -1620,7 +1631,7 @@ struct CallLayout {
 
 // Lays the call out over bp (a null base measures it).
 void layout_all(Bump &bp, std::vector<CloudPlan> &plans, CallLayout &L) {
-  for (auto &p : plans) layout_cloud(bp, p);
+  for (auto &p : plans) layout_cloud(bp, p, plans.size());
   layout_call(bp, plans, L.cb);
   layout_scratch(bp, L.nsort, L.tmax, L.sc);
   L.d_clouds = bp.take<CloudDev>(plans.size());

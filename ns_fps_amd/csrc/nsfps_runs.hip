@@ -1303,7 +1303,8 @@ hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t ma
                          bool split, bool mixed, uint32_t list_cap, uint32_t first,
                          hipStream_t st) {
   if (alias && mixed) return hipErrorInvalidValue;  // leaves of several buckets: one cell each
-  if (list_cap != kListShort && list_cap != kListCap) return hipErrorInvalidValue;
+  if (list_cap < kListShort || list_cap > kListCap || (list_cap & (list_cap - 1)))
+    return hipErrorInvalidValue;
   const dim3 grid(max_nl1, nclouds);
   const dim3 sparse(max_nl1 < kSparseGroups ? max_nl1 : kSparseGroups, nclouds);
   using Launch = void (*)(const CloudDev *, uint32_t, dim3, dim3, uint32_t, uint32_t, uint32_t,

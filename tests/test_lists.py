@@ -72,3 +72,15 @@ def test_a_window_of_coarse_bins_that_ends_above_the_last_keys(lib, oracle):
     P[1 + rs.permutation(39999)[:len(far)]] = far
     rng = (-1e11, 1e11, -1e11, 1e11, -1e11, 1e11, 4, 4, 4)
     assert np.array_equal(lib.fps(P, 1500, rng), oracle.fps(P, 1500, rng))
+
+
+@pytest.mark.parametrize("batch,n", [(2, 33000), (4, 33000), (16, 33000), (64, 33000), (7, 20000)])
+def test_shorter_lists_of_many_clouds_match_the_oracle(lib, oracle, batch, n):
+    kinds = ["cube", "lattice", "dups", "rings"]
+    P = [cloud(kinds[b % 4], n) for b in range(4)]
+    want = [oracle.fps(p, 700, (*UNIT, 16, 16, 16)) for p in P]
+    for m in (40, 700):
+        got = lib.fps_batched(np.stack([P[b % 4] for b in range(batch)]), m,
+                              [(*UNIT, 16, 16, 16)] * batch)
+        for b in range(batch):
+            assert np.array_equal(got[b], want[b % 4][:m]), (b, m)
