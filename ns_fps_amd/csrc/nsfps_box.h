@@ -113,4 +113,30 @@ __device__ __forceinline__ uint2 sample_cube(const RangeDev &r, uint32_t c11, fl
   return make_uint2(pack11(lo_c), pack11(hi_c) | kGuards);
 }
 
+// The bits of v at the set positions of mask, lowest first.
+__device__ __forceinline__ uint32_t deposit_bits(uint32_t v, uint32_t mask) {
+  uint32_t r = 0, k = 0;
+  for (uint32_t m = mask; m; m &= m - 1, ++k) r |= ((v >> k) & 1u) ? m & (0u - m) : 0u;
+  return r;
+}
+
+// The Morton code of a cell (pack11) from the code bits of each axis, and a
+// cell of its bucket inside a cube: with shared buckets a sample updates
+// every point of every bucket of its cube's cells (src/yuezu_fps.cpp:413,
+// 573-597).
+__device__ inline bool bucket_in_cube(const RangeDev &r, uint32_t c11, uint2 cube) {
+  const uint32_t own = deposit_bits(c11 & 1023u, r.cmask[0]) |
+                       deposit_bits((c11 >> 11) & 1023u, r.cmask[1]) |
+                       deposit_bits(c11 >> 22, r.cmask[2]);
+  for (uint64_t code = own % r.T; code < (1ull << r.cbits); code += r.T) {
+    const uint32_t x = extract_bits((uint32_t)code, r.cmask[0]);
+    const uint32_t y = extract_bits((uint32_t)code, r.cmask[1]);
+    const uint32_t z = extract_bits((uint32_t)code, r.cmask[2]);
+    if (x >= r.blocks[0] || y >= r.blocks[1] || z >= r.blocks[2]) continue;
+    const uint32_t a = x | (y << 11) | (z << 22);
+    if (in_box11(a | kGuards, a, cube.x, cube.y)) return true;
+  }
+  return false;
+}
+
 }  // namespace nsfps

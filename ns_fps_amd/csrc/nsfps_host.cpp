@@ -814,6 +814,27 @@ uint32_t list_cap_for(uint32_t n, size_t nclouds) {
   return cap;
 }
 
+// Samples that a call takes one after another from its first lists before it
+// settles layers (k_accept): about 0.8 us each, against 16 to 20 us a round
+// for layers that hold few samples at first.  Calls of up to kSeqOnly samples
+// take all of them so, and end without the layers' final sort.  Per call, all
+// layers, then these rules: 17,000 Gaussian points -> 16 269 and 195 us, 64
+// 372 and 290, 128 438 and 361, 256 496 and 468; 300,000 of a scan -> 64 646
+// and 552; 120,000 of a scan -> 16,384 1.49 and 1.37 ms.  The first 64 of
+// longer calls: 256 459 us, but the 1M-point cube -> 129 938 (940 at 32, 910 at
+// 16) and a scan's 16,384 1.40 ms.  Of a large cloud's many samples the first
+// make no difference but their own: from kSeqLarge points and kSeqFew samples
+// on all are layers (1M-point cube -> 65,536 2.61 ms, with 32 first 2.64;
+// -> 512 1,164 and 1,166 us, 1M Gaussian points -> 512 1,445 and 1,385).
+constexpr uint32_t kSeqOnly = 128, kSeqFirst = 32, kSeqLarge = 524288, kSeqFew = 1024;
+uint32_t seq_samples_for(uint32_t n, uint32_t m) {
+  return m <= kSeqOnly ? kSeqOnly : n < kSeqLarge || m <= kSeqFew ? kSeqFirst : 0u;
+}
+// Rounds in which a call of more than kSeqOnly samples may take some so: the
+// 1M-point cube needs 13 for its first 32, and a later round's layers are as
+// right.
+constexpr uint32_t kSeqRounds = 16;
+
 // Lays out the persistent buffers of one cloud (upper bounds: the padded /
 // dense decision is made on the device data during the build).
 void layout_cloud(Bump &bp, CloudPlan &p, size_t nclouds) {
@@ -1428,13 +1449,13 @@ double ms_between(hipEvent_t a, hipEvent_t b) {
 // and got a list under a quarter full; from the next batch on, every round
 // gets kRefinePasses passes.
 // The batches of rounds (size, refinement passes) the last call of a given
-// shape enqueued, and the rounds it needed.  A call of the same shape enqueues
+// shape (clouds, points, samples, buckets) enqueued, and the rounds it needed.  A call of the same shape enqueues
 // those batches back to back, cut at that many rounds, with no status read in
 // between, then goes on batch by batch if it is not finished; rounds enqueued
 // after a cloud is done return at once.  The samples never depend on how
 // rounds are batched.  Guarded by g_mu.
 struct RoundSchedule {
-  uint64_t shape[5] = {0, 0, 0, 0, 0};
+  uint64_t shape[4] = {0, 0, 0, 0};
   std::vector<std::pair<uint32_t, uint32_t>> batches;
   uint64_t rounds = 0;
 };
@@ -1494,8 +1515,8 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
   const uint32_t hot = wide ? 128u : 64u;
   shape_out->split = split ? kUpdateSplit : 1u;
   shape_out->hot = hot;
-  const uint64_t shape[5] = {nc, plans[0].n, plans[0].m, plans[0].rng.dev.T, max_nl1};
-  const bool replay = std::equal(shape, shape + 5, g_schedule.shape) && !profile;
+  const uint64_t shape[4] = {nc, plans[0].n, plans[0].m, plans[0].rng.dev.T};
+  const bool replay = std::equal(shape, shape + 4, g_schedule.shape) && !profile;
   std::vector<std::pair<uint32_t, uint32_t>> used;
   HIP_TRY(launch_runs_init(d_clouds, nc, split, st));
   // two halves on two streams (kTwoStreamMinClouds); not for the
@@ -1524,20 +1545,22 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
   }
   for (uint32_t k = 0; k <= groups; ++k) g0[k] = (uint32_t)((uint64_t)nc * k / groups);
   uint64_t enqueued = 0;
+  uint32_t max_m = 0;
+  for (auto &p : plans) max_m = std::max(max_m, p.m);
+  const uint32_t seq_rounds =
+      max_m <= kSeqOnly ? ~0u : plans[0].dev.seq_samples ? kSeqRounds : 0u;
   const auto enqueue = [&](uint32_t take, uint32_t np) -> hipError_t {
     if (!two)
       return launch_rounds(d_clouds, nc, max_nl1, take, np, profile, alias, split, mixed,
-                           list_cap, (uint32_t)enqueued, st);
+                           list_cap, (uint32_t)enqueued, seq_rounds, st);
     for (uint32_t k = 0; k < groups; ++k) {
       const hipError_t e = launch_rounds(d_clouds + g0[k], g0[k + 1] - g0[k], max_nl1, take, np,
                                          profile, alias, split, mixed, list_cap,
-                                         (uint32_t)enqueued, sts[k]);
+                                         (uint32_t)enqueued, seq_rounds, sts[k]);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
   };
-  uint32_t max_m = 0;
-  for (auto &p : plans) max_m = std::max(max_m, p.m);
   std::vector<CloudStatus> pr(nc);
   uint64_t last_samples = 0;
   uint32_t batch = 4, stalled = 0, passes = 0;
@@ -1560,8 +1583,9 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
       used.emplace_back(batch, passes);
     }
     launched = false;
-    // the samples in order, once a cloud is done
-    for (uint32_t k = 0; k < groups; ++k)
+    // the samples in order, once a cloud is done (those taken one after
+    // another are)
+    for (uint32_t k = 0; k < groups && max_m > kSeqOnly; ++k)
       HIP_TRY(launch_order(d_clouds + g0[k], g0[k + 1] - g0[k], max_m, sts[k]));
     for (uint32_t k = 1; k < groups; ++k) {  // the statuses are read on st once every group's rounds are done
       HIP_TRY(hipEventRecord(ap2->join[k - 1], sts[k]));
@@ -1586,9 +1610,12 @@ nsfps_status run_rounds(std::vector<CloudPlan> &plans, const CloudDev *d_clouds,
     }
     *rounds_out = rounds;
     if (all) {
-      std::copy(shape, shape + 5, g_schedule.shape);
+      std::copy(shape, shape + 4, g_schedule.shape);
       g_schedule.batches = used;
-      g_schedule.rounds = rounds + 1;  // and the one that finds the end
+      // and the round that finds the end, unless the last sample did
+      bool full = max_m <= kSeqOnly;
+      for (auto &q : pr) full = full && q.iter == max_m;
+      g_schedule.rounds = rounds + (full ? 0 : 1);
       fin = pr;
       break;
     }
@@ -1860,6 +1887,7 @@ nsfps_status sample_clouds(std::vector<CloudPlan> &plans, CallLayout &L, const W
   devs.clear();
   uint32_t lds_bytes = 0;
   for (auto &p : plans) {
+    p.dev.seq_samples = seq_samples_for(p.n, p.m);
     devs.push_back(p.dev);
     lds_bytes = std::max(lds_bytes, p.dev.lds.total);
   }

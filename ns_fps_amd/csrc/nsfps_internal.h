@@ -34,6 +34,8 @@ constexpr uint32_t kListCap = 4096;
 // first rounds of a cloud settle few, however long their lists.
 constexpr uint32_t kListMin = 1024;
 constexpr uint32_t kListGrow = 8;
+// list of the rounds that take samples one after another (seq_samples)
+constexpr uint32_t kSeqList = 1024;
 // list_cap of small clouds (host's kShortListPoints)
 constexpr uint32_t kListShort = 512;
 // rounds in the log that orders the samples, for up to 131,072 samples (more
@@ -115,6 +117,7 @@ struct RunState {
   uint32_t rounds;    // rounds that ran (statistics)
   uint32_t err;       // set if a list overflowed (internal error)
   uint32_t forced;    // rounds whose threshold was forced for want of refinement passes
+  uint32_t seq;       // this round's list is sampled one after another
   uint32_t fin;       // the gather pass found the end (the accept pass then sets done)
 };
 
@@ -178,6 +181,7 @@ struct CloudDev {
   uint64_t *log_ktop;         //    a bound on its keys
   uint32_t *log_start;        //    and the samples before it
   uint32_t list_cap, log_cap;
+  uint32_t seq_samples;       // samples taken one after another before the layers begin
 };
 
 // Argmax key: larger min-distance wins, equal distances go to the smaller

@@ -141,11 +141,12 @@ hipError_t launch_runs_init(const CloudDev *d_clouds, uint32_t nclouds, uint32_t
 // alias: some cloud's cells share buckets; split: the update pass takes
 // kUpdateSplit workgroups per level-1 node; mixed: the clouds' leaves are runs of 64 slots
 // that may hold several buckets (never with alias).  list_cap: the clouds'
-// longest list; first: the rounds enqueued before for these clouds.
+// longest list; first: the rounds enqueued before for these clouds; seq_rounds:
+// the first rounds that may take samples one after another.
 hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t max_nl1,
                          uint32_t rounds, uint32_t passes, bool profile, bool alias,
                          bool split, bool mixed, uint32_t list_cap, uint32_t first,
-                         hipStream_t st);
+                         uint32_t seq_rounds, hipStream_t st);
 // The samples of every finished cloud (at most m each) into its out, in order.
 hipError_t launch_order(const CloudDev *d_clouds, uint32_t nclouds, uint32_t m, hipStream_t st);
 

@@ -249,7 +249,8 @@ __device__ void record_samples(const CloudDev &c, uint32_t par, uint32_t *sc) {
   NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
   const uint32_t nl = min(rs.nl[par ^ 1u], kListCap), base = rs.ntaken, nlog = rs.nlog;
   const uint64_t bkey = rs.bkey, bmin = rs.bmin, ktop = rs.ktop;
-  const uint32_t done = *gptr(c.done);
+  // a list sampled one after another is recorded by the accept pass
+  const uint32_t done = *gptr(c.done) | rs.seq;
   constexpr uint32_t kSlots = kListCap / kPassThreads;
   bool take[kSlots];
   float4 p[kSlots];
@@ -719,14 +720,16 @@ __device__ __forceinline__ uint32_t bit_length(uint64_t v) { return v ? 64u - __
 // the hot leaves whose points it reads and those points.  Its first workgroup
 // also finds the sampling's end: when m samples have keys above every key
 // left, or only points at distance 0 are left (src/yuezu_fps.cpp:705-706).
-// It leaves that in rs.fin, which no workgroup of this launch tests; the
+// may_seq: the accept pass that follows can take samples one after another.
+// The end is left in rs.fin, which no workgroup of this launch tests; the
 // accept pass tests fin and writes done, which none of its own tests.  With
 // one word for both, waves of one workgroup could read it before and after
 // the write, and those that went on would scan LDS words that the others
 // never wrote.
 template <bool PROF>
 __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restrict__ clouds,
-                                                         uint32_t passes, uint32_t par) {
+                                                         uint32_t passes, uint32_t par,
+                                                         uint32_t may_seq) {
   __shared__ uint32_t s_sc[kPassWaves + 3];
   __shared__ uint64_t s_wk[kPassWaves];
   const CloudDev &c = clouds[blockIdx.y];
@@ -755,8 +758,12 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
     }
   };
   read_leaf(blockIdx.x);
-  if (blockIdx.x >= c.nl1 || *gptr(c.done)) return;
   NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
+  if (blockIdx.x >= c.nl1 || *gptr(c.done)) {
+    // done: the accept pass, which sets it, tests fin
+    if (blockIdx.x == 0 && tid == 0) rs.fin = 1;
+    return;
+  }
   uint64_t gt1 = 0, gt2 = 0, gt3 = 0;
   bool forced = false;
   const Sel s = sel_replay(c, passes + 1, passes, s_sc, &forced, &h0);
@@ -802,9 +809,13 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
     if (tid == 0) {
       rs.bkey = bkey;
       rs.ktop = ktop;
+      // rounds that take samples one after another, and the one after them
+      const bool early = rs.seq != 0u || T < c.seq_samples;
+      rs.seq = may_seq && T < c.seq_samples ? 1u : 0u;
       // the first rounds start from windows over the whole key range and are
-      // forced as a rule; later forced rounds ask for refinement passes
-      rs.forced += forced && rs.rounds >= 2 ? 1u : 0u;
+      // forced as a rule, and few of a list are sampled in the early ones;
+      // later forced rounds ask for refinement passes
+      rs.forced += forced && rs.rounds >= 2 && (!early || s.total < 64u) ? 1u : 0u;
       // next round: bins of 1/512 to 1/1024 of this round's key span, over 3
       // spans (a window that ends above the next threshold leaves the list
       // short; most leaves with a key in it are read anyway, for a sample
@@ -814,12 +825,13 @@ __global__ __launch_bounds__(kPassThreads) void k_gather(const CloudDev *__restr
       // 16.2 (1M cube 2.57, 2.55, 2.62, 2.68; with kListGrow 8 for 4, 3 spans
       // 2.56 and 16.0).
       const bool grow = 2 * s.total < rs.cap;
-      const uint64_t span = (grow ? rs.kref0 : ktop) - bkey + 1;
+      const uint64_t span = (grow || T < c.seq_samples ? rs.kref0 : ktop) - bkey + 1;
+      const uint32_t bins = T < c.seq_samples ? 11u : 10u;
       uint32_t nx = bit_length(span);
-      nx = nx > 10u ? nx - 10u : 0u;
+      nx = nx > bins ? nx - bins : 0u;
       nx = nx < kMaxShift ? nx : kMaxShift;
       rs.s0_next = nx;
-      rs.nb_next = grow ? kHistBins : min((uint32_t)(span >> nx) * 3 + 1, kHistBins);
+      rs.nb_next = grow || T < c.seq_samples ? kHistBins : min((uint32_t)(span >> nx) * 3 + 1, kHistBins);
       if (fin) {
         *gptr(c.iter) = min(T, m);
         rs.fin = 1;
@@ -986,6 +998,176 @@ typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 #define NSFPS_CONSTANT
 #endif
 
+// The first seq_samples of a cloud are taken from its lists one after another
+// instead, as the reference does: early layers hold few samples, so a list is
+// worth several rounds of them.  One workgroup, four entries a thread, one
+// barrier a sample: each wave publishes its largest key, every wave takes the
+// largest of those, and the entries that the sample's cube holds are lowered;
+// it ends when no listed key is left at or above the threshold, or they all
+// are taken.  These samples
+// come in order, so a call that ends among them needs no sort.  Bound by the
+// chain of one sample: some 200 instructions, two LDS reads and the barrier,
+// about 0.8 us (1.35 with the cube's half-widths worked out on every lane
+// alike, 1.05 with keys compared as integer pairs).  Lists and windows are
+// the first rounds' there: 1,024 entries, bins of 1/1024 to 1/2048 of the span
+// below the last threshold.
+constexpr uint32_t kSettleSlots = kSeqList / kAcceptThreads;
+static_assert(kSettleSlots * kAcceptThreads == kSeqList, "whole slots");
+
+// Keys as doubles: their high words are finite floats' bits, below the
+// exponent of infinities, so they order as the integers do, and one
+// instruction takes a maximum (subnormal doubles are kept).
+__device__ __forceinline__ double max_key(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+template <int CTRL>
+__device__ __forceinline__ double max_key_dpp(double a) {
+  const uint64_t k = (uint64_t)__double_as_longlong(a);
+  const uint64_t o = ((uint64_t)dpp_mov<CTRL>((uint32_t)(k >> 32)) << 32) | dpp_mov<CTRL>((uint32_t)k);
+  return max_key(a, __longlong_as_double((long long)o));
+}
+__device__ __forceinline__ uint64_t wave_max_key(double a) {
+  a = max_key_dpp<kDppQuad1032>(a);
+  a = max_key_dpp<kDppQuad2301>(a);
+  a = max_key_dpp<kDppHalfMirror>(a);
+  a = max_key_dpp<kDppMirror>(a);
+  const uint64_t k = (uint64_t)__double_as_longlong(a);
+  const uint32_t hi = (uint32_t)(k >> 32), lo = (uint32_t)k;
+  uint64_t best = ((uint64_t)rdlane(hi, 0) << 32) | rdlane(lo, 0);
+#pragma unroll
+  for (uint32_t r = 16; r < 64; r += 16) {
+    const uint64_t v = ((uint64_t)rdlane(hi, r) << 32) | rdlane(lo, r);
+    best = v > best ? v : best;
+  }
+  return best;
+}
+
+template <bool ALIAS>
+__device__ __forceinline__ void settle(const CloudDev &c, uint32_t par, uint32_t nl) {
+  struct Cand {
+    uint64_t key;
+    uint32_t row, cell;  // input row, cell (pack11)
+    float x, y, z;
+    uint32_t entry;  // of the list
+  };
+  __shared__ Cand s_cand[2][kAcceptWaves];
+  // the range at hand: reads of it from memory would wait for the sample's stores
+  __shared__ RangeDev s_r;
+  NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  if (tid < sizeof(RangeDev) / 4)
+    reinterpret_cast<uint32_t *>(&s_r)[tid] = reinterpret_cast<const uint32_t *>(&c.r)[tid];
+  // lane 8 a + k compares the distance with threshold k of axis a (half_axis)
+  static_assert(3 * kCubeThr <= 64, "a lane per threshold");
+  const float thr = lane < 3 * kCubeThr ? (&c.r.cube_thr[0][0])[lane] : INFINITY;
+  // a sample's words, one a lane: distance, ~rank, row, and the row as a result
+  NSFPS_GLOBAL uint32_t *const SW = vgpr_ptr(gptr(
+      lane == 0 ? c.smp_d : lane == 1 ? c.smp_lo : lane == 2 ? c.smp_row : reinterpret_cast<uint32_t *>(c.out)));
+  NSFPS_GLOBAL uint2 *const LC = vgpr_ptr(gptr(c.list_c));
+  const uint32_t T = rs.ntaken, end = min(c.m, c.seq_samples);
+  const uint64_t bkey = rs.bkey;
+  float x[kSettleSlots], y[kSettleSlots], z[kSettleSlots];
+  uint32_t row[kSettleSlots], cell[kSettleSlots];
+  uint64_t key[kSettleSlots];
+#pragma unroll
+  for (uint32_t s = 0; s < kSettleSlots; ++s) {
+    const uint32_t i = s * kAcceptThreads + tid;
+    const float4 p = gptr(c.list_p)[i];
+    const uint2 r = gptr(c.list_r)[i];
+    x[s] = p.x;
+    y[s] = p.y;
+    z[s] = p.z;
+    key[s] = i < nl ? make_key(p.w, r.x) : 0ull;
+    row[s] = r.y;
+    cell[s] = i < nl ? pack11(pack_cell(cell_axis(c.r, 0, p.x), cell_axis(c.r, 1, p.y),
+                                        cell_axis(c.r, 2, p.z)))
+                     : 0u;
+  }
+  uint32_t cnt = 0, taken = 0;
+  uint64_t top;
+  __syncthreads();
+  const uint32_t b0 = uniform(s_r.blocks[0]), b1 = uniform(s_r.blocks[1]), b2 = uniform(s_r.blocks[2]);
+  while (true) {
+    double best = __longlong_as_double((long long)key[0]);
+#pragma unroll
+    for (uint32_t s = 1; s < kSettleSlots; ++s)
+      best = max_key(best, __longlong_as_double((long long)key[s]));
+    const uint64_t mine = wave_max_key(best);
+    Cand *const cd = s_cand[cnt & 1u];
+#pragma unroll
+    for (uint32_t s = 0; s < kSettleSlots; ++s)
+      if (key[s] == mine)  // keys are unique, but for the absent ones' 0
+        cd[wave] = Cand{mine, row[s], cell[s], x[s], y[s], z[s], s * kAcceptThreads + tid};
+    __syncthreads();
+    uint32_t w = 0;
+    top = cd[0].key;
+#pragma unroll
+    for (uint32_t v = 1; v < kAcceptWaves; ++v) {
+      const uint64_t k = cd[v].key;
+      w = k > top ? v : w;
+      top = k > top ? k : top;
+    }
+    top = uni(top);
+    if (top < bkey || (top >> 32) == 0 || T + cnt >= end) break;
+    const Cand p = cd[uniform(w)];
+    const float px = uni(p.x), py = uni(p.y), pz = uni(p.z), D = key_dist(top);
+    const uint32_t c11 = uniform(p.cell), e = uniform(p.entry), at = T + cnt;
+    const uint64_t ge = __ballot(D >= thr);
+    uint32_t lo_c, hi_c, h = 0, beyond = 0;
+#pragma unroll
+    for (uint32_t a = 0; a < 3; ++a) {
+      const uint32_t k = (uint32_t)__popc((uint32_t)(ge >> (a * kCubeThr)) & ((1u << kCubeThr) - 1));
+      h |= k << (10 * a);
+      beyond |= k == kCubeThr ? 1u : 0u;
+    }
+    if (beyond) h = uniform(packed_halves(s_r, D));
+    cube_corners((c11 & 1023u) | (((c11 >> 11) & 1023u) << 10) | ((c11 >> 22) << 20), h, b0, b1, b2,
+                 lo_c, hi_c);
+    const uint2 cube = make_uint2(uniform(pack11(lo_c)), uniform(pack11(hi_c) | kGuards));
+    if (tid < 4) SW[at] = lane == 0 ? (uint32_t)(top >> 32) : lane == 1 ? (uint32_t)top : p.row;
+    if (tid == e % kAcceptThreads) {
+      taken |= 1u << (e / kAcceptThreads);
+      LC[e] = cube;
+    }
+#pragma unroll
+    for (uint32_t s = 0; s < kSettleSlots; ++s) {
+      const uint32_t dd = __float_as_uint(sqdist(x[s], y[s], z[s], px, py, pz));
+      bool in = (dd < (uint32_t)(key[s] >> 32)) &
+                (in_box11(cell[s] | kGuards, cell[s], cube.x, cube.y) != 0);
+      if (ALIAS && dd < (uint32_t)(key[s] >> 32) && !in) in = bucket_in_cube(s_r, cell[s], cube);
+      key[s] = in ? ((uint64_t)dd << 32) | (uint32_t)key[s] : key[s];
+    }
+    ++cnt;
+  }
+#pragma unroll
+  for (uint32_t s = 0; s < kSettleSlots; ++s)
+    if (s * kAcceptThreads + tid < nl)
+      gptr(c.list_f)[s * kAcceptThreads + tid] = (taken >> s) & 1u ? 0u : 1u;
+  if (tid == 0) {
+    // every sample's key is above top, and every key left at or below kref0
+    const uint64_t low = top >= bkey ? top + 1 : bkey, b = low < rs.bmin ? low : rs.bmin;
+    const uint32_t i = rs.nlog < c.log_cap ? rs.nlog : c.log_cap - 1;
+    rs.bmin = b;
+    gptr(c.log_bmin)[i] = b;
+    if (rs.nlog < c.log_cap) {
+      gptr(c.log_ktop)[i] = rs.ktop;
+      gptr(c.log_start)[i] = T;
+      rs.nlog += 1;
+    }
+    rs.ntaken = T + cnt;
+    *gptr(c.iter) = T + cnt;
+    rs.cap = T + cnt < c.seq_samples ? kSeqList : min(kListMin, c.list_cap);
+    rs.kref0 = low - 1;
+    if (T + cnt >= c.m) *gptr(c.done) = 1;
+  }
+}
+
+// SEQ: may take the list's samples one after another (rs.seq); a variant of its
+// own, for it needs registers that the layers' rounds leave to more waves (in
+// one kernel the 50-round scan was 4 % slower).
+template <bool ALIAS, bool SEQ>
 __global__ __launch_bounds__(kAcceptThreads) void k_accept(const CloudDev *__restrict__ clouds,
                                                            uint32_t par, uint32_t ncube) {
   const CloudDev &c = clouds[blockIdx.y];
@@ -1021,6 +1203,10 @@ __global__ __launch_bounds__(kAcceptThreads) void k_accept(const CloudDev *__res
     rs.s0 = rs.s0_next;
     rs.nb = rs.nb_next;
     rs.rounds += 1;
+  }
+  if (SEQ && rs.seq) {  // written by the gather pass
+    if (blockIdx.x == 0) settle<ALIAS>(c, par, min(nl, kSeqList));
+    return;
   }
   if (cubes) {
     const uint32_t i = blockIdx.x * kAcceptThreads + tid;
@@ -1237,7 +1423,8 @@ __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__re
     rs.nl[1] = 1;  // read by round 0
     rs.ntaken = 1;
     rs.nlog = 0;
-    rs.cap = min(kListMin, c.list_cap);
+    rs.cap = c.seq_samples > 1 ? kSeqList : min(kListMin, c.list_cap);
+    rs.seq = 0;
     rs.bmin = ~0ull;
     rs.ktop = ~0ull;
     rs.rounds = 0;
@@ -1246,6 +1433,7 @@ __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__re
     const float4 p0 = *gptr(c.root_pos);
     gptr(c.smp_d)[0] = gptr(c.smp_lo)[0] = 0xffffffffu;
     gptr(c.smp_row)[0] = 0;
+    gptr(c.out)[0] = 0;
     gptr(c.list_f)[0] = 0;
     gptr(c.list_p)[0] = make_float4(p0.x, p0.y, p0.z, INFINITY);
     gptr(c.list_c)[0] = make_uint2(
@@ -1262,7 +1450,8 @@ __global__ __launch_bounds__(kPassThreads) void k_runs_init(const CloudDev *__re
 hipError_t preload_runs_kernels() {
   constexpr uint32_t S = kUpdateSplit;
   return func_attributes(
-      k_runs_init, k_refine, k_gather<false>, k_accept, k_sort_rounds, k_order,
+      k_runs_init, k_refine, k_gather<false>, k_accept<false, false>, k_accept<false, true>,
+      k_accept<true, true>, k_sort_rounds, k_order,
       k_update<false, false, 1, false>, k_update<false, false, S, false>,
       k_update<false, true, 1, false>, k_update<false, true, S, false>,
       k_update<false, false, 1, true>, k_update<false, false, S, true>);
@@ -1278,16 +1467,19 @@ hipError_t launch_runs_init(const CloudDev *d_clouds, uint32_t nclouds, uint32_t
 // round's samples), gather and accept passes.
 template <bool PROF, bool ALIAS, uint32_t SPLIT, bool MIXED>
 void launch_round(const CloudDev *d_clouds, uint32_t nclouds, dim3 grid, dim3 sparse,
-                  uint32_t passes, uint32_t list_cap, uint32_t round, hipStream_t st) {
+                  uint32_t passes, uint32_t list_cap, uint32_t round, bool seq, hipStream_t st) {
   k_update<PROF, ALIAS, SPLIT, MIXED>
       <<<dim3(grid.x * SPLIT + 1, grid.y), kPassThreads, 0, st>>>(d_clouds, round);
   for (uint32_t p = 1; p <= passes; ++p)
     k_refine<<<sparse, kPassThreads, 0, st>>>(d_clouds, p, passes);
-  k_gather<PROF><<<sparse, kPassThreads, 0, st>>>(d_clouds, passes, round & 1u);
+  k_gather<PROF><<<sparse, kPassThreads, 0, st>>>(d_clouds, passes, round & 1u, seq ? 1u : 0u);
   const uint32_t ncube = (list_cap + kAcceptThreads - 1) / kAcceptThreads;
   const uint32_t xgs = list_cap / kAcceptX;
-  k_accept<<<dim3(ncube + xgs * (list_cap / kAcceptChunk) / kAcceptWaves, nclouds),
-             kAcceptThreads, 0, st>>>(d_clouds, round & 1u, ncube);
+  const dim3 blocks(ncube + xgs * (list_cap / kAcceptChunk) / kAcceptWaves, nclouds);
+  if (seq)
+    k_accept<ALIAS, true><<<blocks, kAcceptThreads, 0, st>>>(d_clouds, round & 1u, ncube);
+  else
+    k_accept<false, false><<<blocks, kAcceptThreads, 0, st>>>(d_clouds, round & 1u, ncube);
 }
 
 hipError_t launch_order(const CloudDev *d_clouds, uint32_t nclouds, uint32_t m, hipStream_t st) {
@@ -1301,14 +1493,14 @@ hipError_t launch_order(const CloudDev *d_clouds, uint32_t nclouds, uint32_t m, 
 hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t max_nl1,
                          uint32_t rounds, uint32_t passes, bool profile, bool alias,
                          bool split, bool mixed, uint32_t list_cap, uint32_t first,
-                         hipStream_t st) {
+                         uint32_t seq_rounds, hipStream_t st) {
   if (alias && mixed) return hipErrorInvalidValue;  // leaves of several buckets: one cell each
   if (list_cap < kListShort || list_cap > kListCap || (list_cap & (list_cap - 1)))
     return hipErrorInvalidValue;
   const dim3 grid(max_nl1, nclouds);
   const dim3 sparse(max_nl1 < kSparseGroups ? max_nl1 : kSparseGroups, nclouds);
   using Launch = void (*)(const CloudDev *, uint32_t, dim3, dim3, uint32_t, uint32_t, uint32_t,
-                          hipStream_t);
+                          bool, hipStream_t);
   constexpr uint32_t S = kUpdateSplit;
   // [profile][cells: one per leaf, shared buckets, several per leaf][split]
   static constexpr Launch kRound[2][3][2] = {
@@ -1320,7 +1512,7 @@ hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t ma
        {launch_round<true, false, 1, true>, launch_round<true, false, S, true>}}};
   const Launch one = kRound[profile][alias ? 1 : mixed ? 2 : 0][split];
   for (uint32_t r = 0; r < rounds; ++r)
-    one(d_clouds, nclouds, grid, sparse, passes, list_cap, first + r, st);
+    one(d_clouds, nclouds, grid, sparse, passes, list_cap, first + r, first + r < seq_rounds, st);
   return hipGetLastError();
 }
 

@@ -147,13 +147,6 @@ struct CellRange {
   }
 };
 
-// The bits of v at the set positions of mask, lowest first.
-__device__ __forceinline__ uint32_t deposit_bits(uint32_t v, uint32_t mask) {
-  uint32_t r = 0, k = 0;
-  for (uint32_t m = mask; m; m &= m - 1, ++k) r |= ((v >> k) & 1u) ? m & (0u - m) : 0u;
-  return r;
-}
-
 constexpr uint32_t kSpatialBits = 16;  // two passes of the sort
 
 // One cloud's points in the logical order (by bucket, then input row: rank and
@@ -358,25 +351,6 @@ __global__ __launch_bounds__(kSmThreads) void k_small_sort(SmallDev *devs) {
 
 // ----------------------------------------------------------------- sample
 
-
-// The Morton code of a cell (pack11) from the code bits of each axis, and a
-// cell of its bucket inside a cube: with shared buckets a sample updates
-// every point of every bucket of its cube's cells (src/yuezu_fps.cpp:413,
-// 573-597).
-__device__ bool bucket_in_cube(const RangeDev &r, uint32_t c11, uint2 cube) {
-  const uint32_t own = deposit_bits(c11 & 1023u, r.cmask[0]) |
-                       deposit_bits((c11 >> 11) & 1023u, r.cmask[1]) |
-                       deposit_bits(c11 >> 22, r.cmask[2]);
-  for (uint64_t code = own % r.T; code < (1ull << r.cbits); code += r.T) {
-    const uint32_t x = extract_bits((uint32_t)code, r.cmask[0]);
-    const uint32_t y = extract_bits((uint32_t)code, r.cmask[1]);
-    const uint32_t z = extract_bits((uint32_t)code, r.cmask[2]);
-    if (x >= r.blocks[0] || y >= r.blocks[1] || z >= r.blocks[2]) continue;
-    const uint32_t a = x | (y << 11) | (z << 22);
-    if (in_box11(a | kGuards, a, cube.x, cube.y)) return true;
-  }
-  return false;
-}
 
 // A point is updated by a sample when the sample's cube holds its cell, or
 // with shared buckets another cell of its bucket.

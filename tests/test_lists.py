@@ -74,6 +74,22 @@ def test_a_window_of_coarse_bins_that_ends_above_the_last_keys(lib, oracle):
     assert np.array_equal(lib.fps(P, 1500, rng), oracle.fps(P, 1500, rng))
 
 
+@pytest.mark.parametrize("kind,n,blocks", [
+    ("cube", 17000, (32, 32, 32)), ("cube", 600, (1, 1, 1)), ("cube", 40000, (17, 17, 17)),
+    ("lattice", 20000, (15, 16, 16)), ("dups", 2000, (8, 8, 8)), ("rings", 33000, (32, 32, 4)),
+    ("plane", 300000, (32, 32, 2)),
+])
+def test_first_samples_match_the_oracle(lib, oracle, monkeypatch, kind, n, blocks):
+    """Few samples are taken one after another (128 at most: the whole call;
+    more: about the first 64, the rest by layers), on every list length."""
+    P = cloud(kind, n)
+    monkeypatch.setenv("NSFPS_SMALL", "0")
+    want = oracle.fps(P, 600 if n > 600 else 599, (*UNIT, *blocks))
+    for m in (2, 3, 63, 64, 65, 127, 128, 129, 200, len(want)):
+        got = lib.fps(P, m, (*UNIT, *blocks))
+        assert np.array_equal(got, want[:m]), (m, len(got))
+
+
 @pytest.mark.parametrize("batch,n", [(2, 33000), (4, 33000), (16, 33000), (64, 33000), (7, 20000)])
 def test_shorter_lists_of_many_clouds_match_the_oracle(lib, oracle, batch, n):
     kinds = ["cube", "lattice", "dups", "rings"]

@@ -19,7 +19,7 @@ def bodies():
     with open(SRC) as f:
         text = re.sub(r"//[^\n]*", "", f.read())
     out = {}
-    for m in re.finditer(r"\b(k_\w+|record_samples|sel_replay|node_key)\s*\([^;{}]*\)\s*\{", text):
+    for m in re.finditer(r"\b(k_\w+|record_samples|sel_replay|node_key|settle)\s*\([^;{}]*\)\s*\{", text):
         depth, at = 1, m.end()
         while depth:
             depth += {"{": 1, "}": -1}.get(text[at], 0)
