@@ -1711,14 +1711,27 @@ bool choose_runs(std::vector<CloudPlan> &plans) {
 
 // Calls whose clouds all have the same, small point count are sorted and
 // sampled by one workgroup per cloud (nsfps_small.hip): two launches and one
-// read-back for the call.  The switches that choose or trace the general
-// engines' parts, and the failure injection that counts their operations,
-// take those engines; NSFPS_SMALL=0 or 1 decides it alone.
+// read-back for the call.  Up to 8,192 points (kernels of at most 8 points a
+// thread) that is faster at every sample count; above, one CU is slower than
+// the rounds over the whole chip unless there are many clouds, or the cloud
+// is not much larger and few samples are taken.  Per call, one workgroup and
+// rounds: 8,192 Gaussian points -> 1,024 480 and 612 us; 10,000 -> 312 408
+// and 493, -> 1,250 655 and 660, -> 5,000 1,402 and 910; 16,384 -> 512 571
+// and 518, -> 8,192 2,369 and 1,059 (a lattice 5,128 and 1,846); 64 clouds of
+// 16,384 -> 4,096 1,434, of 17,000 -> 4,250 by rounds 1,855; 4 clouds 1,318
+// and 993.  The switches that choose or trace the general engines' parts, and
+// the failure injection that counts their operations, take those engines;
+// NSFPS_SMALL=0 or 1 decides it alone.
+constexpr uint32_t kSmallAlways = 8192, kSmallFewSamples = 12288, kSmallManyClouds = 16;
 bool small_wanted(const std::vector<CloudPlan> &plans) {
   for (auto &p : plans)
     if (p.n != plans[0].n || p.n > kSmallMaxPoints || p.rng.dev.T > (1u << kSmallMaxBits))
       return false;
   if (const char *e = getenv("NSFPS_SMALL")) return atoi(e) != 0;
+  const uint32_t n = plans[0].n;
+  if (n > kSmallAlways && plans.size() < kSmallManyClouds &&
+      !(n <= kSmallFewSamples && plans[0].m <= n / 8))
+    return false;
   for (const char *v : {"NSFPS_ENGINE", "NSFPS_NO_PADDED", "NSFPS_MIXED", "NSFPS_STREAMS",
                         "NSFPS_GLOBAL_SORT", "NSFPS_HOT", "NSFPS_PROFILE", "NSFPS_INJECT"})
     if (getenv(v)) return false;

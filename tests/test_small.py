@@ -76,6 +76,25 @@ def test_small_clouds_match_the_oracle(lib, hip, oracle, monkeypatch, small, kin
         hip.free(d_out)
 
 
+@pytest.mark.parametrize("n,m,batch,one", [
+    (8192, 8000, 1, True), (8193, 1024, 1, True), (8193, 1025, 1, False), (12288, 1536, 1, True),
+    (12289, 64, 1, False), (16384, 4096, 15, False), (16384, 4096, 16, True), (16385, 64, 16, False),
+])
+def test_which_calls_one_workgroup_a_cloud_takes(lib, oracle, n, m, batch, one):
+    """At each side of the rule's lines.  The statistics tell the two apart:
+    a small call's sampling is one launch, so late_ms is all of sample_ms."""
+    P = [cloud("cube", n), cloud("cube", n + 1)[:n]]
+    rng = (*UNIT, 16, 16, 16)
+    if batch == 1:
+        got = [lib.fps(P[0], m, rng)]
+    else:
+        got = lib.fps_batched(np.stack([P[b % 2] for b in range(batch)]), m, [rng] * batch)
+    st = lib.stats()
+    assert (st["late_ms"] == st["sample_ms"] and st["wide_ms"] == 0.0) == one
+    for b in range(min(batch, 2)):
+        assert np.array_equal(got[b], oracle.fps(P[b], m, rng))
+
+
 @pytest.mark.parametrize("scale", [1.0, 1e-21, 3e18, 1e30])
 def test_small_clouds_at_the_ends_of_the_number_range(lib, oracle, monkeypatch, scale):
     """Squared distances that are subnormal, or overflow."""
