@@ -879,6 +879,9 @@ void layout_cloud(Bump &bp, CloudPlan &p, size_t nclouds) {
   // rounds share its last entry.  A plan learns m later: at most n.
   const uint32_t mmax = p.m ? p.m : n;
   c.log_cap = std::min<uint32_t>(std::max(kLogCap, mmax / 128), mmax + 1);
+  // (NSFPS_LOG_ROUNDS lowers it, so that tests fill it)
+  if (const char *e = getenv("NSFPS_LOG_ROUNDS"))
+    c.log_cap = std::min<uint32_t>(std::max(1, atoi(e)), c.log_cap);
   c.log_bmin = bp.take<uint64_t>(c.log_cap);
   c.log_ktop = bp.take<uint64_t>(c.log_cap);
   c.log_start = bp.take<uint32_t>(c.log_cap);
@@ -1733,7 +1736,8 @@ bool small_wanted(const std::vector<CloudPlan> &plans) {
       !(n <= kSmallFewSamples && plans[0].m <= n / 8))
     return false;
   for (const char *v : {"NSFPS_ENGINE", "NSFPS_NO_PADDED", "NSFPS_MIXED", "NSFPS_STREAMS",
-                        "NSFPS_GLOBAL_SORT", "NSFPS_HOT", "NSFPS_PROFILE", "NSFPS_INJECT"})
+                        "NSFPS_GLOBAL_SORT", "NSFPS_HOT", "NSFPS_PROFILE", "NSFPS_INJECT",
+                        "NSFPS_LOG_ROUNDS"})
     if (getenv(v)) return false;
   return true;
 }

@@ -1243,9 +1243,9 @@ __global__ __launch_bounds__(kAcceptThreads) void k_accept(const CloudDev *__res
 }
 
 // Sorts each round's samples by key, descending (one workgroup a round; a
-// round settles at most kListCap; the log's last entry may stand for more,
-// and is left as it is): bins of equal width over the round's span, then each
-// sample's place among its bin's.
+// round settles at most kListCap): bins of equal width over the round's span,
+// then each sample's place among its bin's.  The log's last entry may stand
+// for many rounds: its samples are sorted kListCap at a time.
 constexpr uint32_t kSortThreads = 512;
 __global__ __launch_bounds__(kSortThreads) void k_sort_rounds(const CloudDev *__restrict__ clouds) {
   const CloudDev &c = clouds[blockIdx.y];
@@ -1258,10 +1258,15 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rounds(const CloudDev *__
   if (!*gptr(c.done)) return;
   const NSFPS_GLOBAL RunState &rs = *gptr(c.rs);
   const uint32_t nlog = rs.nlog, T = min(rs.ntaken, c.n), tid = threadIdx.x;
-  for (uint32_t r = blockIdx.x; r < nlog; r += gridDim.x) {
-    const uint32_t b = gptr(c.log_start)[r], e = r + 1 < nlog ? gptr(c.log_start)[r + 1] : T;
+  if (nlog == 0) return;
+  // the last entry's pieces go on as if each had an entry
+  const uint32_t last = gptr(c.log_start)[nlog - 1];
+  const uint32_t pieces = T > last ? (T - last + kListCap - 1) / kListCap : 1u;
+  for (uint32_t r = blockIdx.x; r < nlog - 1 + pieces; r += gridDim.x) {
+    const uint32_t b = r < nlog ? gptr(c.log_start)[r] : last + (r - (nlog - 1)) * kListCap;
+    const uint32_t e = r + 1 < nlog ? gptr(c.log_start)[r + 1] : min(b + kListCap, T);
     const uint32_t n = e - b;
-    if (n < 2 || n > kListCap) continue;
+    if (n < 2 || n > kListCap) continue;  // never above it
     uint2 k[kSlots];
     uint32_t row[kSlots], bin[kSlots], at[kSlots];
     for (uint32_t j = tid; j < kListCap + 4; j += kSortThreads) s_bin[j] = 0;
@@ -1373,12 +1378,14 @@ __global__ __launch_bounds__(kOrderThreads) void k_order(const CloudDev *__restr
       }
       if (sub == 0) r = a0 < nlog ? gptr(c.log_start)[a0] : T;
       for (uint32_t q = a0 + sub; q < e0; q += kOrderLanes) {
-        const uint32_t b = gptr(c.log_start)[q], e = q + 1 < nlog ? gptr(c.log_start)[q + 1] : T;
-        if (e - b > kListCap) {  // not sorted
-          for (uint32_t j = b; j < e; ++j) r += (((uint64_t)sd[j] << 32) | sl[j]) > k ? 1u : 0u;
-        } else if (i >= b && i < e) {
-          r += i - b;
-        } else {
+        const uint32_t end = q + 1 < nlog ? gptr(c.log_start)[q + 1] : T;
+        // one sorted piece, but for a full log's last entry
+        for (uint32_t b = gptr(c.log_start)[q]; b < end; b += kListCap) {
+          const uint32_t e = min(b + kListCap, end);
+          if (i >= b && i < e) {
+            r += i - b;
+            continue;
+          }
           uint32_t lo = b, hi = e;
           while (lo < hi) {
             const uint32_t mid = (lo + hi) / 2;

@@ -100,3 +100,25 @@ def test_shorter_lists_of_many_clouds_match_the_oracle(lib, oracle, batch, n):
                               [(*UNIT, 16, 16, 16)] * batch)
         for b in range(batch):
             assert np.array_equal(got[b], want[b % 4][:m]), (b, m)
+
+
+@pytest.mark.parametrize("rounds", ["1", "2", "9"])
+@pytest.mark.parametrize("kind,n,m", [("cube", 60000, 30000), ("lattice", 30000, 12000),
+                                      ("dups", 48000, 5900), ("rings", 600, 500)])
+def test_a_full_log_of_rounds_matches_the_oracle(lib, oracle, monkeypatch, rounds, kind, n, m):
+    """Rounds beyond the log's entries share its last one, whose samples are
+    sorted in pieces of a list's length."""
+    P = cloud(kind, n)
+    monkeypatch.setenv("NSFPS_LOG_ROUNDS", rounds)
+    want = oracle.fps(P, m, (*UNIT, 16, 16, 16))
+    assert np.array_equal(lib.fps(P, m, (*UNIT, 16, 16, 16)), want)
+    plan = lib.plan_create(P, n, (*UNIT, 16, 16, 16))
+    try:
+        from ns_fps_amd.capi import Hip
+        hip = Hip()
+        d_out = hip.malloc(m * 4)
+        got = lib.plan_sample(plan, m, d_out)
+        assert np.array_equal(hip.download(d_out, got, np.int32), want)
+        hip.free(d_out)
+    finally:
+        lib.plan_destroy(plan)
