@@ -131,7 +131,25 @@ def sha_i32(a):
     return hashlib.sha256(np.asarray(a, np.int32).tobytes()).hexdigest()
 
 
+def engine_of(stats):
+    """Which engine a call took: one workgroup per cloud (its sampling is one
+    launch, all of sample_ms), rounds over the whole chip, or the tree."""
+    if not stats.get("engine", 0):
+        return "tree"
+    one = stats["late_ms"] == stats["sample_ms"] and stats["wide_ms"] == 0
+    return "one workgroup a cloud" if one else "runs"
+
+
+SAMPLING_KERNELS = {
+    "one workgroup a cloud": "sampling pass (k_small_sample)",
+    "runs": "sampling pass (k_update+k_refine+k_gather+k_accept rounds)",
+    "tree": "sampling pass (k_wide_update+k_late_loop)"}
+
+
 def roofline_of(wname, sample_ms, engine):
+    """The census bytes (what the reference's candidate visits read, point by
+    point) over the sampling time; the kernels here move fewer, so the fraction
+    can exceed 1."""
     census = load_census(wname)
     if census is None or not sample_ms or sample_ms <= 0:
         return None
@@ -140,8 +158,8 @@ def roofline_of(wname, sample_ms, engine):
     return {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 6),
             "traffic": profile_traffic("sampling", wname),
-            "kernel": "sampling pass (k_update+k_refine+k_gather+k_accept rounds)"
-            if engine == "runs" else "sampling pass (k_wide_update+k_late_loop)",
+            "kernel": SAMPLING_KERNELS[engine],
+            "bytes": "census of the reference's candidate visits",
             "alg_bytes_per_launch": alg, "kernel_ms": round(sample_ms, 3)}
 
 
@@ -553,7 +571,7 @@ def workload_line(lib, hip, yf, wname, budget_s, steps, warmup, with_cpu=True):
             e2e, dg = run_host_buffers(lib, w)
             line["e2e_ms"] = round(e2e, 3)
             line["e2e_bit_exact"] = g is not None and dg == g["output_sha256"][0]
-        engine = "runs" if s["engine"] else "tree"
+        engine = engine_of(s)
     else:
         r = run_batched(lib, hip, w, steps, warmup)
         s = r["stats"][-1]
@@ -572,7 +590,7 @@ def workload_line(lib, hip, yf, wname, budget_s, steps, warmup, with_cpu=True):
                 "e2e_ms": round(e2e, 3),
                 "e2e_bit_exact": g is not None and dg == g["output_sha256"],
                 "e2e_input": "host float32 (B,N,3) through the module's fps_batched"}
-        engine = "runs" if s["engine"] else "tree"
+        engine = engine_of(s)
     line["mixed_leaves"] = bool(s.get("mixed", 0))
     line["roofline"] = roofline_of(wname, statistics.mean(x["sample_ms"] for x in r["stats"]),
                                    engine)
@@ -681,7 +699,7 @@ def main():
     exact = (g is not None and len(r["out"]) == g["lengths"][0]
              and all(d == g["output_sha256"][0] for d in r["digests"]))
     sample_ms = statistics.mean(s["sample_ms"] for s in stats)
-    engine = "runs" if stats[-1].get("engine", 0) else "tree"
+    engine = engine_of(stats[-1])
     e2e_ms, e2e_digest = run_host_buffers(lib, w)
     plan = run_plan(lib, hip, w, max(3, args.steps // 2))
     line = {

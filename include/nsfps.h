@@ -103,8 +103,10 @@ typedef struct {
                            (1, or 4 when the call has few level-1 nodes) */
   uint32_t mixed;       /* 1 when leaves were runs of 64 slots that may hold several buckets */
   uint32_t hot_set;     /* density class of the clouds: 128 when every one fills at least 6,912
-                           buckets, else 64 (0 for the tree loop); earlier versions' hot sets
-                           had that many copies, no kernel depends on it now */
+                           buckets and no cells share buckets, else 64; always 64 where one
+                           workgroup sampled each cloud, which counts no buckets, and 0 for the
+                           tree loop.  Earlier versions' hot sets had that many copies; no
+                           kernel depends on it now */
 } nsfps_stats;
 
 /* Library constants mirrored from src/yuezu_fps.h:19-50. */
@@ -205,8 +207,9 @@ nsfps_status nsfps_fps_device(const float *d_xyz, uint64_t n, uint64_t n_samples
  * per device, reserved on every device by the library's code object in each
  * process that loads the library, whether or not this call is used, and
  * held until the process ends.  A cloud whose layout needs more fails with
- * NSFPS_EUNSUPPORTED and a message giving both sizes: measured limits are
- * 450,736 points on a 32^3 grid, 460,416 on 16^3 and 428,160 on 64x64x16.
+ * NSFPS_EUNSUPPORTED and a message giving both sizes: for samples of a
+ * sixteenth the limits are 451,444 points on a 32^3 grid, 460,480 on 16^3 and
+ * 430,720 on 64x64x16; for nearly all points 439,456, 448,540 and 419,312.
  * Same arguments, samples and guards as nsfps_fps_device; no hipMalloc,
  * hipFree, stream or event creation, and no memset nodes (fill kernels clear
  * what must start at zero).  Like every call here it cannot be captured into

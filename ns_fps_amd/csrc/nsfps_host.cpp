@@ -1444,7 +1444,7 @@ double ms_between(hipEvent_t a, hipEvent_t b) {
   return ms;
 }
 
-// Speculative-run rounds until every cloud is done.  Rounds are enqueued in
+// Sampling rounds until every cloud is done.  Rounds are enqueued in
 // growing batches; a round of a finished cloud returns at once.  Between
 // batches the host reads each cloud's done flag, sample count and list
 // overflow flag.  Rounds run without refinement passes (the update pass's
@@ -1467,11 +1467,13 @@ RoundSchedule g_schedule;
 // Rounds with at most this many level-1 nodes over all clouds split each
 // node's leaves over kUpdateSplit workgroups of the update pass (its work
 // then spreads over that many more CUs; a node's key is the largest of the
-// parts its workgroups write).  Measured per call: quickstart (3 nodes)
-// 0.97 -> 0.82 ms, 240,000-point scan 4.45 -> 4.21, 524,288-point clustered
-// cloud 7.45 -> 7.29 (at this bound; 7.45 at 128), 64 clouds of 16,384
-// points (256 nodes) unchanged; the 1M-point uniform cube (512 nodes) 7.7 ->
-// 12.3 with it.
+// parts its workgroups write).  Per call, whole and split: 120,000-point scan
+// 1.59 and 1.28 ms, 240,000 1.67 and 1.47, 40,000 Gaussian points 1.48 and
+// 1.02, 120,000 on 17^3 blocks 2.30 and 1.43; from 128 nodes to this bound it
+// depends on the cloud: 600,000 Gaussian points 3.04 and 2.83, 600,000 of a
+// scan 2.16 and 2.17, 524,288 clustered 2.08 and 2.32, a 500,000-point cube
+// 1.64 and 1.89; above it split is the slower: 600,000-point cube on 32^3
+// 2.01 and 2.70, 1M 2.60 and 3.50.
 constexpr uint32_t kSplitMaxNodes = 256;
 // Clouds whose points fill at least this many buckets report the density
 // class 128, others 64 (stats' hot_set; earlier versions' run kernel took
@@ -1480,8 +1482,11 @@ constexpr uint32_t kHot128MinCells = 6912;
 // Calls of at least this many clouds sample them in two halves on two
 // streams: one half's passes run beside the other's, whose short launches
 // leave CUs idle (clouds are independent).  NSFPS_STREAMS=n asks for n groups
-// (at most kMaxStreams).  64 clouds of 16,384 points, per call on the
-// MI355X: one stream 1.94 ms, two 1.79-1.81, three 1.71-1.80.
+// (at most kMaxStreams).  Per call on one, two and three streams: 64 clouds of
+// 20,000 points 2.02, 1.86, 1.85 ms, of 65,536 4.68, 4.50, 4.45; 16 of 20,000
+// 1.15, 1.10, 1.27, of 65,536 1.86, 1.72, 1.73; 8 of 20,000 1.01, 1.05, 1.24,
+// of 33,000 1.15, 1.11, 1.33, of 65,536 1.40, 1.30, 1.54; 4 of 33,000 0.93,
+// 1.00, 1.25.
 constexpr uint32_t kTwoStreamMinClouds = 8;
 constexpr uint32_t kStreamGroups = 2;
 

@@ -34,10 +34,12 @@
 // samples settle as soon as the few larger keys near them have, so a round of
 // 4,096 listed points settles some 900 to 2,200.  Per call on one MI355X, device-resident,
 // against lists sampled one after another by one workgroup: 120,000-point
-// scan -> 16,384 (50 rounds) 3.65 -> 1.30 ms, 1M-point cube -> 65,536 (75)
+// scan -> 16,384 (47 rounds) 3.65 -> 1.28 ms, 1M-point cube -> 65,536 (75)
 // 7.02 -> 2.56, the same on 30^3 cells 10.6 -> 3.83, 8M clustered points ->
-// 524,288 (243) 59 -> 16.0, 1M -> 524,288 (236) 38 -> 7.2.  Clouds in few
-// samples gain least: 17,000 -> 64 0.34 -> 0.37 ms, 14 rounds for 7.
+// 524,288 (243) 59 -> 16.0, 1M -> 524,288 (236) 38 -> 7.2.  Few samples, and
+// the middle ones of many clouds, gain nothing: 17,000 Gaussian points -> 64
+// 320 -> 292 us, -> 256 425 -> 465; 64 clouds of 17,000 -> 265 0.97 -> 1.10 ms,
+// of 65,536 -> 4,096 3.3 -> 4.1.
 //
 // The cube test compares cell coordinates.  Where cells share buckets (block
 // counts that are not powers of two: the Morton code is taken modulo the

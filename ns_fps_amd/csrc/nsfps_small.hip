@@ -1,7 +1,9 @@
 // Clouds of at most kSmallMaxPoints points (gfx950): one workgroup per cloud
 // sorts it (k_small_sort) and one samples it from start to end
 // (k_small_sample), every point in registers and no pass over memory between
-// samples.
+// samples (the kernels of 16 points a thread, above 8,192, keep some of them
+// in scratch memory: 128 registers a thread are too few, and the compiler
+// spills 100 of the sort's and 36 of the sampling's).
 //
 // The sampling goes in rounds.  Let B be a threshold that leaves at most
 // kSmallList points whose keys (min-distance, then lower logical rank) are at
@@ -21,9 +23,10 @@
 //
 // Against the general engine's launches per round (build, update, gather and
 // run kernels), per call on one MI355X, device-resident: 1,024 points -> 256
-// 269 -> 136 us, quickstart 655 -> 625 us, 32 clouds of 1,024 -> 512 433 ->
-// 190 us, 64 clouds of 16,384 -> 4,096 1,809 -> 1,370 us; a scan's cut of
-// 16,384 -> 1,024 from host arrays 782 -> 742 us.
+// 269 -> 136 us, 8,192 -> 1,024 of a cube 634 -> 427, 32 clouds of 1,024 -> 512
+// 433 -> 190 us, 64 clouds of 16,384 -> 4,096 1,809 -> 1,370 us; the
+// quickstart's 10,000 -> 1,000 hardly gains (639 -> 627).  Tie-heavy clouds
+// sampled to a half lose: an 8,192-point lattice -> 4,096 2.2 -> 2.8 ms.
 #include <hip/hip_runtime.h>
 
 #include <float.h>

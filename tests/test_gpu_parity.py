@@ -84,42 +84,19 @@ def test_workload_hash_in_both_leaf_layouts(yf, lib, wname, mixed, monkeypatch):
     assert [sha256_i32(o) for o in outs] == g["output_sha256"]
 
 
-@pytest.mark.parametrize("hot", ["64", "128"])
+@pytest.mark.parametrize("small", ["0", "1"])
 @pytest.mark.parametrize("wname", ["quickstart", "uniform_cube", "uniform_cube_30", "lidar_scan",
                                    "batched_shapes", "clustered"])
-def test_workload_hash_with_either_hot_set(yf, lib, wname, hot, monkeypatch):
-    """The run kernel takes hot sets of 64 or 128 copies (128 where the points
-    fill many buckets; NSFPS_HOT forces either, and grids whose cells share
-    buckets always take 64).  Both give the reference's samples."""
-    monkeypatch.setenv("NSFPS_HOT", hot)
+def test_workload_hash_on_either_engine(yf, lib, wname, small, monkeypatch):
+    """Clouds of at most 16,384 points (the quickstart, the batch) on one
+    workgroup each and in rounds over the whole chip (NSFPS_SMALL decides);
+    larger ones take the rounds either way.  All give the reference's
+    samples."""
+    monkeypatch.setenv("NSFPS_SMALL", small)
     w, g, outs = run_workload(yf, lib, wname)
-    want = 64 if wname == "uniform_cube_30" else int(hot)
-    assert yf.last_stats()["hot_set"] == want
-    assert [len(o) for o in outs] == g["lengths"]
-    assert [sha256_i32(o) for o in outs] == g["output_sha256"]
-
-
-@pytest.mark.parametrize("dense", ["0", "1"])
-@pytest.mark.parametrize("wname", ["uniform_cube", "clustered"])
-def test_workload_hash_with_either_walk(yf, lib, wname, dense, monkeypatch):
-    """128-copy hot sets walk at most 12 coarse rows a sample on dense clouds
-    (more than 64 points a filled bucket) and 16 elsewhere; NSFPS_DENSE_WALK
-    forces either.  Both give the reference's samples."""
-    monkeypatch.setenv("NSFPS_DENSE_WALK", dense)
-    w, g, outs = run_workload(yf, lib, wname)
-    assert yf.last_stats()["hot_set"] == 128
-    assert [len(o) for o in outs] == g["lengths"]
-    assert [sha256_i32(o) for o in outs] == g["output_sha256"]
-
-
-@pytest.mark.parametrize("lb", ["0", "1"])
-@pytest.mark.parametrize("wname", ["uniform_cube", "clustered", "lidar_scan"])
-def test_workload_hash_with_either_update_bound(yf, lib, wname, lb, monkeypatch):
-    """The update pass bounds each pick by each leaf's box for small clouds
-    and for dense ones (the clustered cloud), not for the uniform cube;
-    NSFPS_LEAF_BOUND forces either way.  Both give the reference's samples."""
-    monkeypatch.setenv("NSFPS_LEAF_BOUND", lb)
-    w, g, outs = run_workload(yf, lib, wname)
+    st = yf.last_stats()
+    one_workgroup = st["late_ms"] == st["sample_ms"] and st["wide_ms"] == 0.0
+    assert one_workgroup == (small == "1" and wname in ("quickstart", "batched_shapes"))
     assert [len(o) for o in outs] == g["lengths"]
     assert [sha256_i32(o) for o in outs] == g["output_sha256"]
 
@@ -127,8 +104,8 @@ def test_workload_hash_with_either_update_bound(yf, lib, wname, lb, monkeypatch)
 @pytest.mark.parametrize("streams", ["1", "2", "3"])
 def test_batched_hash_with_one_to_three_streams(yf, lib, streams, monkeypatch):
     """Calls of many clouds sample them in groups on their own streams (one
-    group's update and gather passes beside another's run kernel; two groups
-    by default); NSFPS_STREAMS sets the number.  All give the reference's
+    group's passes beside another's; two groups by default); NSFPS_STREAMS
+    sets the number, and takes the rounds engine.  All give the reference's
     samples."""
     monkeypatch.setenv("NSFPS_STREAMS", streams)
     w, g, outs = run_workload(yf, lib, "batched_shapes")
@@ -136,37 +113,24 @@ def test_batched_hash_with_one_to_three_streams(yf, lib, streams, monkeypatch):
     assert [sha256_i32(o) for o in outs] == g["output_sha256"]
 
 
-@pytest.mark.parametrize("whole", ["0", "1"])
-@pytest.mark.parametrize("wname", ["quickstart", "lidar_scan", "batched_shapes"])
-def test_workload_hash_with_either_large_cube_form(yf, lib, wname, whole, monkeypatch):
-    """Clouds in few buckets (the quickstart's 8) take the run kernel that
-    applies a large-cube sample whose cube holds the list's cell box with no
-    cell test per entry; NSFPS_WHOLE forces that kernel or the general one.
-    Both give the reference's samples."""
-    monkeypatch.setenv("NSFPS_WHOLE", whole)
-    w, g, outs = run_workload(yf, lib, wname)
-    assert yf.last_stats()["hot_set"] == 64
-    assert [len(o) for o in outs] == g["lengths"]
-    assert [sha256_i32(o) for o in outs] == g["output_sha256"]
-
-
 @pytest.mark.parametrize("wname,hot", [("quickstart", 64), ("lidar_scan", 64), ("batched_shapes", 64),
                                        ("uniform_cube", 128), ("clustered", 128),
                                        ("uniform_cube_30", 64)])
-def test_hot_set_size_follows_the_filled_buckets(yf, lib, wname, hot):
-    """128-copy hot sets where the points fill at least 6,912 buckets (the
-    uniform cube 32,768, the clustered cloud 14,321), 64 otherwise (the
-    quickstart 8, the LiDAR scan 1,266, each batched cloud about 2,530) and
-    wherever cells share buckets."""
+def test_density_class_follows_the_filled_buckets(yf, lib, wname, hot):
+    """The reported density class: 128 where the points fill at least 6,912
+    buckets (the uniform cube 32,768, the clustered cloud 14,321), 64 otherwise
+    (the quickstart 8, the LiDAR scan 1,266, each batched cloud about 2,530)
+    and wherever cells share buckets."""
     run_workload(yf, lib, wname)
     assert yf.last_stats()["hot_set"] == hot
 
 
 @pytest.mark.parametrize("wname", ["quickstart", "batched_shapes"])
 def test_workload_hash_with_either_logical_sort(yf, lib, wname, monkeypatch):
-    """Clouds of at most 16,384 points are sorted by bucket in one workgroup
-    each, in LDS; NSFPS_GLOBAL_SORT=1 takes the radix sort over all clouds
-    instead.  Both give the reference's samples."""
+    """The rounds engine sorts clouds of at most 16,384 points by bucket in
+    one workgroup each, in LDS; NSFPS_GLOBAL_SORT=1 takes the radix sort over
+    all clouds instead.  Both give the reference's samples."""
+    monkeypatch.setenv("NSFPS_SMALL", "0")
     for env in ("1", None):
         if env:
             monkeypatch.setenv("NSFPS_GLOBAL_SORT", env)
@@ -276,17 +240,16 @@ TREE = {"NSFPS_ENGINE": "tree"}
 
 
 @pytest.mark.parametrize("env", [
-    {}, {"NSFPS_NO_PADDED": "1"}, {"NSFPS_MIXED": "0"}, {"NSFPS_MIXED": "1"},
-    {"NSFPS_GLOBAL_SORT": "1"}, {"NSFPS_HOT": "64"}, {"NSFPS_HOT": "128"},
-    {"NSFPS_LEAF_BOUND": "0"}, {"NSFPS_LEAF_BOUND": "1"}, {"NSFPS_HOT": "128", "NSFPS_DENSE_WALK": "1"},
-    {"NSFPS_WHOLE": "0"}, {"NSFPS_WHOLE": "1"}, {"NSFPS_WHOLE": "1", "NSFPS_PROFILE": "1"},
-    {"NSFPS_HOT": "128", "NSFPS_PROFILE": "1"}, {**TREE, "NSFPS_WIDE_ITERS": "0"}, {**TREE, "NSFPS_WIDE_ITERS": "1"},
+    {}, {"NSFPS_SMALL": "0"}, {"NSFPS_SMALL": "1"}, {"NSFPS_NO_PADDED": "1"}, {"NSFPS_MIXED": "0"},
+    {"NSFPS_MIXED": "1"}, {"NSFPS_GLOBAL_SORT": "1"}, {"NSFPS_STREAMS": "1"}, {"NSFPS_LOG_ROUNDS": "3"},
+    {"NSFPS_PROFILE": "1"}, {"NSFPS_MIXED": "1", "NSFPS_PROFILE": "1"},
+    {**TREE, "NSFPS_WIDE_ITERS": "0"}, {**TREE, "NSFPS_WIDE_ITERS": "1"},
     {**TREE, "NSFPS_WIDE_ITERS": "37"}, {**TREE, "NSFPS_WIDE_ITERS": "100000"},
     {**TREE, "NSFPS_NO_PADDED": "1"}, {**TREE, "NSFPS_PROFILE": "1"},
     {**TREE, "NSFPS_LATE_THREADS": "1024"},
 ], ids=lambda e: ",".join(f"{k}={v}" for k, v in e.items()) or "runs")
 def test_schedule_and_layout_do_not_change_results(yf, env, monkeypatch):
-    """The engine (speculative runs, or grid-wide steps + single-workgroup
+    """The engine (one workgroup, rounds, or grid-wide steps + single-workgroup
     tree loop), where the grid-wide phase hands over, the padded, table or
     mixed-leaf layout and the profiling build are result-invariant."""
     for k, v in env.items():
@@ -330,7 +293,7 @@ def test_full_size_properties(yf):
 
 
 def test_engine_choice(yf, monkeypatch):
-    """Speculative runs on every grid (cells sharing buckets included), the
+    """Rounds on every grid (cells sharing buckets included), the
     tree loop when asked for."""
     by = {c.name: c for c in GOLDEN_CASES}
     run_module(yf, by["granularity_32x32x32"])

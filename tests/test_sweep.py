@@ -181,38 +181,19 @@ def test_gpu_matches_oracle_on_second_sweep(yf, oracle, seed):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("env", [{"NSFPS_SMALL": "0"}, {"NSFPS_SMALL": "1"},
+                                 {"NSFPS_SMALL": "0", "NSFPS_MIXED": "1"}],
+                         ids=["rounds", "one_workgroup", "rounds_mixed_leaves"])
 @pytest.mark.parametrize("sweep,seed", [(1, s) for s in SEEDS] + [(2, s) for s in SEEDS2],
                          ids=lambda v: str(v))
-def test_gpu_matches_oracle_with_hot_sets_of_128(yf, oracle, sweep, seed, monkeypatch):
-    """Both sweeps with the run kernel's 128-copy hot sets forced (the size
-    otherwise taken only where the points fill many buckets; grids whose
-    cells share buckets keep 64)."""
+def test_gpu_matches_oracle_on_each_engine(yf, oracle, sweep, seed, env, monkeypatch):
+    """Both sweeps on the rounds engine with the layout it chooses and with
+    leaves of several buckets (where buckets have one cell), and with one
+    workgroup a cloud (clouds of at most 16,384 points; larger ones take the
+    rounds)."""
     from ns_fps_amd.capi import Lib
-    monkeypatch.setenv("NSFPS_HOT", "128")
-    if sweep == 1:
-        shape, p, m, rng = make_case(seed)
-        blocks = rng[6:9]
-    else:
-        shape, p, m, rng, blocks = make_case2(seed)
-    if rng is None:
-        got = Lib().fps_bbox(p, m, blocks)
-    else:
-        got = yf.fps(p, m, yf.make_range(*rng))
-    want = oracle.fps(p, m, rng, blocks=blocks)
-    assert np.array_equal(got, want), (len(got), len(want), f"first difference at "
-                                       f"{np.argmax(got[:len(want)] != want[:len(got)])}")
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("sweep,seed", [(1, s) for s in SEEDS] + [(2, s) for s in SEEDS2],
-                         ids=lambda v: str(v))
-def test_gpu_matches_oracle_with_the_list_box_form(yf, oracle, sweep, seed, monkeypatch):
-    """Both sweeps with the run kernel forced to the form that applies a
-    large-cube sample holding the list's cell box with no cell test (taken
-    otherwise only for clouds in few buckets; grids whose cells share buckets
-    and 128-copy hot sets keep the general form)."""
-    from ns_fps_amd.capi import Lib
-    monkeypatch.setenv("NSFPS_WHOLE", "1")
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
     if sweep == 1:
         shape, p, m, rng = make_case(seed)
         blocks = rng[6:9]
