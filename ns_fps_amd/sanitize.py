@@ -52,7 +52,7 @@ def sanitized_env():
             raise RuntimeError(f"{f} is missing: run python -m ns_fps_amd.build sanitize")
     env = dict(os.environ)
     env.update({
-        "LD_PRELOAD": runtime_path(),
+        "LD_PRELOAD": ":".join(filter(None, [runtime_path(), env.get("LD_PRELOAD")])),
         "NSFPS_LIB": lib,
         "NSFPS_MODULE": mod,
         # the interpreter itself is not instrumented: its allocations at exit

@@ -40,7 +40,7 @@ def test_stated_limits(tmp_path):
     fake = str(tmp_path / "fake_hip.so")
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-Wall", os.path.join(ROOT, "tests", "fake_hip.c"),
                     "-o", fake], check=True)
-    env = dict(os.environ, LD_PRELOAD=fake)
+    env = dict(os.environ, LD_PRELOAD=":".join(filter(None, [fake, os.environ.get("LD_PRELOAD")])))
     p = subprocess.run([sys.executable, "-c", PROBE], cwd=ROOT, env=env, check=True,
                        stdout=subprocess.PIPE, text=True)
     assert [int(v) for v in p.stdout.split()] == said
