@@ -819,10 +819,11 @@ uint32_t list_cap_for(uint32_t n, size_t nclouds) {
 // for layers that hold few samples at first.  Calls of up to kSeqOnly samples
 // take all of them so, and end without the layers' final sort.  Per call, all
 // layers, then these rules: 17,000 Gaussian points -> 16 269 and 195 us, 64
-// 372 and 290, 128 438 and 361, 256 496 and 468; 300,000 of a scan -> 64 646
-// and 552; 120,000 of a scan -> 16,384 1.49 and 1.37 ms.  The first 64 of
-// longer calls: 256 459 us, but the 1M-point cube -> 129 938 (940 at 32, 910 at
-// 16) and a scan's 16,384 1.40 ms.  Of a large cloud's many samples the first
+// 372 and 290, 128 438 and 361, 256 496 and 442; 300,000 of a scan -> 64 646
+// and 552; 120,000 of a scan -> 16,384 1.49 and 1.37 ms.  Longer calls go on
+// to the end of the list that holds sample kSeqFirst (stopping there instead:
+// 256 461 us).  With 64 in its place: 256 454 us, 17,000 of a cube -> 129 494
+// against 444, 64 clouds of 17,000 -> 265 1.12 against 1.14 ms.  Of a large cloud's many samples the first
 // make no difference but their own: from kSeqLarge points and kSeqFew samples
 // on all are layers (1M-point cube -> 65,536 2.61 ms, with 32 first 2.64;
 // -> 512 1,164 and 1,166 us, 1M Gaussian points -> 512 1,445 and 1,385).

@@ -181,7 +181,7 @@ struct CloudDev {
   uint64_t *log_ktop;         //    a bound on its keys
   uint32_t *log_start;        //    and the samples before it
   uint32_t list_cap, log_cap;
-  uint32_t seq_samples;       // samples taken one after another before the layers begin
+  uint32_t seq_samples;       // lists are sampled one after another until so many are taken
 };
 
 // Argmax key: larger min-distance wins, equal distances go to the smaller

@@ -38,8 +38,8 @@
 // 7.02 -> 2.56, the same on 30^3 cells 10.6 -> 3.83, 8M clustered points ->
 // 524,288 (243) 59 -> 16.0, 1M -> 524,288 (236) 38 -> 7.2.  Few samples, and
 // the middle ones of many clouds, gain nothing: 17,000 Gaussian points -> 64
-// 320 -> 292 us, -> 256 425 -> 465; 64 clouds of 17,000 -> 265 0.97 -> 1.10 ms,
-// of 65,536 -> 4,096 3.3 -> 4.1.
+// 320 -> 292 us, -> 256 425 -> 442; 64 clouds of 17,000 -> 265 0.98 -> 1.15 ms,
+// of 65,536 -> 4,096 3.3 -> 3.8.
 //
 // The cube test compares cell coordinates.  Where cells share buckets (block
 // counts that are not powers of two: the Morton code is taken modulo the
@@ -58,7 +58,12 @@ constexpr uint32_t kPassThreads = 1024;  // grid-wide passes: one level-1 node p
 constexpr uint32_t kPassWaves = kPassThreads / 64;
 constexpr uint32_t kLeavesPerWave = kFan / kPassWaves;
 constexpr uint32_t kMaxShift = 52;  // kHistBins << 52 covers the whole u64 key range
-constexpr uint32_t kSparseGroups = 128;  // workgroups per cloud of the refinement and gather passes
+// Workgroups per cloud of the refinement and gather passes, and of a launch's
+// clouds together (each replays the selection from 16 KB of histogram, and
+// takes up to kGatherNodes nodes at a time): 64 clouds of 65,536 points ->
+// 4,096 4.24 ms per call with one a node, 3.78 at 256 a launch (3.62 at 128,
+// where 17,000 Gaussian points x 64 -> 265 lose 3 %).
+constexpr uint32_t kSparseGroups = 128, kSparseLaunch = 256;
 constexpr uint32_t kGatherNodes = 16;    // nodes per list-range claim of the gather pass
 constexpr uint32_t kGatherHold = 4;      // hot leaves per wave whose points stay in registers
 
@@ -1000,19 +1005,18 @@ typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 #define NSFPS_CONSTANT
 #endif
 
-// The first seq_samples of a cloud are taken from its lists one after another
-// instead, as the reference does: early layers hold few samples, so a list is
-// worth several rounds of them.  One workgroup, four entries a thread, one
-// barrier a sample: each wave publishes its largest key, every wave takes the
-// largest of those, and the entries that the sample's cube holds are lowered;
-// it ends when no listed key is left at or above the threshold, or they all
-// are taken.  These samples
-// come in order, so a call that ends among them needs no sort.  Bound by the
-// chain of one sample: some 200 instructions, two LDS reads and the barrier,
-// about 0.8 us (1.35 with the cube's half-widths worked out on every lane
-// alike, 1.05 with keys compared as integer pairs).  Lists and windows are
-// the first rounds' there: 1,024 entries, bins of 1/1024 to 1/2048 of the span
-// below the last threshold.
+// The first seq_samples of a cloud, and the rest of the list that reaches
+// them, are taken one after another instead, as the reference does: early
+// layers hold few samples, so a list is worth several rounds of them.  One
+// workgroup, four entries a thread, one barrier a sample: each wave publishes
+// its largest key, every wave takes the largest of those, and the entries that
+// the sample's cube holds are lowered; it ends when no listed key is left at
+// or above the threshold.  These samples come in order, so a call that ends
+// among them needs no sort.  Bound by the chain of one sample: some 200
+// instructions, two LDS reads and the barrier, about 0.8 us (1.35 with the
+// cube's half-widths worked out on every lane alike, 1.05 with keys compared
+// as integer pairs).  Lists and windows are the first rounds' there: 1,024
+// entries, bins of 1/1024 to 1/2048 of the span below the last threshold.
 constexpr uint32_t kSettleSlots = kSeqList / kAcceptThreads;
 static_assert(kSettleSlots * kAcceptThreads == kSeqList, "whole slots");
 
@@ -1068,7 +1072,7 @@ __device__ __forceinline__ void settle(const CloudDev &c, uint32_t par, uint32_t
   NSFPS_GLOBAL uint32_t *const SW = vgpr_ptr(gptr(
       lane == 0 ? c.smp_d : lane == 1 ? c.smp_lo : lane == 2 ? c.smp_row : reinterpret_cast<uint32_t *>(c.out)));
   NSFPS_GLOBAL uint2 *const LC = vgpr_ptr(gptr(c.list_c));
-  const uint32_t T = rs.ntaken, end = min(c.m, c.seq_samples);
+  const uint32_t T = rs.ntaken, end = c.m;
   const uint64_t bkey = rs.bkey;
   float x[kSettleSlots], y[kSettleSlots], z[kSettleSlots];
   uint32_t row[kSettleSlots], cell[kSettleSlots];
@@ -1507,7 +1511,9 @@ hipError_t launch_rounds(const CloudDev *d_clouds, uint32_t nclouds, uint32_t ma
   if (list_cap < kListShort || list_cap > kListCap || (list_cap & (list_cap - 1)))
     return hipErrorInvalidValue;
   const dim3 grid(max_nl1, nclouds);
-  const dim3 sparse(max_nl1 < kSparseGroups ? max_nl1 : kSparseGroups, nclouds);
+  const uint32_t share = kSparseLaunch / nclouds < 2 ? 2u : kSparseLaunch / nclouds;
+  const uint32_t groups = share < kSparseGroups ? share : kSparseGroups;
+  const dim3 sparse(max_nl1 < groups ? max_nl1 : groups, nclouds);
   using Launch = void (*)(const CloudDev *, uint32_t, dim3, dim3, uint32_t, uint32_t, uint32_t,
                           bool, hipStream_t);
   constexpr uint32_t S = kUpdateSplit;
