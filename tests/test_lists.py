@@ -122,3 +122,17 @@ def test_a_full_log_of_rounds_matches_the_oracle(lib, oracle, monkeypatch, round
         hip.free(d_out)
     finally:
         lib.plan_destroy(plan)
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-21, 3e-20, 3e18, 1e30])
+def test_first_samples_at_the_ends_of_the_number_range(lib, oracle, monkeypatch, scale):
+    """Squared distances that are subnormal or overflow: the keys of the lists
+    sampled one after another are compared as doubles, subnormal ones among
+    them."""
+    P = (np.random.RandomState(9).uniform(-1, 1, (20000, 3)) * scale).astype(np.float32)
+    P[:40] *= np.float32(0.01)
+    rng = tuple(float(np.float32(v * scale)) for v in UNIT) + (8, 8, 8)
+    monkeypatch.setenv("NSFPS_SMALL", "0")
+    want = oracle.fps(P, 400, rng)
+    for m in (100, 400):
+        assert np.array_equal(lib.fps(P, m, rng), want[:m])
